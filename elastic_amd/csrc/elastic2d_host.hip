@@ -86,9 +86,7 @@ static int op3(int nt, int nz, int nx, float* const* hist, const float* const* c
   DevBuf h, cf, dd, dt;
   STCHK(h.alloc(5 * (size_t)nt * n2 * sizeof(float), "adjoint histories"));
   STCHK(cf.alloc(5 * n2 * sizeof(float), "coefficients"));
-  std::vector<float> c5((size_t)5 * nz * nx);
-  for (int c = 0; c < 5; ++c) std::memcpy(c5.data() + (size_t)c * nz * nx, coefs[c], sizeof(float) * nz * nx);
-  STCHK(fill_masked_coefs(c5.data(), nz, nx, ldz, cf.as<float>()));
+  STCHK(store_masked_coefs(coefs, nz, nx, ldz, cf.as<float>(), st));
   float* hp = h.as<float>();
   for (int f = 0; f < 5; ++f)
     HIPCHK(hipMemcpyAsync(hp + (size_t)f * nt * n2, hist[f], (size_t)nt * n2 * sizeof(float), hipMemcpyHostToDevice,
@@ -180,7 +178,7 @@ struct MaskOrigin {
 };
 
 // Zero each (unpadded, ldz = nz) coefficient array outside its operator's
-// range, as fill_masked_coefs does on the host.
+// range, as store_masked_coefs does.
 __global__ void k_mask_coefs(float* __restrict__ coef, int nz, int nx, MaskOrigin m) {
   const long long n2 = (long long)nz * nx;
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < 5 * n2;
@@ -278,12 +276,13 @@ static int op3_noalloc(int nt, int nz, int nx, float* const* hist, const float* 
 
 // Single-shot engine from an rtm_shot_t.
 static int single_engine(Engine& e, const rtm_shot_t* s, const float* coef5, const float* wavelet,
-                         int snap_fmt) {
+                         int snap_fmt, bool modelling = false) {
   if (!s || !coef5 || !wavelet) { set_error("null argument"); return E_ARG; }
   EngineCfg cfg;
   cfg.nt = s->nt; cfg.dx = s->dx; cfg.dt = s->dt; cfg.abc = s->abc; cfg.adj_abc = s->adj_abc;
   cfg.snap_every = s->snap_every < 1 ? 1 : s->snap_every;
   cfg.snap_fmt = snap_fmt;
+  cfg.modelling = modelling;
   cfg.comp = s->comp_image;
   cfg.txr = default_txr();
   cfg.xcd = default_xcd();
@@ -357,16 +356,6 @@ static void ricker(int nt, float dt, float fp, int nsource, float* out) {
   }
 }
 
-// Non-finite scan of a device buffer.
-__global__ void k_nonfinite(const float* p, size_t n, int* flag) {
-  int bad = 0;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    bad |= !isfinite(p[i]);
-  if (bad) atomicOr(flag, 1);
-}
-
-
 // Streaming copy used to measure the achievable HBM bandwidth and to
 // calibrate the FETCH_SIZE / WRITE_SIZE counters (known bytes per dispatch).
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -423,6 +412,7 @@ __global__ __launch_bounds__(256) void k_copy_probe(const v4f* __restrict__ src,
   if (mode == 2 && acc.x == 123.456f) dst[0] = acc;  // keeps the reads live
 }
 
+// Error of the first non-finite value (the device scan found one).
 static int host_finite(const float* p, size_t n, const char* what) {
   for (size_t i = 0; i < n; ++i)
     if (!std::isfinite(p[i])) {
@@ -509,13 +499,13 @@ RTM_EXPORT int rtm_forward_hip(const rtm_shot_t* s, const float* coef5, const fl
                                float* rec, float* last) {
   if (s && s->nrx > 0 && !rec) { set_error("null receiver buffer"); return E_ARG; }
   Engine e;
-  STCHK(single_engine(e, s, coef5, wavelet, SNAP_HIST));
+  STCHK(single_engine(e, s, coef5, wavelet, SNAP_HIST, true));
   STCHK(e.model_data());
   store_timing(e.timing());
-  if (s->nrx > 0) STCHK(e.get_data(0, rec));
+  bool nonfinite = false;
+  if (s->nrx > 0) STCHK(e.get_data(0, rec, &nonfinite));
   if (last) STCHK(e.get_last_levels(0, last));
-  if (s->nrx > 0) STCHK(host_finite(rec, (size_t)5 * s->nt * s->nrx, "receiver data"));
-  return OK;
+  return nonfinite ? host_finite(rec, (size_t)5 * s->nt * s->nrx, "receiver data") : OK;
 }
 
 RTM_EXPORT int rtm_forward_movie_hip(const rtm_shot_t* s, const float* coef5, const float* wavelet, int nsnap,
@@ -536,6 +526,7 @@ RTM_EXPORT int rtm_forward_movie_hip(const rtm_shot_t* s, const float* coef5, co
   cfg.tblock = default_tblock();
   cfg.march_w = default_march_w();
   cfg.march_nw = default_march_nw();
+  cfg.modelling = true;
   cfg.movie_every = every;
   cfg.movie_n = nsnap;
   cfg.movie_z0 = z0; cfg.movie_x0 = x0; cfg.movie_nz = wnz; cfg.movie_nx = wnx;
@@ -559,8 +550,9 @@ RTM_EXPORT int rtm_migrate_hip(const rtm_shot_t* s, const float* coef5, const fl
   if (s->nrx > 0) STCHK(e.set_data(0, rec));
   STCHK(e.migrate());
   store_timing(e.timing());
-  STCHK(e.get_image(0, img));
-  return host_finite(img, (size_t)3 * s->nz * s->nx, "images");
+  bool nonfinite = false;
+  STCHK(e.get_image(0, img, &nonfinite));
+  return nonfinite ? host_finite(img, (size_t)3 * s->nz * s->nx, "images") : OK;
 }
 
 RTM_EXPORT int rtm_born_hip(const rtm_shot_t* s, const float* coef5, const float* wavelet,

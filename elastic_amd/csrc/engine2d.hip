@@ -1,5 +1,6 @@
 // engine2d.hip -- multi-shot 2D elastic RTM engine (host side).
 #include "engine2d.hpp"
+#include "layout.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -75,17 +76,16 @@ void sponge_factors(int n, int abc, std::vector<float>& k) {
 const int kMaskIx0[5] = {5, 4, 4, 5, 4};
 const int kMaskIz0[5] = {4, 5, 4, 5, 4};
 
-int fill_masked_coefs(const float* coef5, int nz, int nx, int ldz, float* dev) {
-  const size_t n2 = (size_t)ldz * nx;
-  std::vector<float> h(5 * n2, 0.0f);
-  for (int c = 0; c < 5; ++c) {
-    const float* src = coef5 + (size_t)c * nz * nx;
-    float* dst = h.data() + c * n2;
-    for (int ix = kMaskIx0[c]; ix <= nx - 6; ++ix)
-      for (int iz = kMaskIz0[c]; iz <= nz - 6; ++iz) dst[iz + (size_t)ldz * ix] = src[iz + (size_t)nz * ix];
-  }
-  HIPCHK(hipMemcpy(dev, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));
-  return OK;
+int store_masked_coefs(const float* const* coefs, int nz, int nx, int ldz, float* dev, hipStream_t st) {
+  FieldBox box[5];
+  for (int c = 0; c < 5; ++c) box[c] = FieldBox{kMaskIz0[c], nz - 6, kMaskIx0[c], nx - 6};
+  return store_fields(coefs, 5, nz, nx, ldz, dev, (size_t)ldz * nx, box, st);
+}
+
+int fill_masked_coefs(const float* coef5, int nz, int nx, int ldz, float* dev, hipStream_t st) {
+  const float* c[5];
+  for (int k = 0; k < 5; ++k) c[k] = coef5 + (size_t)k * nz * nx;
+  return store_masked_coefs(c, nz, nx, ldz, dev, st);
 }
 
 static int nstrips(int nz, int nx, int txr) {
@@ -182,7 +182,7 @@ int Engine::setup(const EngineCfg& cfg, const std::vector<ShotSpec>& shots,
       return E_ARG;
     }
     STCHK(r.coef.alloc(5 * r.n2 * sizeof(float), "coefficients"));
-    STCHK(fill_masked_coefs(coef5[s], p.nz, p.nx, r.ldz, r.coef.as<float>()));
+    STCHK(fill_masked_coefs(coef5[s], p.nz, p.nx, r.ldz, r.coef.as<float>(), st_));
     if (cfg_.abc > 0) {
       std::vector<float> hz, hx;
       sponge_factors(p.nz, cfg_.abc, hz);
@@ -217,6 +217,11 @@ int Engine::setup(const EngineCfg& cfg, const std::vector<ShotSpec>& shots,
 // its source-wavefield snapshots (and their per-strip scales).
 static void shot_work(const EngineCfg& c, long long n2, int nstrip, size_t* snap, size_t* scale, size_t* work) {
   const long long K = c.nt / c.snap_every;
+  if (c.modelling) {
+    *snap = *scale = 0;
+    *work = (size_t)5 * kEngineRing * n2 * sizeof(float);
+    return;
+  }
   switch (c.snap_fmt) {
     case SNAP_HIST: *snap = (size_t)2 * c.nt * n2 * sizeof(float); *scale = 0; break;
     case SNAP_F32: *snap = (size_t)4 * K * n2 * sizeof(float); *scale = 0; break;
@@ -658,7 +663,7 @@ int Engine::set_true_model(const std::vector<const float*>& coef5_true) {
   for (size_t s = 0; s < specs_.size(); ++s) {
     Res& r = res_[s];
     STCHK(r.coef_true.alloc(5 * r.n2 * sizeof(float), "true-model coefficients"));
-    STCHK(fill_masked_coefs(coef5_true[s], specs_[s].nz, specs_[s].nx, r.ldz, r.coef_true.as<float>()));
+    STCHK(fill_masked_coefs(coef5_true[s], specs_[s].nz, specs_[s].nx, r.ldz, r.coef_true.as<float>(), st_));
   }
   for (int g = 0; g < (int)groups_.size(); ++g) STCHK(fill_desc(g, true, false));
   return OK;
@@ -666,25 +671,12 @@ int Engine::set_true_model(const std::vector<const float*>& coef5_true) {
 
 int Engine::set_data(int shot, const float* h) {
   if (shot < 0 || shot >= (int)specs_.size() || !h) { set_error("bad shot index or null data"); return E_ARG; }
-  const int nt = cfg_.nt, nr = specs_[shot].nrx;
-  std::vector<float> t((size_t)5 * nt * nr);
-  for (int f = 0; f < 5; ++f)
-    for (int ix = 0; ix < nr; ++ix)
-      for (int it = 0; it < nt; ++it) t[((size_t)f * nt + it) * nr + ix] = h[(size_t)f * nt * nr + it + (size_t)nt * ix];
-  if (!t.empty()) HIPCHK(hipMemcpy(res_[shot].rec.p, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice));
-  return OK;
+  return store_records(h, 5, cfg_.nt, specs_[shot].nrx, res_[shot].rec.as<float>(), st_);
 }
 
-int Engine::get_data(int shot, float* h) {
+int Engine::get_data(int shot, float* h, bool* nonfinite) {
   if (shot < 0 || shot >= (int)specs_.size() || !h) { set_error("bad shot index or null data"); return E_ARG; }
-  HIPCHK(hipStreamSynchronize(st_));
-  const int nt = cfg_.nt, nr = specs_[shot].nrx;
-  std::vector<float> t((size_t)5 * nt * nr);
-  if (!t.empty()) HIPCHK(hipMemcpy(t.data(), res_[shot].rec.p, t.size() * sizeof(float), hipMemcpyDeviceToHost));
-  for (int f = 0; f < 5; ++f)
-    for (int ix = 0; ix < nr; ++ix)
-      for (int it = 0; it < nt; ++it) h[(size_t)f * nt * nr + it + (size_t)nt * ix] = t[((size_t)f * nt + it) * nr + ix];
-  return OK;
+  return fetch_records(h, 5, cfg_.nt, specs_[shot].nrx, res_[shot].rec.as<float>(), nonfinite, st_);
 }
 
 int Engine::synthesize() {
@@ -715,6 +707,7 @@ int Engine::model_data() {
 }
 
 int Engine::migrate() {
+  if (cfg_.modelling) { set_error("this engine holds no snapshots (modelling only)"); return E_ARG; }
   tm_ = Timing{};
   if (stack_.p) HIPCHK(hipMemsetAsync(stack_.p, 0, stack_.bytes, st_));
   for (int g = 0; g < (int)groups_.size(); ++g) {
@@ -750,6 +743,7 @@ int Engine::migrate() {
 }
 
 int Engine::born(const std::vector<const float*>& dm) {
+  if (cfg_.modelling) { set_error("this engine holds no snapshots (modelling only)"); return E_ARG; }
   if (groups_.size() != 1) { set_error("Born modelling runs single-group engines only"); return E_ARG; }
   if (dm.size() != specs_.size()) { set_error("dm list size mismatch"); return E_ARG; }
   if (cfg_.snap_fmt != SNAP_HIST) { set_error("Born modelling needs the fp32 history format"); return E_ARG; }
@@ -759,9 +753,10 @@ int Engine::born(const std::vector<const float*>& dm) {
   for (size_t k = 0; k < specs_.size(); ++k) {
     const ShotSpec& p = specs_[k];
     float* d = born_buf_.as<float>() + k * 8 * n2max_ + 5 * n2max_;
-    for (int c = 0; c < 3; ++c)  // component stride = the shot's own n2 (as the kernels index it)
-      HIPCHK(hipMemcpy2D(d + c * res_[k].n2, res_[k].ldz * sizeof(float), dm[k] + (size_t)c * p.nz * p.nx,
-                         p.nz * sizeof(float), p.nz * sizeof(float), p.nx, hipMemcpyHostToDevice));
+    const size_t nn = (size_t)p.nz * p.nx;
+    const float* c[3] = {dm[k], dm[k] + nn, dm[k] + 2 * nn};
+    // component stride = the shot's own n2 (as the kernels index it)
+    STCHK(store_fields(c, 3, p.nz, p.nx, res_[k].ldz, d, res_[k].n2, nullptr, st_));
     STCHK(launch_fill(res_[k].rec.as<float>(), (size_t)5 * cfg_.nt * std::max(p.nrx, 1), 0.f, st_));
   }
   STCHK(fill_desc(0, false, true));
@@ -779,25 +774,16 @@ int Engine::born(const std::vector<const float*>& dm) {
   return OK;
 }
 
-int Engine::get_image(int shot, float* img3) {
+int Engine::get_image(int shot, float* img3, bool* nonfinite) {
   if (shot < 0 || shot >= (int)specs_.size() || !img3) { set_error("bad shot index or null output"); return E_ARG; }
-  HIPCHK(hipStreamSynchronize(st_));
   const ShotSpec& p = specs_[shot];
   const Res& r = res_[shot];
-  for (int c = 0; c < 3; ++c)
-    HIPCHK(hipMemcpy2D(img3 + (size_t)c * p.nz * p.nx, p.nz * sizeof(float), r.img.as<float>() + c * r.n2,
-                       r.ldz * sizeof(float), p.nz * sizeof(float), p.nx, hipMemcpyDeviceToHost));
-  return OK;
+  return fetch_fields(img3, 3, p.nz, p.nx, r.ldz, r.img.as<float>(), r.n2, nonfinite, st_);
 }
 
 int Engine::get_stack(float* img3) {
   if (!stack_.p || !img3) { set_error("no stacked image configured"); return E_ARG; }
-  HIPCHK(hipStreamSynchronize(st_));
-  const size_t n = (size_t)3 * cfg_.stack_nz * cfg_.stack_nx;
-  std::vector<double> h(n);
-  HIPCHK(hipMemcpy(h.data(), stack_.p, n * sizeof(double), hipMemcpyDeviceToHost));
-  for (size_t i = 0; i < n; ++i) img3[i] = (float)h[i];
-  return OK;
+  return fetch_rounded(img3, stack_.as<double>(), (size_t)3 * cfg_.stack_nz * cfg_.stack_nx, st_);
 }
 
 int Engine::get_last_levels(int shot, float* last10) {
@@ -805,7 +791,6 @@ int Engine::get_last_levels(int shot, float* last10) {
   const Group& gr = groups_[last_group_];
   auto it = std::find(gr.shots.begin(), gr.shots.end(), shot);
   if (it == gr.shots.end() || !last10) { set_error("shot %d is not in the last group run", shot); return E_ARG; }
-  HIPCHK(hipStreamSynchronize(st_));
   const float* base = ring_of(shot);
   const ShotSpec& p = specs_[shot];
   const Res& r = res_[shot];
@@ -813,10 +798,8 @@ int Engine::get_last_levels(int shot, float* last10) {
   const int nt = cfg_.nt;
   for (int lv = 0; lv < 2; ++lv) {
     const int L = nt - 1 + lv;  // levels nt-1, nt (slot L % kRing)
-    for (int f = 0; f < 5; ++f)
-      HIPCHK(hipMemcpy2D(last10 + (size_t)(5 * lv + f) * nn, p.nz * sizeof(float),
-                         base + (size_t)(L % kRing) * 5 * r.n2 + f * r.n2, r.ldz * sizeof(float), p.nz * sizeof(float),
-                         p.nx, hipMemcpyDeviceToHost));
+    STCHK(fetch_fields(last10 + 5 * lv * nn, 5, p.nz, p.nx, r.ldz, base + (size_t)(L % kRing) * 5 * r.n2, r.n2,
+                       nullptr, st_));
   }
   return OK;
 }

@@ -43,6 +43,11 @@ struct EngineCfg {
                        // the marching forward with the tile adjoint
   int march_w = 32;    // strip width (columns, even) of the marching form
   int march_nw = 2;    // strip height of the marching form in waves (64 rows each): 1, 2, 4
+  // Modelling only (model_data): no room for source-wavefield snapshots. A
+  // call that allocates and frees gigabytes it never touches waits for the
+  // driver to clear them (a 390 x 690 x 2000 record: 113 ms with the unused
+  // 4.3 GB history, of 16 ms of kernels).
+  bool modelling = false;
   int max_group = 0;   // cap on shots per group (0 = memory bound only)
   int stack_nz = 0, stack_nx = 0;  // stacked image (0 = none)
   double mem_fraction = 0.85;      // share of free memory the working set may use
@@ -109,7 +114,7 @@ class Engine {
   // Second coefficient set per shot (the "true" model) for data synthesis.
   int set_true_model(const std::vector<const float*>& coef5_true);
   int set_data(int shot, const float* rec_host);  // 5*(nt,nrx)
-  int get_data(int shot, float* rec_host);
+  int get_data(int shot, float* rec_host, bool* nonfinite = nullptr);
   // observed = forward(true) - forward(migration) for every shot
   int synthesize();
   // forward + adjoint + imaging of every shot, images stacked
@@ -118,7 +123,7 @@ class Engine {
   int model_data();
   // Born modelling of one-group runs (single shot API); dm 3*(nz,nx) per shot
   int born(const std::vector<const float*>& dm);
-  int get_image(int shot, float* img3);          // 3*(nz,nx)
+  int get_image(int shot, float* img3, bool* nonfinite = nullptr);  // 3*(nz,nx)
   int get_stack(float* img3);                    // 3*(stack_nz,stack_nx)
   int get_last_levels(int shot, float* last10);  // levels nt-1, nt of the last run
   // Use (w = the network's packed inference weights on the device) or drop
@@ -196,7 +201,10 @@ class Engine {
 // The engine of a batch handle (elastic2d_host.hip).
 Engine* batch_engine(struct rtm_batch* b);
 
-int fill_masked_coefs(const float* coef5, int nz, int nx, int ldz, float* dev);
+// The five (nz, nx) coefficient arrays (five pointers, or back to back) on the
+// device with column stride ldz, zeroed outside each operator's range.
+int store_masked_coefs(const float* const* coefs, int nz, int nx, int ldz, float* dev, hipStream_t st);
+int fill_masked_coefs(const float* coef5, int nz, int nx, int ldz, float* dev, hipStream_t st);
 void sponge_factors(int n, int abc, std::vector<float>& k);
 int ensure_device();
 int default_txr();

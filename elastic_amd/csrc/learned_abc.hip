@@ -8,6 +8,7 @@
 
 #include "../../include/learned_abc.h"
 #include "engine2d.hpp"
+#include "layout.hpp"
 
 #include <algorithm>
 #include <functional>
@@ -916,7 +917,7 @@ struct LGrid {
     // readable for the learned layer's inference after the step
     STCHK(ring.alloc(20 * n2 * 4, "ring"));
     STCHK(coef.alloc(5 * n2 * 4, "coefficients"));
-    STCHK(fill_masked_coefs(coef5, nz, nx, ldz, coef.as<float>()));
+    STCHK(fill_masked_coefs(coef5, nz, nx, ldz, coef.as<float>(), nullptr));
     STCHK(launch_fill(ring.as<float>(), 20 * n2, 0.f, nullptr));
     h.nz = nz; h.nx = nx; h.ldz = ldz; h.nt = nt; h.n2 = n2;
     h.lev = ring.as<float>(); h.lev_stride = 5 * n2; h.fstride = n2; h.lev_mod = 4; h.lev_off = 4;
@@ -1240,21 +1241,11 @@ RTM_EXPORT int labc_forward(labc_net* n, const rtm_shot_t* s, const float* coef5
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   g_last_ms = ms;
-  if (s->nrx > 0) {
-    const int nt = s->nt;
-    std::vector<float> t((size_t)5 * nt * s->nrx);
-    HIPCHK(hipMemcpy(t.data(), recd.p, t.size() * 4, hipMemcpyDeviceToHost));
-    for (int f = 0; f < 5; ++f)
-      for (int ix = 0; ix < s->nrx; ++ix)
-        for (int it = 0; it < nt; ++it)
-          rec[(size_t)f * nt * s->nrx + it + (size_t)nt * ix] = t[((size_t)f * nt + it) * s->nrx + ix];
-  }
+  if (s->nrx > 0) STCHK(fetch_records(rec, 5, s->nt, s->nrx, recd.as<float>(), nullptr, nullptr));
   if (last) {
     const size_t nn = (size_t)s->nz * s->nx;
     for (int lv = 0; lv < 2; ++lv)
-      for (int f = 0; f < 5; ++f)
-        HIPCHK(hipMemcpy2D(last + (size_t)(5 * lv + f) * nn, s->nz * 4, g.level(s->nt - 1 + lv) + f * g.n2,
-                           g.ldz * 4, s->nz * 4, s->nx, hipMemcpyDeviceToHost));
+      STCHK(fetch_fields(last + 5 * lv * nn, 5, s->nz, s->nx, g.ldz, g.level(s->nt - 1 + lv), g.n2, nullptr, nullptr));
   }
   return OK;
 }

@@ -36,6 +36,7 @@ constexpr int AWY = 4;     // waves along n2
 constexpr int ATXR = 4;    // n2 cells per thread
 constexpr int AX = AWY * ATXR;
 constexpr int AH = 5;
+constexpr int AC3_MAX_CHUNK = 128;  // planes a workgroup marches at most
 constexpr int ALZ = AZ + 2 * AH, ALX = AX + 2 * AH;
 
 struct Ac3Args {
@@ -326,6 +327,46 @@ std::vector<float> taper(int n, int abc) {
   return k;
 }
 
+// Step workgroups resident at once on the current device (109 VGPRs without
+// imaging: 4 waves per SIMD, so 4 workgroups a CU, 1024 on the chip).
+int resident_workgroups() {
+  static const int n = [] {
+    int dev = 0, cus = 0, per = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_ac3_step<false>, AZ * AWY, 0) != hipSuccess ||
+        cus * per <= 0)
+      return 1024;
+    return cus * per;
+  }();
+  return n;
+}
+
+// Planes a workgroup marches along y. A plane costs a workgroup about 1.7 us
+// whatever the grid (the latency of its loads), and a chunk some six planes
+// more for its first loads, so the step takes (rounds of resident workgroups)
+// x (planes + 6): the number of chunks that minimises it. Both sides,
+// source-pass step: 203 x 181 x 247 (44 tiles) 64 planes 115 us, 12 planes
+// 42 us; 266^3 64 planes 115 us, 16 planes (one whole round) 59 us; 64^3 64
+// planes 94 us, 8 planes 18 us. At 522^3 (256 tiles), where memory bounds the
+// step, 20 to 128 planes take 530 to 558 us.
+int planes_per_workgroup(int tiles, int n) {
+  const int resident = resident_workgroups();
+  long long best = -1;
+  int ych = n;
+  for (int chunks = 1; chunks <= n; ++chunks) {
+    const int c = (n + chunks - 1) / chunks;
+    if (c > AC3_MAX_CHUNK) continue;
+    const long long rounds = ((long long)tiles * ((n + c - 1) / c) + resident - 1) / resident;
+    const long long cost = rounds * (c + 6);
+    if (best < 0 || cost < best) {
+      best = cost;
+      ych = c;
+    }
+  }
+  return ych;
+}
+
 }  // namespace
 
 }  // namespace erm
@@ -336,6 +377,7 @@ struct ac3d {
   ac3d_cfg_t cfg{};
   size_t n = 0;
   long long plane = 0;
+  int ychunk = 0;  // planes per step workgroup
   DevBuf c, c_alt, k, f0, f1, rec, rec_tmp, snap, smax, img, amp_h_dummy;
   std::vector<float> amp;
   std::vector<float> scales;  // per snapshot (host copy after the source pass)
@@ -373,13 +415,7 @@ static int ac3_launch(ac3d* a, const float* p, float* pp, const float* c, int mo
   x.snap_scale = scale;
   x.snap_bf16 = g.snap_prec == 1;
   x.img = img;
-  // planes per workgroup along y (RTM_AC3_YCHUNK overrides; experiments)
-  static const int ychunk = [] {
-    const char* e = getenv("RTM_AC3_YCHUNK");
-    const int v = e ? atoi(e) : 64;
-    return v >= 8 ? v : 64;
-  }();
-  x.ychunk = ychunk;
+  x.ychunk = a->ychunk;
   const int nbz = (g.n1 - 10 + AZ - 1) / AZ, nbx = (g.n2 - 10 + AX - 1) / AX;
   const int nby = (g.n3 - 10 + x.ychunk - 1) / x.ychunk;
   if (mode == 1 && img)
@@ -460,6 +496,11 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
     return E_ARG;
   }
   a->plane = (long long)g.n2 * g.n3;
+  // RTM_AC3_YCHUNK overrides the planes per workgroup (experiments)
+  const char* fixed = getenv("RTM_AC3_YCHUNK");
+  a->ychunk = fixed && atoi(fixed) > 0
+                  ? atoi(fixed)
+                  : planes_per_workgroup(((g.n1 - 10 + AZ - 1) / AZ) * ((g.n2 - 10 + AX - 1) / AX), g.n3 - 10);
   HIPCHK(hipStreamCreateWithFlags(&a->st, hipStreamNonBlocking));
   for (auto& e : a->ev) HIPCHK(hipEventCreate(&e));
   STCHK(a->c.alloc(a->n * 4, "velocity term"));

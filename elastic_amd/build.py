@@ -17,11 +17,15 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librtm_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
+# Kernel arguments are preloaded into scalar registers while a launch is being
+# dispatched, instead of being loaded by each wave first: 0.3 to 0.5 us of a 4
+# to 9 us step launch on small grids.
 # Packed-FP32 VALU forms are disabled for all device code; the compiler still
 # vectorises ordinary float code with the other instructions.
 HIP_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
 

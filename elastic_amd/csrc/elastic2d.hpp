@@ -71,7 +71,7 @@ enum : int {
   F_RECSUB = 2,  // record by subtracting (observed = true - smooth)
   F_K = 4,       // apply the sponge
   F_SRC = 8,     // inject the explosive source
-  F_BORN = 16,   // add the Born sources bsrc
+  F_BORN = 16,   // add the Born sources (marching forward: from bsrc)
   F_SNAP = 32,   // write the source-wavefield snapshot belonging to this step
   F_NTS = 64,    // non-temporal stores of the new level
   F_SNAP2 = 128  // two-level step: also write the snapshot of level L
@@ -104,13 +104,25 @@ __device__ __forceinline__ int xcd_tile(int L, int N) {
 // x-cells, 256 threads, radius-5 halo staged in LDS.
 constexpr int TILE_Z = 64;
 constexpr int TILE_WY = 4;
-inline int tile_x(int txr) { return TILE_WY * txr; }
+// Tile width 1 with fp32 snapshots and one level per launch: one cell per
+// thread in eight waves, 64 x 8 cells (width code kSmallTile): the cells of
+// width 2's tile over twice the waves, so a thread's chain of loads, stencils
+// and stores is half as long and twice the waves hide it. With 16-bit
+// snapshots, whose scales go by the width, and two levels per launch the tile
+// of width 1 is 64 x 4.
+constexpr int kSmallTile = -1;
+constexpr int SMALL_WY = 8;
+inline int tile_code(int txr, int tblock, int snap_fmt) {
+  return txr == 1 && tblock == 0 && snap_fmt <= SNAP_F32 ? kSmallTile : txr;
+}
+inline int tile_x(int txr) { return txr == kSmallTile ? SMALL_WY : TILE_WY * txr; }
 
-// Step launches over a tile table covering one or many shots.
+// Step launches over a tile table covering one or many shots; for one shot,
+// nbz (its tiles along z) lets the kernel do without the table.
 int launch_fwd(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags,
-               int txr, int snap_fmt, int xcd, hipStream_t st);
+               int txr, int snap_fmt, int xcd, hipStream_t st, int nbz = 0);
 int launch_adj(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags,
-               int txr, int snap_fmt, int xcd, hipStream_t st);
+               int txr, int snap_fmt, int xcd, hipStream_t st, int nbz = 0);
 // Levels L and L+1 in one pass (temporal blocking; TXR 1, 2, 4). The ring
 // must hold four levels. No Born sources.
 int launch_fwd2(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags,
@@ -137,9 +149,10 @@ int fwdm_resident_blocks(int nw, int snap_fmt);
 // Snapshot of the last level (no later step writes it): dV = 0.
 int launch_snap_last(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int txr,
                      int snap_fmt, hipStream_t st);
-// Born scattering sources of level L of every shot (image_op2 forward branch).
-int launch_born_sources(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int txr,
-                        hipStream_t st);
+// Born scattering sources of level L of every shot (image_op2 forward branch)
+// into bsrc, for the marching forward; the tile forward forms them itself.
+// The tile table is that of tile width 2.
+int launch_born_sources(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, hipStream_t st);
 
 int launch_fill(float* out, size_t n, float value, hipStream_t st);
 int launch_apply_k(float* f, int nz, int nx, int ldz, const float* kz, const float* kx,

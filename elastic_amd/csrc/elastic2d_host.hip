@@ -96,11 +96,16 @@ static int op3(int nt, int nz, int nx, float* const* hist, const float* const* c
   d.nz = nz; d.nx = nx; d.ldz = ldz; d.nt = nt; d.n2 = n2;
   d.lev = hp; d.lev_stride = n2; d.fstride = (long long)nt * n2; d.lev_mod = nt; d.lev_off = 0;
   d.coef = cf.as<float>();
-  const int txr = default_txr();
+  const int width = single_shot_txr(SNAP_HIST);
+  const int txr = tile_code(width, default_tblock() == 2 ? 2 : 0, SNAP_HIST);
   // kernel form 2 (RTM_TBLOCK=2): strips of RTM_MARCH_W columns marching
   // along x (form 3 marches the forward only: tiles here)
   const bool march = default_tblock() == 2;
   const int mw = default_march_w(), mnw = default_march_nw();
+  if (!march && width != 1 && width != 2 && width != 4 && width != 8) {
+    set_error("unsupported tile width %d", width);
+    return E_ARG;
+  }
   if (march && (mw < 2 || (mw & 1))) { set_error("RTM_MARCH_W=%d is not a positive even number", mw); return E_ARG; }
   const int tx = march ? mw : tile_x(txr), tz = march ? TILE_Z * mnw : TILE_Z;
   const int nbz = (nz + tz - 1) / tz, nbx = (nx + tx - 1) / tx;
@@ -118,7 +123,7 @@ static int op3(int nt, int nz, int nx, float* const* hist, const float* const* c
                         default_xcd(), st));
     else
       STCHK(launch_adj(dd.as<ShotDev>(), dt.as<TileRef>(), (int)tiles.size(), it, A_XIN, txr, SNAP_HIST,
-                       default_xcd(), st));
+                       default_xcd(), st, nbz));
   }
   HIPCHK(hipEventRecord(e1, st));
   for (int f = 0; f < 5; ++f)
@@ -212,9 +217,10 @@ static int op3_noalloc(int nt, int nz, int nx, float* const* hist, const float* 
     return E_ARG;
   }
   const bool march = default_tblock() == 2;
-  const int txr = default_txr(), mw = default_march_w(), mnw = default_march_nw();
+  const int width = single_shot_txr(SNAP_HIST);
+  const int txr = tile_code(width, default_tblock() == 2 ? 2 : 0, SNAP_HIST), mw = default_march_w(), mnw = default_march_nw();
   if (march && (mw < 2 || (mw & 1))) { set_error("RTM_MARCH_W=%d is not a positive even number", mw); return E_ARG; }
-  if (!march && txr != 1 && txr != 2 && txr != 4 && txr != 8) { set_error("unsupported tile width %d", txr); return E_ARG; }
+  if (!march && width != 1 && width != 2 && width != 4 && width != 8) { set_error("unsupported tile width %d", width); return E_ARG; }
   const int tx = march ? mw : tile_x(txr), tz = march ? TILE_Z * mnw : TILE_Z;
   const int nbz = (nz + tz - 1) / tz, nbx = (nx + tx - 1) / tx, ntiles = nbz * nbx;
   const size_t n2 = (size_t)nz * nx;
@@ -265,7 +271,7 @@ static int op3_noalloc(int nt, int nz, int nx, float* const* hist, const float* 
     if (march)
       STCHK(launch_adjm(dd, tt, ntiles, it, A_XIN, mw, mnw, SNAP_HIST, default_xcd(), st));
     else
-      STCHK(launch_adj(dd, tt, ntiles, it, A_XIN, txr, SNAP_HIST, default_xcd(), st));
+      STCHK(launch_adj(dd, tt, ntiles, it, A_XIN, txr, SNAP_HIST, default_xcd(), st, nbz));
     for (int f = 0; f < 5; ++f)
       HIPCHK(hipMemcpyAsync(hist[f] + (size_t)it * n2, slot(it) + f * n2, n2 * sizeof(float), hipMemcpyDeviceToHost,
                             st));
@@ -284,7 +290,7 @@ static int single_engine(Engine& e, const rtm_shot_t* s, const float* coef5, con
   cfg.snap_fmt = snap_fmt;
   cfg.modelling = modelling;
   cfg.comp = s->comp_image;
-  cfg.txr = default_txr();
+  cfg.txr = single_shot_txr(snap_fmt);
   cfg.xcd = default_xcd();
   cfg.tblock = default_tblock();
   cfg.march_w = default_march_w();
@@ -521,7 +527,7 @@ RTM_EXPORT int rtm_forward_movie_hip(const rtm_shot_t* s, const float* coef5, co
   HIPCHK(hipDeviceSynchronize());
   EngineCfg cfg;
   cfg.nt = s->nt; cfg.dx = s->dx; cfg.dt = s->dt; cfg.abc = s->abc;
-  cfg.txr = default_txr();
+  cfg.txr = single_shot_txr(SNAP_HIST);
   cfg.xcd = default_xcd();
   cfg.tblock = default_tblock();
   cfg.march_w = default_march_w();

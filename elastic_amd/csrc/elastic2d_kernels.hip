@@ -24,10 +24,11 @@
 
 namespace erm {
 
-template <int TXR>
+template <int TXR, int WAVES = TILE_WY>
 struct Tile {
   static constexpr int TZ = TILE_Z;
-  static constexpr int WY = TILE_WY;
+  static constexpr int WY = WAVES;
+  static constexpr int NT = TZ * WY;  // threads
   static constexpr int TX = WY * TXR;
   static constexpr int H = 5;
   static constexpr int LZ = TZ + 2 * H;  // LDS column length (z incl. halo)
@@ -129,6 +130,49 @@ __device__ __forceinline__ T gldm(const T* p, int i, bool in) {
   return in ? v : T(0);
 }
 
+// Born scattering sources of one cell of level L (image_op2's forward branch,
+// W/image-mod-rtm.f90:146-162) from the background Vx, Vz tiles hx, hz at LDS
+// position p, the next level's Vx, Vz (next) and the perturbation d. Fused only
+// where written, so that every caller rounds it the same way.
+template <int SX>
+__device__ __forceinline__ void born_sources(const ShotDev& S, const float* hx, const float* hz, int p, int gz, int gx,
+                                             bool has_next, const float (&next)[2], const float (&d)[3],
+                                             float (&q)[5]) {
+#pragma clang fp contract(off)
+  const int nz = S.nz, nx = S.nx;
+  float s1 = 0.f, s2 = 0.f, s4 = 0.f, s5 = 0.f, s6 = 0.f;
+  if (has_next) {
+    s1 = S.inv_dt * (next[0] - hx[p]);
+    s2 = S.inv_dt * (next[1] - hz[p]);
+  }
+  if (gz >= 4 && gz <= nz - 6 && gx >= 4 && gx <= nx - 6) {
+    s4 = sp<SX>(hx, p) * S.inv_dx;
+    s5 = sp<1>(hz, p) * S.inv_dx;
+  }
+  if (gz >= 5 && gz <= nz - 6 && gx >= 5 && gx <= nx - 6) {
+    s6 = sm<1>(hx, p) * S.inv_dx;
+    s6 = fmaf(sm<SX>(hz, p), S.inv_dx, s6);
+  }
+  const float s3 = s4 + s5;
+  q[0] = d[0] * s1;
+  q[1] = d[0] * s2;
+  q[2] = fmaf(-(d[2] * 2.f), s4, -(d[1] * s3));
+  q[3] = fmaf(-(d[2] * 2.f), s5, -(d[1] * s3));
+  q[4] = -(d[2] * s6);
+}
+
+// The tile of this workgroup. A launch over one shot (nbz: its tiles along z)
+// works it out from the workgroup's number, which is one dependent memory
+// latency less than the table's entry (about 0.5 us of a 5 us launch on small
+// grids); several shots share a table.
+template <int TX>
+__device__ __forceinline__ TileRef tile_of(const TileRef* tiles, int ntiles, int xcd, int nbz) {
+  const int b = xcd ? xcd_tile(blockIdx.x, ntiles) : (int)blockIdx.x;
+  if (nbz == 0) return tiles[b];
+  const int bx = b / nbz;
+  return TileRef{0, (b - bx * nbz) * TILE_Z, bx * TX, b};
+}
+
 // ---------------------------------------------------------------------------
 // Forward step, W/rtm-mod-adj.f90:225-252 (Born propagation :323-348):
 //   Vx  = K(Vx(L-2)  + m1_x (S-x sxx + S+z sxz))            Ax, Bx
@@ -138,17 +182,23 @@ __device__ __forceinline__ T gldm(const T* p, int i, bool in) {
 //   sxz = K(sxz(L-2) + m3 (S-z Vx + S-x Vz))                H, J
 // all differences of level L-1. Coefficients are zero outside each
 // operator's range, which reproduces the reference loop bounds exactly.
+// BORN (Born modelling): the scattering sources of level L are formed in the
+// same pass from the background history, instead of a launch of their own that
+// wrote and read five fields more (231 x 347: 10.5 + 6.2 us a level -> 4.9).
+// Every load of a step, the sponge factors and the source amplitude among
+// them, is issued before the barrier.
 // With F_SNAP the step also stores the snapshot of the imaging level L-1
 // (Vx, Vz of L-1 from the staged tile and dV = V(L) - V(L-1)), or with
 // SNAP_HIST the Vx, Vz of level L.
-template <int TXR, int SNAP>
-__global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
+template <int TXR, int SNAP, int WY = TILE_WY, bool BORN = false>
+__global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__ shots,
                                              const TileRef* __restrict__ tiles, int ntiles, int L,
-                                             int flags, int xcd) {
-  using T = Tile<TXR>;
-  constexpr int NIT = (T::N + 255) / 256;  // staged cells per thread
-  __shared__ float sh[5][T::N];
-  const TileRef tr = tiles[xcd ? xcd_tile(blockIdx.x, ntiles) : (int)blockIdx.x];
+                                             int flags, int xcd, int nbz) {
+  using T = Tile<TXR, WY>;
+  constexpr int NIT = (T::N + T::NT - 1) / T::NT;  // staged cells per thread
+  static_assert(!BORN || SNAP == SNAP_HIST, "Born sources come from the fp32 history");
+  __shared__ float sh[BORN ? 7 : 5][T::N];
+  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz);
   const ShotDev& S = shots[tr.shot];
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   // offsets inside one field are 32-bit (5 * n2 < 2^31, checked by the
@@ -169,7 +219,7 @@ __global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
   float st[NIT][5];
 #pragma unroll
   for (int k = 0; k < NIT; ++k) {
-    const int c = tid + 256 * k;
+    const int c = tid + T::NT * k;
     const int lx = c / T::LZ, lz = c - lx * T::LZ;
     const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
     const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
@@ -177,31 +227,64 @@ __global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
 #pragma unroll
     for (int f = 0; f < 5; ++f) st[k][f] = gldm(y1 + f * fs, gi, in);
   }
+  // Born: the background Vx, Vz of level L over the tile and its halo, of the
+  // next level at the own cells, and the model perturbation
+  const float* const bg = BORN ? static_cast<const float*>(S.snap) + (long long)(L - 1) * 2 * (long long)n2 : nullptr;
+  const bool bnext = BORN && L < S.nt;
+  float bs[BORN ? NIT : 1][2];
+  if (BORN) {
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+      const int c = tid + T::NT * k;
+      const int lx = c / T::LZ, lz = c - lx * T::LZ;
+      const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
+      const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
+      const int gi = gz + ldz * gx;
+      bs[k][0] = gldm(bg, gi, in);
+      bs[k][1] = gldm(bg + n2, gi, in);
+    }
+  }
   const int gz = z0 + tz;
   const bool zok = gz < nz;
-  float ox[TXR][5], oc[TXR][5];
+  // sponge factors and the source amplitude: loaded with the rest (after the
+  // barrier each would be one more memory latency before the stores)
+  const bool sponge = flags & F_K;
+  const float kz = sponge ? gld(S.kz, zok ? gz : 0) : 1.f;
+  const float amp = (flags & F_SRC) ? gldu(S.src_amp, L - 1) : 0.f;
+  float ox[TXR][5], oc[TXR][5], kx[TXR];
+  float bn[BORN ? TXR : 1][2], bd[BORN ? TXR : 1][3];
 #pragma unroll
   for (int j = 0; j < TXR; ++j) {
     const int gx = x0 + ty * TXR + j;
     const bool ok = zok && gx < nx;
     const int gi = gz + ldz * gx;
+    kx[j] = sponge ? gldu(S.kx, __builtin_amdgcn_readfirstlane(min(gx, nx - 1))) : 1.f;
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
       ox[j][f] = gld(x2 + f * fs, ok ? gi : 0);
       oc[j][f] = gld(coef + f * n2, ok ? gi : 0);
     }
+    if (BORN) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a) bn[j][a] = gld(bg + (bnext ? 2 + a : a) * n2, ok ? gi : 0);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) bd[j][a] = gld(S.dm + a * n2, ok ? gi : 0);
+    }
   }
 #pragma unroll
   for (int k = 0; k < NIT; ++k) {
-    const int c = tid + 256 * k;
+    const int c = tid + T::NT * k;
     if (c < T::N) {
 #pragma unroll
       for (int f = 0; f < 5; ++f) sh[f][c] = st[k][f];
+      if (BORN) {
+        sh[BORN ? 5 : 0][c] = bs[BORN ? k : 0][0];
+        sh[BORN ? 6 : 0][c] = bs[BORN ? k : 0][1];
+      }
     }
   }
   __syncthreads();
 
-  const float kz = ((flags & F_K) && zok) ? gld(S.kz, gz) : 1.f;
   constexpr int SX = T::LZ;
   float sv[4][TXR];
 #pragma unroll
@@ -218,9 +301,13 @@ __global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
     float v[5];
 #pragma unroll
     for (int f = 0; f < 5; ++f) v[f] = ox[j][f];
-    if (flags & F_BORN) {
+    if (BORN) {
+      float q[5];
+      const float* const hx = sh[BORN ? 5 : 0];
+      const float* const hz = sh[BORN ? 6 : 0];
+      born_sources<SX>(S, hx, hz, p, gz, gx, bnext, bn[BORN ? j : 0], bd[BORN ? j : 0], q);
 #pragma unroll
-      for (int f = 0; f < 5; ++f) v[f] = gld(S.bsrc + f * n2, gi) + v[f];
+      for (int f = 0; f < 5; ++f) v[f] = q[f] + v[f];
     }
     const float dxx_xm = sm<SX>(sh[2], p);  // Ax
     const float dxz_zp = sp<1>(sh[4], p);   // Bx
@@ -235,7 +322,6 @@ __global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
     v[1] = fmaf(m1z, dxz_xp, v[1]);
     v[1] = fmaf(m1z, dzz_zm, v[1]);
     if ((flags & F_SRC) && gz == S.zs && gx == S.xs) {
-      const float amp = gld(S.src_amp, L - 1);
       v[2] = v[2] + amp;
       v[3] = v[3] + amp;
     }
@@ -245,10 +331,9 @@ __global__ __launch_bounds__(256) void k_fwd(const ShotDev* __restrict__ shots,
     v[3] = fmaf(m2m3, dvz_zp, v[3]);
     v[4] = fmaf(m3, dvx_zm, v[4]);
     v[4] = fmaf(m3, dvz_xm, v[4]);
-    if (flags & F_K) {
-      const float kx = gldu(S.kx, gx);
+    if (sponge) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) v[f] = (v[f] * kz) * kx;
+      for (int f = 0; f < 5; ++f) v[f] = (v[f] * kz) * kx[j];
     }
     if (flags & F_NTS) {
 #pragma unroll
@@ -767,14 +852,19 @@ struct SrcView {
 // level L+2. K' is the sponge (exact adjoint) or identity (the drop-in).
 // With A_IMG the Lame imaging condition of level L (W/image-mod-rtm.f90:
 // 154-162 with S1..S6 of :26-67) is accumulated in the same pass.
-template <int TXR, int SNAP>
-__global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
+template <int TXR, int SNAP, int WY = TILE_WY>
+__global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__ shots,
                                              const TileRef* __restrict__ tiles, int ntiles, int L,
-                                             int flags, int xcd) {
-  using T = Tile<TXR>;
-  constexpr int NIT = (T::N + 255) / 256;
-  __shared__ float sh[5][T::N];
-  const TileRef tr = tiles[xcd ? xcd_tile(blockIdx.x, ntiles) : (int)blockIdx.x];
+                                             int flags, int xcd, int nbz) {
+  using T = Tile<TXR, WY>;
+  constexpr int NIT = (T::N + T::NT - 1) / T::NT;
+  // the eight-wave tile: branch-free loads, and the source fields staged beside
+  // the products (one barrier a level instead of three; 300 x 300: 7.5 us a
+  // launch with four waves, 6.2 with this)
+  constexpr bool kEarly = SNAP == SNAP_HIST || SNAP == SNAP_F32;
+  constexpr bool kSmall = kEarly && WY != TILE_WY;
+  __shared__ float sh[kSmall ? 7 : 5][T::N];
+  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz);
   const ShotDev& S = shots[tr.shot];
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   const long long fs = S.fstride;
@@ -792,15 +882,17 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
   float st[NIT][5];
 #pragma unroll
   for (int k = 0; k < NIT; ++k) {
-    const int c = tid + 256 * k;
+    const int c = tid + T::NT * k;
     const int lx = c / T::LZ, lz = c - lx * T::LZ;
     const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
     const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
     // With the fp32 history out-of-range cells issue no loads; with
     // decimated snapshots the loads are branch-free (clamped index, masked
-    // products). Each form measured faster for its format.
+    // products). Each form measured faster for its format with four waves; in
+    // the first form a cell's loads end before the next cell's begin, so the
+    // eight-wave tile takes the second one.
     float p0 = 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f, p4 = 0.f;
-    if (SNAP != SNAP_HIST || in) {
+    if (SNAP != SNAP_HIST || kSmall || in) {
       const int gi = in ? gz + ldz * gx : 0;
       const float vx = gld(y1, gi), vz = gld(y1 + fs, gi), xx = gld(y1 + 2 * fs, gi), zz = gld(y1 + 3 * fs, gi),
                   xz = gld(y1 + 4 * fs, gi);
@@ -821,7 +913,10 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
   const int gz = z0 + tz;
   const bool zok = gz < nz;
   const bool row = (flags & A_INJ) && gz == S.zr;
-  float b[TXR][5];
+  const bool sponge = flags & A_K;
+  const float kz = sponge ? gld(S.kz, zok ? gz : 0) : 1.f;
+  const bool tile_row = (flags & A_INJ) && S.zr >= z0 && S.zr < z0 + T::TZ;  // the tile holds the receiver row
+  float b[TXR][5], kx[TXR], inj[TXR][5];
 #pragma unroll
   for (int j = 0; j < TXR; ++j) {
     const int gx = x0 + ty * TXR + j;
@@ -829,14 +924,18 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
     const int gi = gz + ldz * gx;
 #pragma unroll
     for (int f = 0; f < 5; ++f) b[j][f] = gld(x2 + f * fs, ok ? gi : 0);  // used where ok only
+    kx[j] = sponge ? gldu(S.kx, __builtin_amdgcn_readfirstlane(min(gx, nx - 1))) : 1.f;
+    // the level's own content (drop-in form) or the receiver row, added after
+    // the barrier: nothing waits for it here
     if (flags & A_XIN) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) b[j][f] = gld(out + f * fs, ok ? gi : 0) + b[j][f];
-    } else if (!(flags & A_KSRC) && ok && row && gx >= S.rx0 && gx < S.rx0 + S.nrx) {
-      const float* r = S.rec + (long long)(L - 1) * S.nrx + (gx - S.rx0);
+      for (int f = 0; f < 5; ++f) inj[j][f] = gld(out + f * fs, ok ? gi : 0);
+    } else if (tile_row) {
+      const bool in = row && gx >= S.rx0 && gx < S.rx0 + S.nrx;
+      const float* r = S.rec + (long long)(L - 1) * S.nrx + (in ? gx - S.rx0 : 0);
       const long long rs = (long long)S.nt * S.nrx;
 #pragma unroll
-      for (int f = 0; f < 5; ++f) b[j][f] = gld(r + f * rs, 0) + b[j][f];
+      for (int f = 0; f < 5; ++f) inj[j][f] = gld(r + f * rs, 0);
     }
   }
   // Imaging inputs: the source Vx, Vz of level L with their halo, the
@@ -846,13 +945,12 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
   // need their strip scales too and are loaded after the step (fewer live
   // registers, higher occupancy, measured faster for them).
   const bool imaging = flags & A_IMG;  // uniform over the launch
-  constexpr bool kEarly = SNAP == SNAP_HIST || SNAP == SNAP_F32;
   const SrcView<SNAP> sv(S, L);
   float sx[NIT][2], nt2[TXR][2], im[TXR][3], imc[TXR][3];
   auto load_imaging = [&]() {
 #pragma unroll
     for (int k = 0; k < NIT; ++k) {
-      const int c = tid + 256 * k;
+      const int c = tid + T::NT * k;
       const int lx = c / T::LZ, lz = c - lx * T::LZ;
       const int gx = x0 - T::H + lx, gz2 = z0 - T::H + lz;
       const bool in = c < T::N && gx >= 0 && gx < nx && gz2 >= 0 && gz2 < nz;
@@ -878,15 +976,18 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
   if (kEarly && imaging) load_imaging();
 #pragma unroll
   for (int k = 0; k < NIT; ++k) {
-    const int c = tid + 256 * k;
+    const int c = tid + T::NT * k;
     if (c < T::N) {
 #pragma unroll
       for (int f = 0; f < 5; ++f) sh[f][c] = st[k][f];
+      if (kSmall && imaging) {
+        sh[kSmall ? 5 : 0][c] = sx[k][0];
+        sh[kSmall ? 6 : 0][c] = sx[k][1];
+      }
     }
   }
   __syncthreads();
 
-  const float kz = ((flags & A_K) && zok) ? gld(S.kz, gz) : 1.f;
   float o[TXR][5];
   constexpr int SX = T::LZ;
 #pragma unroll
@@ -899,17 +1000,12 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
     for (int f = 0; f < 5; ++f) o[j][f] = 0.f;
     if (!ok) continue;
     const int gi = gz + ldz * gx;
-    if (flags & A_KSRC) {
-      // R/Src sponge: the injection is added to the damped level L+2
-      const float kxx = gldu(S.kx, gx);
-      const bool inj = row && gx >= S.rx0 && gx < S.rx0 + S.nrx;
-      const float* r = S.rec + (long long)(L - 1) * S.nrx + (inj ? gx - S.rx0 : 0);
-      const long long rs = (long long)S.nt * S.nrx;
+    const bool add = (flags & A_XIN) || (row && gx >= S.rx0 && gx < S.rx0 + S.nrx);
 #pragma unroll
-      for (int f = 0; f < 5; ++f) {
-        b[j][f] = (b[j][f] * kz) * kxx;
-        if (inj) b[j][f] = gld(r + f * rs, 0) + b[j][f];
-      }
+    for (int f = 0; f < 5; ++f) {
+      // R/Src sponge: the injection is added to the damped level L+2
+      if (flags & A_KSRC) b[j][f] = (b[j][f] * kz) * kx[j];
+      if (add) b[j][f] = inj[j][f] + b[j][f];
     }
     float v0 = b[j][0] - sm<SX>(sh[0], p);
     v0 -= sp<1>(sh[2], p);
@@ -923,11 +1019,9 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
     // with the R/Src sponge, level 1 (read by no later step) keeps its
     // undamped value, which is also the one imaged
     const bool ksrc = flags & A_KSRC;
-    float kx = 1.f;
-    if ((flags & A_K) && (!ksrc || L >= 2)) {
-      kx = gldu(S.kx, gx);
+    if (sponge && (!ksrc || L >= 2)) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) v[f] = (v[f] * kz) * kx;
+      for (int f = 0; f < 5; ++f) v[f] = (v[f] * kz) * kx[j];
     }
     if (flags & A_NTS) {
 #pragma unroll
@@ -937,23 +1031,25 @@ __global__ __launch_bounds__(256) void k_adj(const ShotDev* __restrict__ shots,
       for (int f = 0; f < 5; ++f) gst(out + f * fs, gi, v[f]);
     }
 #pragma unroll
-    for (int f = 0; f < 5; ++f) o[j][f] = ksrc && L >= 3 ? (v[f] * kz) * kx : v[f];
+    for (int f = 0; f < 5; ++f) o[j][f] = ksrc && L >= 3 ? (v[f] * kz) * kx[j] : v[f];
   }
 
   if (!imaging) return;
   if (!kEarly) load_imaging();
-  // the source tile replaces the products in LDS
-  __syncthreads();
-  float* const ss[2] = {sh[0], sh[1]};
+  float* const ss[2] = {sh[kSmall ? 5 : 0], sh[kSmall ? 6 : 1]};
+  if (!kSmall) {
+    // the source tile replaces the products in LDS
+    __syncthreads();
 #pragma unroll
-  for (int k = 0; k < NIT; ++k) {
-    const int c = tid + 256 * k;
-    if (c < T::N) {
-      ss[0][c] = sx[k][0];
-      ss[1][c] = sx[k][1];
+    for (int k = 0; k < NIT; ++k) {
+      const int c = tid + T::NT * k;
+      if (c < T::N) {
+        ss[0][c] = sx[k][0];
+        ss[1][c] = sx[k][1];
+      }
     }
+    __syncthreads();
   }
-  __syncthreads();
   const bool next = flags & A_NEXT;
   const bool zin4 = gz >= 4 && gz <= nz - 6, zin5 = gz >= 5 && gz <= nz - 6;
   float* const img = S.img;
@@ -1381,33 +1477,17 @@ __global__ __launch_bounds__(256) void k_born_sources(const ShotDev* __restrict_
   if (gz >= nz) return;
   constexpr int SX = T::LZ;
   for (int j = 0; j < TXR; ++j) {
-#pragma clang fp contract(off)
     const int lxo = ty * TXR + j;
     const int gx = x0 + lxo;
     if (gx >= nx) break;
     const int p = (lxo + T::H) * T::LZ + (tz + T::H);
     const long long gi = (long long)gz + (long long)ldz * gx;
-    float s1 = 0.f, s2 = 0.f, s4 = 0.f, s5 = 0.f, s6 = 0.f;
-    if (h1) {
-      s1 = S.inv_dt * (h1[gi] - sh[0][p]);
-      s2 = S.inv_dt * (h1[n2 + gi] - sh[1][p]);
-    }
-    if (gz >= 4 && gz <= nz - 6 && gx >= 4 && gx <= nx - 6) {
-      s4 = sp<SX>(sh[0], p) * S.inv_dx;
-      s5 = sp<1>(sh[1], p) * S.inv_dx;
-    }
-    if (gz >= 5 && gz <= nz - 6 && gx >= 5 && gx <= nx - 6) {
-      s6 = sm<1>(sh[0], p) * S.inv_dx;
-      s6 = fmaf(sm<SX>(sh[1], p), S.inv_dx, s6);
-    }
-    const float s3 = s4 + s5;
-    const float d1 = S.dm[gi], d2 = S.dm[n2 + gi], d3 = S.dm[2 * n2 + gi];
-    float* src = S.bsrc;
-    src[gi] = d1 * s1;
-    src[n2 + gi] = d1 * s2;
-    src[2 * n2 + gi] = fmaf(-(d3 * 2.f), s4, -(d2 * s3));
-    src[3 * n2 + gi] = fmaf(-(d3 * 2.f), s5, -(d2 * s3));
-    src[4 * n2 + gi] = -(d3 * s6);
+    const float next[2] = {h1 ? h1[gi] : 0.f, h1 ? h1[n2 + gi] : 0.f};
+    const float d[3] = {S.dm[gi], S.dm[n2 + gi], S.dm[2 * n2 + gi]};
+    float q[5];
+    born_sources<SX>(S, sh[0], sh[1], p, gz, gx, h1 != nullptr, next, d, q);
+#pragma unroll
+    for (int f = 0; f < 5; ++f) S.bsrc[f * n2 + gi] = q[f];
   }
 }
 
@@ -2125,13 +2205,13 @@ __global__ void k_stack(double* stack, int snz, int snx, const float* img, int l
 // ---------------------------------------------------------------------------
 template <int TXR>
 static void fwd_dispatch(int snap, dim3 g, hipStream_t st, const ShotDev* s, const TileRef* t,
-                         int n, int L, int fl, int xcd) {
+                         int n, int L, int fl, int xcd, int nbz) {
   const dim3 b(TILE_Z, TILE_WY);
   switch (snap) {
-    case SNAP_HIST: hipLaunchKernelGGL((k_fwd<TXR, SNAP_HIST>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    case SNAP_F32: hipLaunchKernelGGL((k_fwd<TXR, SNAP_F32>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    case SNAP_BF16: hipLaunchKernelGGL((k_fwd<TXR, SNAP_BF16>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    default: hipLaunchKernelGGL((k_fwd<TXR, SNAP_F16>), g, b, 0, st, s, t, n, L, fl, xcd); break;
+    case SNAP_HIST: hipLaunchKernelGGL((k_fwd<TXR, SNAP_HIST>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    case SNAP_F32: hipLaunchKernelGGL((k_fwd<TXR, SNAP_F32>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    case SNAP_BF16: hipLaunchKernelGGL((k_fwd<TXR, SNAP_BF16>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    default: hipLaunchKernelGGL((k_fwd<TXR, SNAP_F16>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
   }
 }
 template <int TXR>
@@ -2147,13 +2227,13 @@ static void fwd2_dispatch(int snap, dim3 g, hipStream_t st, const ShotDev* s, co
 }
 template <int TXR>
 static void adj_dispatch(int snap, dim3 g, hipStream_t st, const ShotDev* s, const TileRef* t,
-                         int n, int L, int fl, int xcd) {
+                         int n, int L, int fl, int xcd, int nbz) {
   const dim3 b(TILE_Z, TILE_WY);
   switch (snap) {
-    case SNAP_HIST: hipLaunchKernelGGL((k_adj<TXR, SNAP_HIST>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    case SNAP_F32: hipLaunchKernelGGL((k_adj<TXR, SNAP_F32>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    case SNAP_BF16: hipLaunchKernelGGL((k_adj<TXR, SNAP_BF16>), g, b, 0, st, s, t, n, L, fl, xcd); break;
-    default: hipLaunchKernelGGL((k_adj<TXR, SNAP_F16>), g, b, 0, st, s, t, n, L, fl, xcd); break;
+    case SNAP_HIST: hipLaunchKernelGGL((k_adj<TXR, SNAP_HIST>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    case SNAP_F32: hipLaunchKernelGGL((k_adj<TXR, SNAP_F32>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    case SNAP_BF16: hipLaunchKernelGGL((k_adj<TXR, SNAP_BF16>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
+    default: hipLaunchKernelGGL((k_adj<TXR, SNAP_F16>), g, b, 0, st, s, t, n, L, fl, xcd, nbz); break;
   }
 }
 template <int TXR>
@@ -2180,14 +2260,44 @@ static void snap_last_dispatch(int snap, dim3 g, hipStream_t st, const ShotDev* 
 }
 
 int launch_fwd(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags, int txr,
-               int snap, int xcd, hipStream_t st) {
+               int snap, int xcd, hipStream_t st, int nbz) {
   if (ntiles <= 0) return OK;
   const dim3 g(ntiles);
+  if (flags & F_BORN) {
+    if (snap != SNAP_HIST) { set_error("Born sources need the fp32 history format"); return E_ARG; }
+    const dim3 b(TILE_Z, TILE_WY);
+    switch (txr) {
+      case 1: hipLaunchKernelGGL((k_fwd<1, SNAP_HIST, TILE_WY, true>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+      case 2: hipLaunchKernelGGL((k_fwd<2, SNAP_HIST, TILE_WY, true>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+      case 4: hipLaunchKernelGGL((k_fwd<4, SNAP_HIST, TILE_WY, true>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+      case 8: hipLaunchKernelGGL((k_fwd<8, SNAP_HIST, TILE_WY, true>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+      case kSmallTile:
+        hipLaunchKernelGGL((k_fwd<1, SNAP_HIST, SMALL_WY, true>), g, dim3(TILE_Z, SMALL_WY), 0, st, shots, tiles, ntiles, L,
+                           flags, xcd, nbz);
+        break;
+      default: set_error("unsupported tile width %d", txr); return E_ARG;
+    }
+    HIPCHK(hipGetLastError());
+    return OK;
+  }
+  if (txr == kSmallTile) {  // fp32 formats only
+    const dim3 b(TILE_Z, SMALL_WY);
+    if (snap == SNAP_HIST)
+      hipLaunchKernelGGL((k_fwd<1, SNAP_HIST, SMALL_WY>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz);
+    else if (snap == SNAP_F32)
+      hipLaunchKernelGGL((k_fwd<1, SNAP_F32, SMALL_WY>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz);
+    else {
+      set_error("the small tile has no 16-bit snapshots");
+      return E_ARG;
+    }
+    HIPCHK(hipGetLastError());
+    return OK;
+  }
   switch (txr) {
-    case 1: fwd_dispatch<1>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 2: fwd_dispatch<2>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 4: fwd_dispatch<4>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 8: fwd_dispatch<8>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
+    case 1: fwd_dispatch<1>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 2: fwd_dispatch<2>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 4: fwd_dispatch<4>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 8: fwd_dispatch<8>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
     default: set_error("unsupported tile width %d", txr); return E_ARG;
   }
   HIPCHK(hipGetLastError());
@@ -2210,14 +2320,27 @@ int launch_fwd2(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, i
 }
 
 int launch_adj(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags, int txr,
-               int snap, int xcd, hipStream_t st) {
+               int snap, int xcd, hipStream_t st, int nbz) {
   if (ntiles <= 0) return OK;
   const dim3 g(ntiles);
+  if (txr == kSmallTile) {  // fp32 formats only
+    const dim3 b(TILE_Z, SMALL_WY);
+    if (snap == SNAP_HIST)
+      hipLaunchKernelGGL((k_adj<1, SNAP_HIST, SMALL_WY>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz);
+    else if (snap == SNAP_F32)
+      hipLaunchKernelGGL((k_adj<1, SNAP_F32, SMALL_WY>), g, b, 0, st, shots, tiles, ntiles, L, flags, xcd, nbz);
+    else {
+      set_error("the small tile has no 16-bit snapshots");
+      return E_ARG;
+    }
+    HIPCHK(hipGetLastError());
+    return OK;
+  }
   switch (txr) {
-    case 1: adj_dispatch<1>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 2: adj_dispatch<2>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 4: adj_dispatch<4>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
-    case 8: adj_dispatch<8>(snap, g, st, shots, tiles, ntiles, L, flags, xcd); break;
+    case 1: adj_dispatch<1>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 2: adj_dispatch<2>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 4: adj_dispatch<4>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
+    case 8: adj_dispatch<8>(snap, g, st, shots, tiles, ntiles, L, flags, xcd, nbz); break;
     default: set_error("unsupported tile width %d", txr); return E_ARG;
   }
   HIPCHK(hipGetLastError());
@@ -2243,6 +2366,7 @@ int launch_snap_last(const ShotDev* shots, const TileRef* tiles, int ntiles, int
                      int snap, hipStream_t st) {
   if (ntiles <= 0 || snap == SNAP_HIST) return OK;
   const dim3 g(ntiles);
+  if (txr == kSmallTile) txr = 2;  // the same 64 x 8 cells (fp32 snapshots: no strips)
   switch (txr) {
     case 1: snap_last_dispatch<1>(snap, g, st, shots, tiles, L); break;
     case 2: snap_last_dispatch<2>(snap, g, st, shots, tiles, L); break;
@@ -2254,17 +2378,9 @@ int launch_snap_last(const ShotDev* shots, const TileRef* tiles, int ntiles, int
   return OK;
 }
 
-int launch_born_sources(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int txr,
-                        hipStream_t st) {
+int launch_born_sources(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, hipStream_t st) {
   if (ntiles <= 0) return OK;
-  const dim3 g(ntiles), b(TILE_Z, TILE_WY);
-  switch (txr) {
-    case 1: hipLaunchKernelGGL(k_born_sources<1>, g, b, 0, st, shots, tiles, L); break;
-    case 2: hipLaunchKernelGGL(k_born_sources<2>, g, b, 0, st, shots, tiles, L); break;
-    case 4: hipLaunchKernelGGL(k_born_sources<4>, g, b, 0, st, shots, tiles, L); break;
-    case 8: hipLaunchKernelGGL(k_born_sources<8>, g, b, 0, st, shots, tiles, L); break;
-    default: set_error("Born sources: unsupported tile width %d", txr); return E_ARG;
-  }
+  hipLaunchKernelGGL(k_born_sources<2>, dim3(ntiles), dim3(TILE_Z, TILE_WY), 0, st, shots, tiles, L);
   HIPCHK(hipGetLastError());
   return OK;
 }

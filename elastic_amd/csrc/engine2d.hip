@@ -29,6 +29,16 @@ int ensure_device() {
 // numbering; RTM_TXR / RTM_XCD_REMAP override them (experiments). The batch
 // API tunes the width per workload unless a width is given.
 int default_txr() { return env_int("RTM_TXR", 2); }
+// Single-shot calls: width 1 (eight waves of one cell per thread, see
+// tile_code) with fp32 snapshots, where it measured faster than width 2 on
+// every grid, us per level forward / adjoint: 64 x 64 3.7 / 5.6 against 4.7 /
+// 8.9; 300 x 300 4.1 / 6.2 against 5.0 / 9.1; 390 x 690 6.7 / 10.9 against
+// 7.4 / 12.7; 890 x 1290 16.9 / 30.1 against 17.7 / 37.1; 2000 x 4000 152 /
+// 247 against 153 / 269. Width 2 with 16-bit snapshots: their scales, and so
+// the images, go by the width.
+int single_shot_txr(int snap_fmt) {
+  return snap_fmt <= SNAP_F32 && !getenv("RTM_TXR") && default_tblock() == 0 ? 1 : default_txr();
+}
 int default_xcd() { return env_int("RTM_XCD_REMAP", 1); }
 // Non-temporal stores of the new level (RTM_NT=1).
 static int nt_stores() { return env_int("RTM_NT", 0); }
@@ -313,7 +323,7 @@ int Engine::build_groups() {
   fresident_ = march_fit_ ? march_resident(cfg_, true) : 0;
   const int ns = (int)specs_.size();
   std::vector<TileRef> tiles, strips;
-  const int tx = tile_x(cfg_.txr);
+  const int tx = tile_x(tile_code());
   const bool march = cfg_.tblock >= 2;  // forms 2, 3 march (3: the forward only)
   int s = 0;
   G_ = 0;
@@ -479,6 +489,12 @@ int Engine::fill_desc(int g, bool true_model, bool born_mode) {
   return OK;
 }
 
+// Tiles along z of a group of one shot (the step kernels then do without the
+// tile table), 0 for several shots.
+int Engine::single_nbz(const Group& gr) const {
+  return gr.shots.size() == 1 ? (specs_[gr.shots[0]].nz + TILE_Z - 1) / TILE_Z : 0;
+}
+
 // mode 0: imaging forward (migration model, snapshots); 1: record with the
 // true model (store); 2: record with the migration model (subtract);
 // 3: record with the migration model (store); 4: Born background (fp32
@@ -490,6 +506,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
   const TileRef* tiles = d_tiles_.as<TileRef>() + gr.tile0;
   const bool march = cfg_.tblock >= 2;
   const TileRef* strips = march ? d_strips_.as<TileRef>() + gr.fstrip0 : nullptr;
+  const int nbz = single_nbz(gr);
   const int snap = (mode == 0) ? cfg_.snap_fmt : SNAP_HIST;
   for (int s : gr.shots) {
     STCHK(launch_fill(ring_of(s), (size_t)5 * kRing * res_[s].n2, 0.f, st));
@@ -513,7 +530,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
     if (!born) fl |= F_SRC;
     if (born) {
       fl |= F_BORN | F_REC;
-      STCHK(launch_born_sources(desc, tiles, gr.ntiles, L, cfg_.txr, st));
+      if (march) STCHK(launch_born_sources(desc, tiles, gr.ntiles, L, st));
     }
     if (mode == 1 || mode == 3) fl |= F_REC;
     if (mode == 2) fl |= F_RECSUB;
@@ -532,7 +549,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
     else if (march)
       STCHK(launch_fwdm(desc, strips, gr.fnstrips, L, fl, gr.fmarch_w, cfg_.march_nw, snap, cfg_.xcd, st));
     else
-      STCHK(launch_fwd(desc, tiles, gr.ntiles, L, fl, cfg_.txr, snap, cfg_.xcd, st));
+      STCHK(launch_fwd(desc, tiles, gr.ntiles, L, fl, tile_code(), snap, cfg_.xcd, st, nbz));
     if (learn && L >= 3)
       STCHK(launch_labc_infer(cfg_.labc_w, desc, lcells, gr.nlband, gr.nlrim, L,
                               mode == 0 && cfg_.snap_fmt == SNAP_HIST, st));
@@ -553,7 +570,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
     L += two ? 2 : 1;
   }
   if (mode == 0 && cfg_.snap_fmt != SNAP_HIST && cfg_.nt % cfg_.snap_every == 0)
-    STCHK(launch_snap_last(desc, tiles, gr.ntiles, cfg_.nt, cfg_.txr, cfg_.snap_fmt, st));
+    STCHK(launch_snap_last(desc, tiles, gr.ntiles, cfg_.nt, tile_code(), cfg_.snap_fmt, st));
   return OK;
 }
 
@@ -563,6 +580,7 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
   const TileRef* tiles = d_tiles_.as<TileRef>() + gr.tile0;
   const bool march = cfg_.tblock == 2;  // form 3 marches the forward only
   const TileRef* strips = march ? d_strips_.as<TileRef>() + gr.strip0 : nullptr;
+  const int nbz = single_nbz(gr);
   for (size_t k = 0; k < gr.shots.size(); ++k) {
     Res& r = res_[gr.shots[k]];
     STCHK(launch_fill(ring_of(gr.shots[k]), (size_t)5 * kRing * r.n2, 0.f, st));
@@ -588,7 +606,7 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
     else if (march)
       STCHK(launch_adjm(desc, strips, gr.nstrips, L, fl, gr.march_w, cfg_.march_nw, cfg_.snap_fmt, cfg_.xcd, st));
     else
-      STCHK(launch_adj(desc, tiles, gr.ntiles, L, fl, cfg_.txr, cfg_.snap_fmt, cfg_.xcd, st));
+      STCHK(launch_adj(desc, tiles, gr.ntiles, L, fl, tile_code(), cfg_.snap_fmt, cfg_.xcd, st, nbz));
     if (lcells) STCHK(launch_labc_infer(cfg_.labc_wa, desc, lcells, gr.nlband, gr.nlrim, L, false, st, true));
     L -= two ? 2 : 1;
   }

@@ -170,6 +170,8 @@ class Engine {
     hipGraphExec_t gfwd = nullptr, gadj = nullptr, gsyn = nullptr;
   };
   int build_lcells();
+  int tile_code() const { return erm::tile_code(cfg_.txr, cfg_.tblock, cfg_.snap_fmt); }
+  int single_nbz(const Group& gr) const;
   int alloc_working();
   int build_groups();
   int fill_desc(int g, bool true_model, bool born_mode);
@@ -208,6 +210,8 @@ int fill_masked_coefs(const float* coef5, int nz, int nx, int ldz, float* dev, h
 void sponge_factors(int n, int abc, std::vector<float>& k);
 int ensure_device();
 int default_txr();
+// Tile width of the single-shot calls.
+int single_shot_txr(int snap_fmt);
 int default_xcd();
 int default_tblock();
 int default_march_w();

@@ -12,16 +12,19 @@
 // Here the gathers of one output along one axis are merged: the products
 // coefficient * field that share an axis and a tap set are summed first
 // (e.g. m2m3 sxx + m2 syy + m2 szz for Vx along x), which leaves 18 gathers
-// over 9 distinct product arrays. A workgroup of 64 x EW threads (EW = 8 or
-// 16 waves) owns a 64 (z) x EW (x) tile of the (z, x) plane and marches
-// along y over a chunk of planes:
-//   * the 6 products gathered along x, over the tile plus its 5-column
-//     x-halo, and the 6 gathered along z, over the tile plus its 5-row
+// over 9 distinct product arrays. The step falls into two halves that read
+// nothing in common: the velocity outputs come from the six stresses and m2,
+// m3, m2m3, the stress outputs from the three velocities and m1_x, m1_y, m1_z.
+// A workgroup of 16 waves computes one half of a tz (z) x tx (x) tile of the
+// (z, x) plane, at most 1024 cells, marching along y over a chunk of planes:
+//   * the 3 products gathered along x, over the tile plus its 5-column
+//     x-halo, and the 3 gathered along z, over the tile plus its 5-row
 //     z-halo, go to LDS;
-//   * the 6 products gathered along y live in an 11-deep register queue of
+//   * the 3 products gathered along y live in an 11-deep register queue of
 //     the thread's own column (planes y-5 .. y+5), refilled 5 planes ahead.
 // Each step moves 168 algorithmic bytes per cell (in, in1, out and the 6
-// coefficients read, out written): HBM-bound.
+// coefficients read, out written): HBM-bound once the loads of a plane are in
+// flight while the plane before it is computed (see el3_march).
 
 #include "../../include/elastic3d.h"
 #include "common.hpp"
@@ -40,10 +43,14 @@ namespace {
 enum { VY, VX, VZ, SYY, SXX, SZZ, SXY, SXZ, SYZ };
 enum { M1Y, M1X, M1Z, M2, M3, M2M3 };
 
-constexpr int EZ = 64;               // tile rows (z): one wave64
 constexpr int EH = 5;                // stencil radius
-constexpr int ELZ = EZ + 2 * EH;     // z-band rows (tile + z-halo)
-constexpr int NXH = 2 * EH * EZ;     // x-halo cells (10 columns x 64 rows)
+constexpr int ENT = 1024;            // threads of a workgroup: 16 waves
+constexpr int EZ = 64;               // tile rows (z) at most
+constexpr int EX = 22;               // tile columns (x) at most
+constexpr int EHN = 832;             // halo cells at most
+constexpr int EP = EZ + 2 * EH;      // rows of one product's column in LDS
+constexpr int EC = 3 * EP;           // a column's three products
+constexpr int EBAND = (2 * EX + 2 * EH) * EC;  // x-band (EX + 10 columns), z-band (EX)
 
 struct El3Args {
   int ny, nz, nx;
@@ -52,13 +59,23 @@ struct El3Args {
   const float* in1[9];
   float* out[9];
   const float* m[6];
+  int tz, tx;  // tile: tz <= EZ, tx <= EX, tz * tx <= ENT, 10 (tz + tx) <= EHN
   int nbz, nbx, ych, nblk;
   int xcd;
 };
 
-template <class T>
-__device__ __forceinline__ T gl(const T* p, int i) {
-  return ((const __attribute__((address_space(1))) T*)p)[i];
+// Element at byte offset o of a plane: a scalar base and a 32-bit lane offset.
+// (opaque() keeps the compiler from hoisting the sums of 33 array bases and a
+// lane's offset out of the march as 66 vector registers.)
+__device__ __forceinline__ unsigned opaque(unsigned o) {
+  asm volatile("" : "+v"(o));
+  return o;
+}
+__device__ __forceinline__ float gl(const float* plane, unsigned o) {
+  return *(const __attribute__((address_space(1))) float*)((const __attribute__((address_space(1))) char*)plane + o);
+}
+__device__ __forceinline__ void gs(float* plane, unsigned o, float v) {
+  *(__attribute__((address_space(1))) float*)((__attribute__((address_space(1))) char*)plane + o) = v;
 }
 
 // The 9 distinct products of one cell that the 18 gathers read:
@@ -68,31 +85,6 @@ __device__ __forceinline__ T gl(const T* p, int i) {
 //   Qx = m1_x Vx (x: sxx, y: sxy, z: sxz)   Qy = m1_y Vy (x: sxy, y: syy, z: syz)
 //   Qz = m1_z Vz (x: sxz, y: syz, z: szz); every other gather uses set B.
 enum { PX, PY, PZ, PXY, PXZ, PYZ, QX, QY, QZ };
-
-__device__ __forceinline__ void products(const El3Args& a, int gi, float p[9]) {
-  const float vy = gl(a.in[VY], gi), vx = gl(a.in[VX], gi), vz = gl(a.in[VZ], gi);
-  const float syy = gl(a.in[SYY], gi), sxx = gl(a.in[SXX], gi), szz = gl(a.in[SZZ], gi);
-  const float sxy = gl(a.in[SXY], gi), sxz = gl(a.in[SXZ], gi), syz = gl(a.in[SYZ], gi);
-  const float m1y = gl(a.m[M1Y], gi), m1x = gl(a.m[M1X], gi), m1z = gl(a.m[M1Z], gi);
-  const float m2 = gl(a.m[M2], gi), m3 = gl(a.m[M3], gi), m2m3 = gl(a.m[M2M3], gi);
-  p[PX] = fmaf(m2m3, sxx, m2 * (syy + szz));
-  p[PY] = fmaf(m2m3, syy, m2 * (szz + sxx));
-  p[PZ] = fmaf(m2m3, szz, m2 * (sxx + syy));
-  p[PXY] = m3 * sxy;
-  p[PXZ] = m3 * sxz;
-  p[PYZ] = m3 * syz;
-  p[QX] = m1x * vx;
-  p[QY] = m1y * vy;
-  p[QZ] = m1z * vz;
-}
-
-// LDS slots of the x-band (gathers along x) and the z-band (along z).
-constexpr int XB[6] = {PX, PXY, PXZ, QX, QY, QZ};
-constexpr int ZB[6] = {PXZ, PYZ, PZ, QZ, QX, QY};
-// register queue along y: planes y-5 .. y+5 of these products
-constexpr int YQ[6] = {PY, PXY, PYZ, QX, QY, QZ};
-// the own cell's x/z products that are not in the y-queue wait 5 planes
-constexpr int DL[3] = {PX, PZ, PXZ};
 
 // Gathers at cell i of products P along one axis, P(k) = product at i + k:
 //   set A: sum_d c_(6-d) (P(-d) - P(d-1))     set B: sum_d c_(6-d) (P(1-d) - P(d))
@@ -121,151 +113,306 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// EW waves per workgroup, one tile column (x) each: a 64 x EW tile.
-// Every input column is loaded once per plane by its owner, 5 planes ahead
-// (plane y+5): its y-products enter the queue and its other x/z products a
-// 5-plane delay line, so plane y's own cells reach LDS from registers; only
-// the x- and z-halo cells are loaded at plane y.
-template <int EW>
-__global__ __launch_bounds__(EZ * EW) __attribute__((amdgpu_waves_per_eu(4)))
-void k_el3_adj(const El3Args a) {
-  constexpr int ET = EZ * EW, ELX = EW + 2 * EH, NZH = 2 * EH * EW;
-  __shared__ float xs[6][ELX][EZ];   // x-band: [k][x0-5+lx][z0+lz]
-  __shared__ float zs[6][EW][ELZ];   // z-band: [k][x0+lx][z0-5+lz]
-  const int b = a.xcd ? xcd_tile(blockIdx.x, a.nblk) : (int)blockIdx.x;
+// The two halves. own(): the raw operands of a cell of the thread's own column;
+// halo(): those of a cell of the x-band (x) or of the z-band, whose three
+// products differ in two operands; queue(): the products along y; band slots
+// of the x- and z-band (the own cell's products that are not in the queue wait
+// 5 planes in registers, keep()).
+struct Velocity {  // outputs Vx, Vy, Vz
+  static constexpr int NO = 9, NH = 8, NK = 3, NF = 3;
+  static constexpr int OUT[NF] = {VX, VY, VZ};
+  static __device__ __forceinline__ void own(const El3Args& a, long long py, unsigned o, float (&w)[NO]) {
+    constexpr int f[6] = {SXX, SYY, SZZ, SXY, SXZ, SYZ};
+#pragma unroll
+    for (int k = 0; k < 6; ++k) w[k] = gl(a.in[f[k]] + py, o);
+    w[6] = gl(a.m[M2] + py, o);
+    w[7] = gl(a.m[M3] + py, o);
+    w[8] = gl(a.m[M2M3] + py, o);
+  }
+  static __device__ __forceinline__ void products(const float (&w)[NO], float (&p)[9]) {
+    p[PX] = fmaf(w[8], w[0], w[6] * (w[1] + w[2]));
+    p[PY] = fmaf(w[8], w[1], w[6] * (w[2] + w[0]));
+    p[PZ] = fmaf(w[8], w[2], w[6] * (w[0] + w[1]));
+    p[PXY] = w[7] * w[3];
+    p[PXZ] = w[7] * w[4];
+    p[PYZ] = w[7] * w[5];
+  }
+  static constexpr int QUEUE[3] = {PY, PXY, PYZ};
+  static constexpr int KEEP[3] = {PX, PZ, PXZ};
+  static constexpr int XB[3] = {PX, PXY, PXZ};
+  static constexpr int ZB[3] = {PZ, PYZ, PXZ};
+  // the band's own shear stress differs: x-band sxy, z-band syz
+  static __device__ __forceinline__ const float* split(const El3Args& a, bool x) { return x ? a.in[SXY] : a.in[SYZ]; }
+  static __device__ __forceinline__ void halo(const El3Args& a, const float* sp, long long py, unsigned o, float (&w)[NH]) {
+    w[0] = gl(a.in[SXX] + py, o);
+    w[1] = gl(a.in[SYY] + py, o);
+    w[2] = gl(a.in[SZZ] + py, o);
+    w[3] = gl(sp + py, o);
+    w[4] = gl(a.in[SXZ] + py, o);
+    w[5] = gl(a.m[M2] + py, o);
+    w[6] = gl(a.m[M3] + py, o);
+    w[7] = gl(a.m[M2M3] + py, o);
+  }
+  static __device__ __forceinline__ void halo_products(const float (&w)[NH], bool x, float (&p)[3]) {
+    const float d = x ? w[0] : w[2], e = x ? w[2] : w[0];
+    p[0] = fmaf(w[7], d, w[5] * (w[1] + e));
+    p[1] = w[6] * w[3];
+    p[2] = w[6] * w[4];
+  }
+  template <class FX, class FY, class FZ>
+  static __device__ __forceinline__ void gather(FX X, FY Y, FZ Z, float (&g)[NF]) {
+    g[0] = gather_a(X(0)) + gather_b(Y(1)) + gather_b(Z(2));
+    g[1] = gather_a(Y(0)) + gather_b(Z(1)) + gather_b(X(1));
+    g[2] = gather_a(Z(0)) + gather_b(Y(2)) + gather_b(X(2));
+  }
+};
+struct Stress {  // the six stress outputs
+  static constexpr int NO = 6, NH = 6, NK = 0, NF = 6;
+  static constexpr int OUT[NF] = {SXX, SYY, SZZ, SXY, SXZ, SYZ};
+  static __device__ __forceinline__ void own(const El3Args& a, long long py, unsigned o, float (&w)[NO]) {
+    w[0] = gl(a.in[VX] + py, o);
+    w[1] = gl(a.in[VY] + py, o);
+    w[2] = gl(a.in[VZ] + py, o);
+    w[3] = gl(a.m[M1X] + py, o);
+    w[4] = gl(a.m[M1Y] + py, o);
+    w[5] = gl(a.m[M1Z] + py, o);
+  }
+  static __device__ __forceinline__ void products(const float (&w)[NO], float (&p)[9]) {
+    p[QX] = w[3] * w[0];
+    p[QY] = w[4] * w[1];
+    p[QZ] = w[5] * w[2];
+  }
+  static constexpr int QUEUE[3] = {QX, QY, QZ};
+  static constexpr int KEEP[1] = {QX};  // none kept
+  static constexpr int XB[3] = {QX, QY, QZ};
+  static constexpr int ZB[3] = {QX, QY, QZ};
+  static __device__ __forceinline__ const float* split(const El3Args&, bool) { return nullptr; }
+  static __device__ __forceinline__ void halo(const El3Args& a, const float*, long long py, unsigned o, float (&w)[NH]) {
+    own(a, py, o, w);
+  }
+  static __device__ __forceinline__ void halo_products(const float (&w)[NH], bool, float (&p)[3]) {
+    p[0] = w[3] * w[0];
+    p[1] = w[4] * w[1];
+    p[2] = w[5] * w[2];
+  }
+  template <class FX, class FY, class FZ>
+  static __device__ __forceinline__ void gather(FX X, FY Y, FZ Z, float (&g)[NF]) {
+    g[0] = gather_b(X(0));
+    g[1] = gather_b(Y(1));
+    g[2] = gather_b(Z(2));
+    g[3] = gather_b(X(1)) + gather_b(Y(0));
+    g[4] = gather_b(Z(0)) + gather_b(X(2));
+    g[5] = gather_b(Z(1)) + gather_b(Y(2));
+  }
+};
+
+// One half of a tile's chunk. Every input column is loaded once per plane by
+// its owner, 5 planes ahead (plane y+5), so plane y's own cells reach the bands
+// from registers. The halo cells, at most one per thread, are loaded with the
+// own column's plane y+5 too, which is when the neighbouring tiles load them as
+// theirs (so the second read is an L2 hit), and their products wait in a
+// 5-plane ring in LDS that only the thread reads. All loads of a plane are
+// issued while the plane before it is computed, and the bands are
+// double-buffered (one barrier a plane, whose fences cover LDS only).
+template <class H>
+__device__ __forceinline__ void el3_march(const El3Args& a, int b, float* lds, float* ring) {
   const int bz = b % a.nbz;
   const int r = b / a.nbz;
   const int bx = r % a.nbx;
   const int yc = r / a.nbx;
-  const int z0 = bz * EZ, x0 = bx * EW, y0 = yc * a.ych;
+  const int tz = a.tz, tx = a.tx;
+  const int z0 = bz * tz, x0 = bx * tx, y0 = yc * a.ych;
   const int y1 = min(y0 + a.ych, a.ny);
   const int t = threadIdx.x;
-  const int lane = t & 63, w = t >> 6;
-  const int gz = z0 + lane, gx = x0 + w;
-  const bool own = gz < a.nz && gx < a.nx;
-  // the own column's products are needed (as LDS halo of valid cells) up to
-  // nz+5 / nx+5; beyond that the padded array ends
-  const bool ownp = gz < a.nz + EH && gx < a.nx + EH;
-  const int sx = a.sx, sy = a.sy;
-  auto at = [&](int iz, int ix, int iy) { return (iz + EH) + sx * (ix + EH) + sy * (iy + EH); };
+  const int lx = t / tz, lz = t - lx * tz;
+  const int gz = z0 + lz, gx = x0 + lx;
+  const bool act = lx < tx;
+  const bool own = act && gz < a.nz && gx < a.nx;
+  // the own column's products are needed (as halo of valid cells) up to nz+5 /
+  // nx+5; beyond that the padded array ends, and the lanes load its first cell,
+  // whose products no valid cell reads (so nothing is masked)
+  const bool ownp = act && gz < a.nz + EH && gx < a.nx + EH;
+  const unsigned oo0 = ownp ? 4u * (unsigned)((gz + EH) + a.sx * (gx + EH)) : 0u;
+  // halo cells: 10 columns of tz rows beside the tile (x-band), then 10 rows
+  // above and below its tx columns (z-band)
+  const int h2 = t - 2 * EH * tz;
+  const bool hx = h2 < 0, hact = h2 < 2 * EH * tx;
+  int hcol, hrow, hz, hc;
+  if (hx) {
+    const int c = t / tz;
+    hcol = c < EH ? c : c + tx;
+    hrow = t - c * tz;
+    hz = z0 + hrow;
+    hc = x0 - EH + hcol;
+  } else {
+    const int c = h2 / (2 * EH), rr = h2 - c * (2 * EH);
+    hrow = rr < EH ? rr : rr + tz;
+    hz = z0 - EH + hrow;
+    hc = x0 + c;
+    hcol = c + EX + 2 * EH;  // the z-band follows the x-band
+  }
+  const unsigned ho0 = hact && hz < a.nz + EH && hc < a.nx + EH ? 4u * (unsigned)((hz + EH) + a.sx * (hc + EH)) : 0u;
+  const int hdst = hact ? hcol * EC + hrow : 0;
+  const float* const hsp = H::split(a, hx);
+  // waves without halo cells skip their loads (EHN is whole waves: every lane
+  // of the others has a place in the ring)
+  const bool halo_wave = __builtin_amdgcn_readfirstlane(t) < 2 * EH * (tz + tx);
+  const int xo = (lx + EH) * EC + lz, zo = (EX + 2 * EH + lx) * EC + lz + EH;
+  const long long sy = a.sy;
+  auto plane = [&](int y) { return sy * (y + EH); };
 
-  float q[6][11];  // YQ products, slot j = plane y-5+j
-  float dl[3][6];  // DL products, slot j = plane y+j
-  // prime planes y0-5 .. y0+4
+  float q[3][11];                  // QUEUE products, slot j = plane y-5+j
+  float keep[H::NK > 0 ? H::NK : 1][6];  // KEEP products, slot j = plane y+j
+  // prime planes y0-5 .. y0+4 (the loop shifts the queue first)
 #pragma unroll
   for (int j = 0; j < 10; ++j) {
-    float p[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (ownp) products(a, at(gz, gx, y0 - 5 + j), p);
+    float w[H::NO], p[9];
+    H::own(a, plane(y0 - 5 + j), opaque(oo0), w);
+    H::products(w, p);
 #pragma unroll
-    for (int k = 0; k < 6; ++k) q[k][j] = p[YQ[k]];
-    if (j >= 5) {
+    for (int k = 0; k < 3; ++k) q[k][j + 1] = p[H::QUEUE[k]];
 #pragma unroll
-      for (int k = 0; k < 3; ++k) dl[k][j - 5] = p[DL[k]];
+    for (int k = 0; k < H::NK; ++k)
+      if (j >= 5) keep[k][j - 4] = p[H::KEEP[k]];
+  }
+  // halo products of planes y0 .. y0+4 into the ring
+  if (halo_wave) {
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      float h[H::NH], e[3];
+      H::halo(a, hsp, plane(min(y0 + j, a.ny + EH - 1)), opaque(ho0), h);
+      H::halo_products(h, hx, e);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) ring[(j * 3 + k) * EHN + t] = e[k];
     }
   }
+  float w[H::NO], h[H::NH];
+  auto load_next = [&](int y) {
+    H::own(a, plane(y + 5), opaque(oo0), w);
+    if (halo_wave) H::halo(a, hsp, plane(y + 5), opaque(ho0), h);
+  };
+  load_next(y0);
+  int slot = 0;  // (y - y0) % 5
 
   for (int y = y0; y < y1; ++y) {
-    // own column, plane y+5
+    float* const bd = lds + ((y - y0) & 1) * EBAND;
     {
-      float p[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (ownp) products(a, at(gz, gx, y + 5), p);
+      float p[9], c[9];
+      H::products(w, p);
 #pragma unroll
-      for (int k = 0; k < 6; ++k) q[k][10] = p[YQ[k]];
+      for (int k = 0; k < 3; ++k) {
 #pragma unroll
-      for (int k = 0; k < 3; ++k) dl[k][5] = p[DL[k]];
-    }
-    // own cells of plane y into LDS, from the queue (slot 5) and the delay line (slot 0)
-    {
-      float c[9];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) c[YQ[k]] = q[k][5];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) c[DL[k]] = dl[k][0];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        xs[k][w + EH][lane] = c[XB[k]];
-        zs[k][w][lane + EH] = c[ZB[k]];
+        for (int j = 0; j < 10; ++j) q[k][j] = q[k][j + 1];
+        q[k][10] = p[H::QUEUE[k]];
+        c[H::QUEUE[k]] = q[k][5];
       }
-    }
-    // x-halo: columns x0-5..x0-1 and x0+EW..x0+EW+4, 64 rows
 #pragma unroll
-    for (int h0 = 0; h0 < NXH; h0 += ET) {
-      const int h = h0 + t;
-      if (h < NXH) {
-        const int hc = h >> 6;
-        const int lx = hc < EH ? hc : hc + EW;
-        const int hx = x0 - EH + lx, hz = z0 + (h & 63);
-        float p[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (hz < a.nz + EH && hx < a.nx + EH) products(a, at(hz, hx, y), p);
+      for (int k = 0; k < H::NK; ++k) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) xs[k][lx][h & 63] = p[XB[k]];
+        for (int j = 0; j < 5; ++j) keep[k][j] = keep[k][j + 1];
+        keep[k][5] = p[H::KEEP[k]];
+        c[H::KEEP[k]] = keep[k][0];
       }
-    }
-    // z-halo: rows z0-5..z0-1 and z0+64..z0+68 of the EW columns
-    if (t < NZH) {
-      const int rr = t % (2 * EH), cc = t / (2 * EH);
-      const int lz = rr < EH ? rr : rr + EZ;
-      const int hz = z0 - EH + lz, hx = x0 + cc;
-      float p[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (hz < a.nz + EH && hx < a.nx + EH) products(a, at(hz, hx, y), p);
+      if (act) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) zs[k][cc][lz] = p[ZB[k]];
+        for (int k = 0; k < 3; ++k) {
+          bd[xo + k * EP] = c[H::XB[k]];
+          bd[zo + k * EP] = c[H::ZB[k]];
+        }
+      }
+      if (halo_wave) {
+        float e[3];
+        H::halo_products(h, hx, e);
+        float* const rg = ring + slot * 3 * EHN + t;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          if (hact) bd[hdst + k * EP] = rg[k * EHN];
+          rg[k * EHN] = e[k];
+        }
+      }
+      slot = slot == 4 ? 0 : slot + 1;
     }
     lds_barrier();
-
+    // this plane's out and in1, added after the gathers, then the next plane's
+    // operands
+    const unsigned oo = opaque(oo0);
+    float u[H::NF], v[H::NF], g[H::NF];
+#pragma unroll
+    for (int f = 0; f < H::NF; ++f) {
+      u[f] = gl(a.out[H::OUT[f]] + plane(y), oo);
+      v[f] = gl(a.in1[H::OUT[f]] + plane(y), oo);
+    }
+    load_next(y + 1 < y1 ? y + 1 : y);
     if (own) {
-      const int gi = at(gz, gx, y);
-      float o[9];
+      H::gather([&](int k) { return [&, k](int d) { return bd[xo + d * EC + k * EP]; }; },
+                [&](int k) { return [&, k](int d) { return q[k][5 + d]; }; },
+                [&](int k) { return [&, k](int d) { return bd[zo + d + k * EP]; }; }, g);
 #pragma unroll
-      for (int f = 0; f < 9; ++f) o[f] = gl(a.out[f], gi) + gl(a.in1[f], gi);
-      const int cx = w + EH, cz = lane + EH;
-      // XB / ZB / YQ slot of each product
-      auto X = [&](int k) { return [&, k](int d) { return xs[k][cx + d][lane]; }; };
-      auto Z = [&](int k) { return [&, k](int d) { return zs[k][w][cz + d]; }; };
-      auto Y = [&](int k) { return [&, k](int d) { return q[k][5 + d]; }; };
-      // XB = {PX, PXY, PXZ, QX, QY, QZ}, ZB = {PXZ, PYZ, PZ, QZ, QX, QY},
-      // YQ = {PY, PXY, PYZ, QX, QY, QZ}
-      o[VX] += gather_a(X(0)) + gather_b(Y(1)) + gather_b(Z(0));
-      o[VY] += gather_a(Y(0)) + gather_b(Z(1)) + gather_b(X(1));
-      o[VZ] += gather_a(Z(2)) + gather_b(Y(2)) + gather_b(X(2));
-      o[SXX] += gather_b(X(3));
-      o[SYY] += gather_b(Y(4));
-      o[SZZ] += gather_b(Z(3));
-      o[SXY] += gather_b(X(4)) + gather_b(Y(3));
-      o[SXZ] += gather_b(Z(4)) + gather_b(X(5));
-      o[SYZ] += gather_b(Z(5)) + gather_b(Y(5));
-#pragma unroll
-      for (int f = 0; f < 9; ++f) a.out[f][gi] = o[f];
+      for (int f = 0; f < H::NF; ++f) gs(a.out[H::OUT[f]] + plane(y), oo, (u[f] + v[f]) + g[f]);
     }
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-#pragma unroll
-      for (int j = 0; j < 10; ++j) q[k][j] = q[k][j + 1];
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-#pragma unroll
-      for (int j = 0; j < 5; ++j) dl[k][j] = dl[k][j + 1];
-    lds_barrier();
   }
 }
 
-// tile width in x (= waves per workgroup): RTM_EL3_W = 4, 8 or 16
-int default_el3_width() {
-  const char* s = std::getenv("RTM_EL3_W");
-  const int v = s ? std::atoi(s) : 8;
-  return (v == 4 || v == 16) ? v : 8;
+// Both halves in one launch, the two of a tile next to each other; 16 waves and
+// 146 KB of LDS, one workgroup a CU. What bounds a step is the traffic beyond
+// the L2 (171 + 37 B a cell against 168 algorithmic at 4.4 TB/s). Step at 200^3
+// (us, algorithmic GB/s): 64 x 8 tiles of 8 waves for both halves at once, a
+// plane's loads issued and awaited in that plane, 530 (2540; 267 + 39 B a
+// cell); next plane's loads in flight, 768 threads for both halves, 451; halves
+// apart, two workgroups of 512 threads a CU, 446; 1024 threads with the halo
+// loaded at plane y+5, 376 (3580). 64^3: 18 us; 260^3: 830 us (3560).
+__global__ __launch_bounds__(ENT) __attribute__((amdgpu_waves_per_eu(4))) void k_el3_adj(const El3Args a) {
+  __shared__ float lds[2 * EBAND];
+  __shared__ float ring[5 * 3 * EHN];
+  const int b = a.xcd ? xcd_tile(blockIdx.x, 2 * a.nblk) : (int)blockIdx.x;
+  if (b & 1)
+    el3_march<Stress>(a, b >> 1, lds, ring);
+  else
+    el3_march<Velocity>(a, b >> 1, lds, ring);
 }
 
-int default_el3_ychunk(int ny, int tiles) {
-  if (const char* s = std::getenv("RTM_EL3_YCHUNK")) {
-    const int v = std::atoi(s);
-    if (v > 0) return std::min(v, ny);
+// Workgroups resident at once: one per CU.
+int el3_resident() {
+  static const int n = [] {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+      return 256;
+    return cus;
+  }();
+  return n;
+}
+
+// Tile and planes per workgroup: the tiles along z as even as they come, as
+// many columns as the workgroup's threads and LDS take (RTM_EL3_W fixes them),
+// and the number of chunks along y (RTM_EL3_YCHUNK: their planes) that
+// minimises rounds of resident workgroups x (planes + EPRIME); a chunk's first
+// loads cost about that many planes.
+constexpr int EPRIME = 8;
+void el3_partition(El3Args& a) {
+  const char* ws = std::getenv("RTM_EL3_W");
+  const char* ys = std::getenv("RTM_EL3_YCHUNK");
+  const int wfix = ws ? std::min(std::max(std::atoi(ws), 0), EX) : 0, yfix = ys ? std::atoi(ys) : 0;
+  const int res = el3_resident();
+  long long best = -1;
+  const int nbz0 = (a.nz + EZ - 1) / EZ;
+  for (int nbz = nbz0; nbz < nbz0 + 3 && nbz <= a.nz; ++nbz) {
+    const int tz = (a.nz + nbz - 1) / nbz;
+    int tx = std::min(wfix > 0 ? wfix : EX, std::min(ENT / tz, EHN / 10 - tz));
+    const int nbx = (a.nx + tx - 1) / tx;
+    if (wfix <= 0) tx = (a.nx + nbx - 1) / nbx;
+    for (int chunks = 1; chunks <= a.ny; ++chunks) {
+      const int ych = yfix > 0 ? std::min(yfix, a.ny) : (a.ny + chunks - 1) / chunks;
+      const long long blocks = 2LL * nbz * nbx * ((a.ny + ych - 1) / ych);
+      const long long cost = (blocks + res - 1) / res * (ych + EPRIME);
+      if (best < 0 || cost < best) {
+        best = cost;
+        a.tz = tz; a.tx = tx; a.nbz = (a.nz + tz - 1) / tz; a.nbx = nbx; a.ych = ych;
+      }
+      if (yfix > 0) break;
+    }
   }
-  // at least 256 workgroups, 10 to 40 planes per chunk (a chunk primes its
-  // queue with 10 planes; 40 measured best on 200^3 and 400^3, 6% and 3%
-  // faster than 20)
-  const int chunks = std::max(1, (256 + tiles - 1) / tiles);
-  return std::min(ny, std::min(40, std::max(10, (ny + chunks - 1) / chunks)));
+  a.nblk = a.nbz * a.nbx * ((a.ny + a.ych - 1) / a.ych);
 }
 
 struct El3Timing {
@@ -297,12 +444,7 @@ static int el3_steps(int ny, int nz, int nx, float* in[9], float* in1[9], float*
   a.sx = nz + 10;
   a.sy = (nz + 10) * (nx + 10);
   for (int k = 0; k < 6; ++k) a.m[k] = m[k];
-  const int ew = default_el3_width();
-  a.nbz = (nz + EZ - 1) / EZ;
-  a.nbx = (nx + ew - 1) / ew;
-  a.ych = default_el3_ychunk(ny, a.nbz * a.nbx);
-  const int nyc = (ny + a.ych - 1) / a.ych;
-  a.nblk = a.nbz * a.nbx * nyc;
+  el3_partition(a);
   a.xcd = default_xcd();
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
@@ -318,12 +460,7 @@ static int el3_steps(int ny, int nz, int nx, float* in[9], float* in1[9], float*
       a.in1[f] = in1[f];
       a.out[f] = out[f];
     }
-    if (ew == 16)
-      hipLaunchKernelGGL(k_el3_adj<16>, dim3(a.nblk), dim3(EZ * 16), 0, st, a);
-    else if (ew == 4)
-      hipLaunchKernelGGL(k_el3_adj<4>, dim3(a.nblk), dim3(EZ * 4), 0, st, a);
-    else
-      hipLaunchKernelGGL(k_el3_adj<8>, dim3(a.nblk), dim3(EZ * 8), 0, st, a);
+    hipLaunchKernelGGL(k_el3_adj, dim3(2 * a.nblk), dim3(ENT), 0, st, a);
     HIPCHK(hipGetLastError());
     if (s < nsteps - 1) {
       for (int f = 0; f < 9; ++f) {

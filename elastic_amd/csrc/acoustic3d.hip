@@ -17,6 +17,7 @@
 #include "../../include/acoustic3d.h"
 #include "common.hpp"
 #include "engine2d.hpp"
+#include "hostcopy.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -504,7 +505,7 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
   HIPCHK(hipStreamCreateWithFlags(&a->st, hipStreamNonBlocking));
   for (auto& e : a->ev) HIPCHK(hipEventCreate(&e));
   STCHK(a->c.alloc(a->n * 4, "velocity term"));
-  HIPCHK(hipMemcpy(a->c.p, c, a->n * 4, hipMemcpyHostToDevice));
+  STCHK(copy_to_device(a->c.p, c, a->n * 4));
   STCHK(a->k.alloc((size_t)(g.n1 + g.n2 + g.n3) * 4, "sponge"));
   std::vector<float> k1 = taper(g.n1, g.abc), k2 = taper(g.n2, g.abc), k3 = taper(g.n3, g.abc);
   HIPCHK(hipMemcpy(a->k.p, k1.data(), g.n1 * 4, hipMemcpyHostToDevice));
@@ -531,7 +532,7 @@ RTM_EXPORT int ac3d_model_data(ac3d* a, const float* c_true) {
   HIPCHK(hipEventRecord(a->ev[0], a->st));
   if (c_true) {
     STCHK(a->c_alt.alloc(a->n * 4, "true model"));
-    HIPCHK(hipMemcpy(a->c_alt.p, c_true, a->n * 4, hipMemcpyHostToDevice));
+    STCHK(copy_to_device(a->c_alt.p, c_true, a->n * 4));
     if (!a->rec_tmp.p) STCHK(a->rec_tmp.alloc((size_t)a->cfg.nt * a->plane * 4, "receiver scratch"));
     STCHK(ac3_source_pass(a, a->c_alt.as<float>(), 1, 0, 0));
     STCHK(ac3_source_pass(a, a->c.as<float>(), 1, 1, 0));
@@ -595,22 +596,19 @@ RTM_EXPORT int ac3d_migrate(ac3d* a) {
 
 RTM_EXPORT int ac3d_set_data(ac3d* a, const float* rec) {
   if (!a || !rec) { set_error("null argument"); return E_ARG; }
-  HIPCHK(hipMemcpy(a->rec.p, rec, (size_t)a->cfg.nt * a->plane * 4, hipMemcpyHostToDevice));
-  return OK;
+  return copy_to_device(a->rec.p, rec, (size_t)a->cfg.nt * a->plane * 4);
 }
 
 RTM_EXPORT int ac3d_get_data(ac3d* a, float* rec) {
   if (!a || !rec) { set_error("null argument"); return E_ARG; }
   HIPCHK(hipStreamSynchronize(a->st));
-  HIPCHK(hipMemcpy(rec, a->rec.p, (size_t)a->cfg.nt * a->plane * 4, hipMemcpyDeviceToHost));
-  return OK;
+  return copy_to_host(rec, a->rec.p, (size_t)a->cfg.nt * a->plane * 4);
 }
 
 RTM_EXPORT int ac3d_get_image(ac3d* a, float* img) {
   if (!a || !img) { set_error("null argument"); return E_ARG; }
   HIPCHK(hipStreamSynchronize(a->st));
-  HIPCHK(hipMemcpy(img, a->img.p, a->n * 4, hipMemcpyDeviceToHost));
-  return OK;
+  return copy_to_host(img, a->img.p, a->n * 4);
 }
 
 RTM_EXPORT int ac3d_get_snapshot_scales(ac3d* a, float* out, int n) {

@@ -10,6 +10,7 @@
 // here run at HBM rates, so they only have to be launched over enough
 // workgroups; the scratch is allocated per call (under 50 us for 32 MiB).
 #include "layout.hpp"
+#include "hostcopy.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -129,6 +130,17 @@ bool host_nonfinite(const float* p, size_t n) {
   return false;
 }
 
+// Copy from the scratch to a caller's array behind the stream's kernels; a large
+// one from several threads.
+int to_host(void* dst, const void* src, size_t n, hipStream_t st) {
+  if (n < kLargeToHost) {
+    HIPCHK(hipMemcpyAsync(dst, src, n, hipMemcpyDeviceToHost, st));
+    return OK;
+  }
+  HIPCHK(hipStreamSynchronize(st));
+  return copy_to_host(dst, src, n);
+}
+
 int transpose(const float* src, float* dst, int rows, int cols, long long src_ld, long long dst_ld, int nb,
               long long src_bs, long long dst_bs, int* flag, hipStream_t st) {
   // grid.y counts blocks of rows: 65535 of them hold 4.19 million levels or traces
@@ -201,7 +213,7 @@ int fetch_fields(float* dst, int nf, int nz, int nx, int ldz, const float* src, 
     hipLaunchKernelGGL(k_unpad, dim3(blocks_of(all), nf), dim3(256), 0, st, src, s.data(), nz, ldz, (long long)all,
                        (long long)fs, (long long)all, flag);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dst, s.data(), nf * all * sizeof(float), hipMemcpyDeviceToHost, st));
+    STCHK(to_host(dst, s.data(), nf * all * sizeof(float), st));
   } else {
     const int most = (int)std::min<size_t>(s.bytes / col, nx);
     for (int f = 0; f < nf; ++f)
@@ -211,7 +223,7 @@ int fetch_fields(float* dst, int nf, int nz, int nx, int ldz, const float* src, 
         hipLaunchKernelGGL(k_unpad, dim3(blocks_of(n), 1), dim3(256), 0, st, src + f * fs + (size_t)ldz * ix, s.data(),
                            nz, ldz, n, 0LL, 0LL, flag);
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(dst + f * all + (size_t)nz * ix, s.data(), nc * col, hipMemcpyDeviceToHost, st));
+        STCHK(to_host(dst + f * all + (size_t)nz * ix, s.data(), nc * col, st));
       }
   }
   STCHK(read_flag(s, nonfinite, st));
@@ -271,14 +283,14 @@ int fetch_records(float* dst, int nc, int nt, int nrx, const float* src, bool* n
   int* flag = nonfinite ? s.flag : nullptr;
   if (tr * nrx * nc <= s.bytes) {
     STCHK(transpose(src, s.data(), nt, nrx, nrx, nt, nc, comp, comp, flag, st));
-    HIPCHK(hipMemcpyAsync(dst, s.data(), nc * comp * sizeof(float), hipMemcpyDeviceToHost, st));
+    STCHK(to_host(dst, s.data(), nc * comp * sizeof(float), st));
   } else {
     const int most = (int)std::min<size_t>(s.bytes / tr, nrx);
     for (int f = 0; f < nc; ++f)
       for (int ix = 0; ix < nrx; ix += most) {
         const int n = std::min(most, nrx - ix);
         STCHK(transpose(src + f * comp + ix, s.data(), nt, n, nrx, nt, 1, 0, 0, flag, st));
-        HIPCHK(hipMemcpyAsync(dst + f * comp + (size_t)nt * ix, s.data(), n * tr, hipMemcpyDeviceToHost, st));
+        STCHK(to_host(dst + f * comp + (size_t)nt * ix, s.data(), n * tr, st));
       }
   }
   STCHK(read_flag(s, nonfinite, st));
@@ -301,7 +313,7 @@ int fetch_rounded(float* dst, const double* src, size_t n, hipStream_t st) {
     const size_t m = std::min(most, n - i);
     hipLaunchKernelGGL(k_round, dim3(blocks_of(m)), dim3(256), 0, st, src + i, s.data(), m);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(dst + i, s.data(), m * sizeof(float), hipMemcpyDeviceToHost, st));
+    STCHK(to_host(dst + i, s.data(), m * sizeof(float), st));
   }
   HIPCHK(hipStreamSynchronize(st));
   return OK;

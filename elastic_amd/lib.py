@@ -98,10 +98,17 @@ def rtm_op3(hist, coefs, zrec=0, inplace=False):
                 raise ValueError("in-place histories must be Fortran-contiguous float32")
         h = list(hist)
     else:
-        h = [_f32F(a).copy(order="F") for a in hist]
+        src = [_f32F(a) for a in hist]
+        h = [np.empty(src[0].shape, np.float32, order="F") for _ in src]
     c = [_f32F(a) for a in coefs]
     nz, nx, nt = h[0].shape
-    _chk(lib.rtm_op3_hip(C.c_int(nt), C.c_int(nz), C.c_int(nx), C.c_int(zrec), *[_p(a) for a in h], *[_p(a) for a in c]))
+    if inplace:
+        _chk(lib.rtm_op3_hip(C.c_int(nt), C.c_int(nz), C.c_int(nx), C.c_int(zrec), *[_p(a) for a in h],
+                             *[_p(a) for a in c]))
+    else:
+        P5 = C.c_void_p * 5
+        _chk(lib.rtm_op3_hip_to(C.c_int(nt), C.c_int(nz), C.c_int(nx), P5(*[a.ctypes.data for a in src]),
+                                P5(*[a.ctypes.data for a in h]), P5(*[a.ctypes.data for a in c])))
     return h
 
 

@@ -55,6 +55,13 @@ int rtm_op3_hip(int nt, int nz, int nx, int zrec, float *Vx0, float *Vz0, float 
                 float *sigmazz0, float *sigmaxz0, const float *m1_x, const float *m1_z,
                 const float *aux_m2_c, const float *aux_m3_c, const float *aux_m2m3_c);
 
+/* rtm_op3_hip from five histories (Vx, Vz, sxx, szz, sxz) into five others,
+ * for callers that keep their input: the result is written once instead of the
+ * input being copied first. hist and out must not overlap, except that all of
+ * out may be hist (in place). coefs: m1_x, m1_z, aux_m2, aux_m3, aux_m2m3. */
+int rtm_op3_hip_to(int nt, int nz, int nx, const float *const *hist, float *const *out,
+                   const float *const *coefs);
+
 /* Allocation-free form of rtm_op3_hip: same arguments, semantics and status
  * codes, bit-for-bit the same results. No counterpart in the reference; it
  * is for callers that cannot allocate device memory (serving loops,

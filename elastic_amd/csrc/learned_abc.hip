@@ -27,7 +27,6 @@ constexpr int OW1 = 0, OB1 = NF * H, OW2 = OB1 + H, OB2 = OW2 + H * H, OW3 = OB2
               OB3 = OW3 + H * NO, NP = OB3 + NO;
 static_assert(NP == LABC_NPARAM, "parameter count");
 constexpr float Z0 = LABC_Z0;
-constexpr int NRAW = 230;  // wavefield features (scaled by the cell's max-abs)
 
 struct Band {
   int nz, nx, nT, nL, total;
@@ -368,13 +367,22 @@ __global__ void k_sample(int* idx, int batch, int n, unsigned seed) {
 // matrix products with FP32 accumulation (the features and weights are
 // BF16-rounded already, so the products are exact and only the summation
 // order differs from a scalar loop), layer 2 on FP32 matrix cores and
-// layer 3 in FP32 from LDS. A workgroup of 12 waves (the weights copied to
-// LDS once, 148 KB of LDS: one workgroup per CU, 3 waves per SIMD) loops
-// over batches of 192 cells.
+// layer 3 in FP32 from LDS. A workgroup of 16 waves (the weights copied to LDS
+// once, the hidden layers in the place of the features: 157 KB, one workgroup
+// per CU, 4 waves per SIMD) loops over batches of 256 cells.
+// What bounds it is the chain of a batch (cell entry, descriptor, patch,
+// products, GELUs), so waves in flight count: 6 grids of 426 x 826 (7296
+// batches of a wave) took 33 us in three rounds of 12 waves a CU, 25.7 in two
+// of 16. 16 fit since the patch loads take ten byte offsets a lane for the five
+// fields' scalar bases instead of an address each: 121 registers for 168, 300
+// VALU instructions a batch for 540. The features, their order and the GELUs
+// stay as they are to the bit: a rounding that differs anywhere flips BF16
+// features, and the flips feed back through the wavefield (2e-5 of the images
+// after 400 levels).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int MC = 16;        // cells per wave (rows of the matrix product)
-constexpr int IW = 12;        // waves per inference workgroup (one per CU: 3 per SIMD)
+constexpr int IW = 16;        // waves per inference workgroup (one per CU: 4 per SIMD)
 constexpr int IT = 64 * IW;   // its threads
 constexpr int KX = 256;       // features padded to 8 K-steps of 32
 constexpr int KXP = KX + 8;   // LDS row pitch (bf16): rows 16 B apart in the banks
@@ -387,21 +395,13 @@ __device__ __forceinline__ __bf16 to_bf16(float x) {  // x already bf16-represen
 __device__ __forceinline__ float gldv(const float* p, int i) {
   return ((const __attribute__((address_space(1))) float*)p)[i];
 }
+// Load at a byte offset from a base that is the same in every lane.
+__device__ __forceinline__ float gldb(const float* base, unsigned o) {
+  return *(const __attribute__((address_space(1))) float*)((const __attribute__((address_space(1))) char*)base + o);
+}
 __device__ __forceinline__ void gstv(float* p, int i, float v) {
   ((__attribute__((address_space(1))) float*)p)[i] = v;
 }
-
-struct GridView {
-  const float* l1;  // level L-1, field f at + f*fs
-  const float* l2;  // level L-2
-  long long fs;
-  int ldz, nz, nx;
-  __device__ __forceinline__ float get(const float* p, int f, int iz, int ix) const {
-    if (iz < 0 || iz >= nz || ix < 0 || ix >= nx) return 0.f;
-    const float v = p[f * fs + iz + ldz * ix];
-    return f >= 2 ? v * (1.f / Z0) : v;
-  }
-};
 
 // Inference weights as the kernel keeps them in LDS, packed once per weight
 // update: W1 transposed to [hidden][feature] in BF16 (rows KXP long), then
@@ -461,8 +461,7 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
   // features and hidden layers: each wave uses only its own [wv] rows, so
   // after the weights are in place the waves of a workgroup run their
   // batches without workgroup barriers
-  __shared__ __bf16 sX[IW][MC][KXP];
-  __shared__ float sH[IW][MC][H];
+  __shared__ __align__(16) __bf16 sX[IW][MC][KXP];
   const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
   for (int i = t; i < PBYTES / 16; i += IT)
     reinterpret_cast<uint4*>(sWp)[i] = reinterpret_cast<const uint4*>(packed)[i];
@@ -499,56 +498,106 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
   const int dz = edge == 0 ? 1 : edge == 1 ? -1 : 0, dx = edge == 2 ? 1 : edge == 3 ? -1 : 0;
   const int nstep = dz + ldz * dx, tstep = edge >= 2 ? 1 : ldz;
   const int base = live ? cc.iz + ldz * cc.ix : 2 * tstep;  // dead lanes read near element 0
-  // the cell's coefficients and its outputs (level L, the Vx, Vz history),
-  // loaded with the features
-  float cp = 0.f, cs = 0.f, zp = 0.f;
-  Mat{S.coef, (int)S.n2, S.ldz}.at(cc.iz, cc.ix, cp, cs, zp);
+  // the cell's outputs (level L, the Vx, Vz history) and its coefficients (one
+  // material value per lane), loaded with the features
   float* const out = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L);
   float* const hh = !ADJ && hist ? static_cast<float*>(S.snap) + (long long)(L - 1) * 2 * S.n2 : nullptr;
   const int gi0 = cc.iz + ldz * cc.ix;
+  const int cn2 = (int)S.n2;
+  const float cm1 = gldv(S.coef, gi0), cmx = gldv(S.coef, (part == 1 ? 3 : 4) * cn2 + gi0);
   float ov[2], hv[2];
 #pragma unroll
   for (int q = 0; q < 2; ++q) {
     const int o = part + 4 * q;
     ov[q] = o < NO ? gldv(out, o * fs + gi0) : 0.f;
-    hv[q] = (hh && o < 2) ? gldv(hh, (int)S.n2 * o + gi0) : 0.f;
+    hv[q] = (hh && o < 2) ? gldv(hh, cn2 * o + gi0) : 0.f;
   }
-  constexpr int NV = (NRAW + 3) / 4;  // values per lane
-  float rv[NV];
-  float m = 0.f;
+  // Patch values: lane part takes inward steps 2 part and 2 part + 1 of every
+  // field and offset (ten byte offsets serve the five fields, whose bases are
+  // scalar), the ninth step of offset part, and for the last offset and level
+  // L-2 field part; field 4 of those two comes in all four lanes. Dead lanes
+  // read valid cells too; their rows are not used.
+  float rp[5][5][2], r8[5], rt[2], ro[2];
+  unsigned po[5][2];
 #pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int k = part + 4 * u;
-    float v = 0.f;
-    if (k < 225) {  // field f of level L-1 (L+1) at (kn inward, mm - 2 along the edge)
-      const int fm = k / 9, kn = k - 9 * fm, f = fm / 5, mi = fm - 5 * f;
-      v = gldv(l1, f * fs + base + kn * nstep + (mi - 2) * tstep);
-      if (z_scaled(f, ADJ)) v = v * (1.f / Z0);
-    } else if (k < NRAW) {  // the cell's own fields of level L-2 (L+2)
-      const int f = k - 225;
-      v = gldv(l2, f * fs + base);
-      if (z_scaled(f, ADJ)) v = v * (1.f / Z0);
+  for (int m = 0; m < 5; ++m) {
+    po[m][0] = 4u * (unsigned)(base + (m - 2) * tstep + 2 * part * nstep);
+    po[m][1] = po[m][0] + 4u * (unsigned)nstep;
+  }
+  const unsigned o8 = 4u * (unsigned)(base + (part - 2) * tstep + 8 * nstep);
+  const int i84 = base + 2 * tstep + 8 * nstep;
+#pragma unroll
+  for (int f = 0; f < 5; ++f) {
+    const float* const lf = l1 + (long long)f * fs;
+#pragma unroll
+    for (int mi = 0; mi < 5; ++mi) {
+      rp[f][mi][0] = gldb(lf, po[mi][0]);
+      rp[f][mi][1] = gldb(lf, po[mi][1]);
     }
-    v = live ? v : 0.f;
-    rv[u] = v;
-    m = fmaxf(m, fabsf(v));
+    r8[f] = gldb(lf, o8);
+  }
+  rt[0] = gldv(l1, part * fs + i84);
+  rt[1] = gldv(l1, 4 * fs + i84);
+  ro[0] = gldv(l2, part * fs + base);
+  ro[1] = gldv(l2, 4 * fs + base);
+  float m = 0.f;
+  auto scaled = [&](int f, float v) { return z_scaled(f, ADJ) ? v * (1.f / Z0) : v; };
+#pragma unroll
+  for (int f = 0; f < 5; ++f) {
+#pragma unroll
+    for (int mi = 0; mi < 5; ++mi)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        rp[f][mi][i] = scaled(f, rp[f][mi][i]);
+        m = fmaxf(m, fabsf(rp[f][mi][i]));
+      }
+    r8[f] = scaled(f, r8[f]);
+    m = fmaxf(m, fabsf(r8[f]));
+  }
+  const bool zpart = z_scaled(part, ADJ);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float(&v)[2] = i == 0 ? rt : ro;
+    v[0] = zpart ? v[0] * (1.f / Z0) : v[0];
+    v[1] = scaled(4, v[1]);
+    m = fmaxf(m, fmaxf(fabsf(v[0]), fabsf(v[1])));
   }
   m = fmaxf(m, __shfl_xor(m, 1, 64));
   m = fmaxf(m, __shfl_xor(m, 2, 64));
   const float inv = m > 1e-30f ? 1.f / m : 0.f;
+  // the hardware conversion (round to nearest even, as bf16r)
+  __bf16* const xr = sX[wv][cl];
 #pragma unroll
-  for (int u = 0; u < NV; ++u) {
-    const int k = part + 4 * u;
-    // the hardware conversion (round to nearest even, as bf16r) in one
-    // instruction
-    if (k < NRAW) sX[wv][cl][k] = (__bf16)(rv[u] * inv);
+  for (int f = 0; f < 5; ++f) {
+#pragma unroll
+    for (int mi = 0; mi < 5; ++mi) {
+      xr[(f * 5 + mi) * 9 + 2 * part] = (__bf16)(rp[f][mi][0] * inv);
+      xr[(f * 5 + mi) * 9 + 2 * part + 1] = (__bf16)(rp[f][mi][1] * inv);
+    }
+    xr[(f * 5 + part) * 9 + 8] = (__bf16)(r8[f] * inv);
   }
-  for (int k = NRAW + part; k < KX; k += 4)
-    sX[wv][cl][k] = (__bf16)(live ? static_feature(edge, depth, cp, cs, zp, k) : 0.f);
+  xr[(part * 5 + 4) * 9 + 8] = (__bf16)(rt[0] * inv);
+  xr[224] = (__bf16)(rt[1] * inv);
+  xr[225 + part] = (__bf16)(ro[0] * inv);
+  xr[229] = (__bf16)(ro[1] * inv);
+  // one-hot edge and depth, then P and S Courant numbers and P impedance
+  const float one = 1.f, zero = 0.f;
+  xr[230 + part] = (__bf16)(part == edge ? one : zero);
+  xr[234 + part] = (__bf16)(part == depth ? one : zero);
+  xr[238 + part] = (__bf16)(part + 4 == depth ? one : zero);
+  {
+    const float q = part < 2 ? cm1 * cmx : cm1 > 0.f ? cmx / cm1 : 0.f;
+    const float v = sqrtf(q);
+    xr[242 + part] = (__bf16)(part == 3 ? zero : part == 2 ? v * (1.f / Z0) : v);
+  }
+#pragma unroll
+  for (int k = 246; k < KX; k += 4)
+    if (k + part < KX) xr[k + part] = (__bf16)zero;
   wave_sync();
 
   // layer 1 on MFMA: Z1[16 x 32] = X[16 x 256] W1[256 x 32], two 16-column tiles
   const int r16 = lane & 15, kq = (lane >> 4) * 8;
+  f32x4 z1[2];
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -558,10 +607,17 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
       const bf16x8 b = *reinterpret_cast<const bf16x8*>(&sW1[nt * 16 + r16][kk * 32 + kq]);
       acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
     }
-    // this lane holds rows (lane / 16) * 4 + i of column nt * 16 + r16
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sH[wv][(lane >> 4) * 4 + i][nt * 16 + r16] = gelu(acc[i] + sB[nt * 16 + r16]);
+    z1[nt] = acc;
   }
+  // the hidden layers take the place of the wave's features, which every lane
+  // has read by then (a wave's LDS operations run in program order)
+  float(*const sH)[H] = reinterpret_cast<float(*)[H]>(&sX[wv][0][0]);
+  wave_sync();
+  // this lane holds rows (lane / 16) * 4 + i of column nt * 16 + r16
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sH[(lane >> 4) * 4 + i][nt * 16 + r16] = gelu(z1[nt][i] + sB[nt * 16 + r16]);
   wave_sync();
   // layer 2 on FP32 MFMA: Z2[16 x 32] = H1[16 x 32] W2[32 x 32] in 8 steps
   // of 4 (lane: A row r16, B column r16, k = lane / 16); the wave's own
@@ -575,14 +631,14 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kk = 0; kk < H / 4; ++kk)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sH[wv][r16][kk * 4 + kr], sW2[(kk * 4 + kr) * H + nt * 16 + r16],
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(sH[r16][kk * 4 + kr], sW2[(kk * 4 + kr) * H + nt * 16 + r16],
                                                    acc, 0, 0, 0);
       z[nt] = acc;
     }
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sH[wv][kr * 4 + i][nt * 16 + r16] = gelu(z[nt][i] + sB[H + nt * 16 + r16]);
+      for (int i = 0; i < 4; ++i) sH[kr * 4 + i][nt * 16 + r16] = gelu(z[nt][i] + sB[H + nt * 16 + r16]);
   }
   // layer 3: partial sums over hidden units part*8 .. part*8+7 of cell cl,
   // reduced over the cell's 4 lanes
@@ -590,7 +646,7 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
 #pragma unroll
   for (int u = 0; u < 8; ++u) {
     const int j = part * 8 + u;
-    const float h2 = sH[wv][cl][j];
+    const float h2 = sH[cl][j];
 #pragma unroll
     for (int o = 0; o < NO; ++o) y[o] = fmaf(h2, sW3[j * NO + o], y[o]);
   }
@@ -610,7 +666,7 @@ __global__ __launch_bounds__(IT) void k_infer_mfma(const unsigned char* __restri
       }
     }
   }
-  wave_sync();  // sX and sH are rewritten by the next batch
+  wave_sync();  // sX is rewritten by the next batch
   }
 }
 

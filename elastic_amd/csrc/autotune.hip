@@ -13,7 +13,8 @@
 // HBM traffic of the fields but recompute a radius-5 ring of the first level
 // and run at lower occupancy; so are the marching forms (workgroups per
 // strip walking along x, halo columns read once per strip) at strip widths
-// 16, 24, 28 and 32. Which form wins is measured, not assumed.
+// 16, 24, 28 and 32. Which form wins is measured, not assumed. With 16-bit
+// snapshots the candidates are those of width 2.
 #include "engine2d.hpp"
 
 #include <algorithm>
@@ -153,12 +154,16 @@ int autotune_txr(const EngineCfg& cfg, const std::vector<ShotSpec>& shots, const
     return OK;
   };
   for (int i = 0; i < 8; ++i) {
+    t[i] = -1;
+    // 16-bit snapshots are scaled per strip of the tile's width, so the images
+    // go by it (by about 1e-3): timings must not choose it, and only width 2
+    // (which the marching forms share) is a candidate
+    if (c.snap_fmt > SNAP_F32 && cand[i][0] != 2) continue;
     if (i < 7) {
       STCHK(time_form(cand[i][0], cand[i][1], &t[i]));
     } else {
       // marching: forms 2 and 3 at each strip width; the fastest stands for
       // the slot.
-      t[7] = -1;
       double tw[kMW] = {-1, -1, -1, -1};
       int fw[kMW] = {2, 2, 2, 2};
       for (int m = 0; m < nmw; ++m) {

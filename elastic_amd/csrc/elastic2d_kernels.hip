@@ -2280,6 +2280,12 @@ int launch_fwd(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, in
     HIPCHK(hipGetLastError());
     return OK;
   }
+  // a level of width 2's tiles without a snapshot runs on the eight-wave tile,
+  // which has the same cells, whatever the format
+  if (txr == 2 && !(flags & F_SNAP)) {
+    txr = kSmallTile;
+    snap = SNAP_HIST;
+  }
   if (txr == kSmallTile) {  // fp32 formats only
     const dim3 b(TILE_Z, SMALL_WY);
     if (snap == SNAP_HIST)
@@ -2323,6 +2329,12 @@ int launch_adj(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, in
                int snap, int xcd, hipStream_t st, int nbz) {
   if (ntiles <= 0) return OK;
   const dim3 g(ntiles);
+  // a level of width 2's tiles without a snapshot runs on the eight-wave tile,
+  // which has the same cells, whatever the format
+  if (txr == 2 && !(flags & A_IMG)) {
+    txr = kSmallTile;
+    snap = SNAP_HIST;
+  }
   if (txr == kSmallTile) {  // fp32 formats only
     const dim3 b(TILE_Z, SMALL_WY);
     if (snap == SNAP_HIST)

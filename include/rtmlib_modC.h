@@ -245,7 +245,8 @@ int rtm_batch_march_w(rtm_batch *b);
  * levels; same options) with tile widths 1, 2, 4, 8 at one level per
  * launch, 1, 2, 4 at two levels per launch (temporal blocking) and the
  * marching forms (strips of 16, 24, 28 and 32 columns), and returns the fastest in
- * *txr, *tblock;
+ * *txr, *tblock. With 16-bit snapshots, whose scales and so images go by the
+ * width, only width 2 and the marching forms (which share its scales) run;
  * ms8[tblock*4 + log2(txr)] receives the times of the first seven and ms8[7]
  * that of the faster marching form, 2 or 3 (ms, -1 for candidates not run).
  * The result

@@ -88,3 +88,24 @@ def test_uneven_batch(hip):
         imgs.append([a for i in range(3) for a in b.image(i)])
         b.close()
     _same(imgs)
+
+
+@pytest.mark.parametrize("prec", ["bf16", "fp16"])
+def test_tuner_keeps_the_scales_of_width_2(hip, prec):
+    """16-bit snapshots are scaled per strip of the tile width: a tuned batch
+    gives the images of width 2 bit for bit."""
+    nz, nx, nt = 70, 90, 24
+    c, rng = _model(nz, nx, 3)
+    spec = dict(nz=nz, nx=nx, xs=45, zs=30, zr=20, rx0=1, nrx=nx - 2)
+    rec = rng.standard_normal((5, nx - 2, nt)).astype(np.float32)
+    wav = rng.standard_normal(nt).astype(np.float32)
+    imgs = []
+    for txr in (0, 2):
+        b = hip.Batch(nt, 10.0, 1e-3, [spec], [c], wav, abc=5, adj_abc=1, snap_every=3, snap_prec=prec, comp_image=1,
+                      txr=txr)
+        assert b.txr == 2
+        b.set_data(0, rec)
+        b.migrate()
+        imgs.append(list(b.image(0)))
+        b.close()
+    _same(imgs)

@@ -131,6 +131,19 @@ int launch_fwd2(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, i
 // the drop-in history form).
 int launch_adj2(const ShotDev* shots, const TileRef* tiles, int ntiles, int L, int flags,
                 int txr, int snap_fmt, int xcd, hipStream_t st);
+// Levels L and L+1 of the forward (Born propagation too), or L and L-1 of the
+// adjoint (without the R/Src sponge), of one shot in one launch, for grids too
+// small to fill the GPU (elastic2d_pair.hip); fp32 snapshots, four-level ring, s
+// the host's copy of the descriptor, amp0 / amp1 the source terms of the two
+// levels, tile that of pair_tile(), which is PAIR_ONE where launch_fwd /
+// launch_adj are faster. Bitwise the same results as those.
+enum : int { PAIR_ONE = 0, PAIR_S, PAIR_M, PAIR_L, PAIR_X };
+constexpr long long kPairCells = 1 << 24;  // cells of a field (ring offsets are 32-bit there)
+int pair_tile(int nz, int nx, bool forward, bool born);
+int launch_fwd_pair(const ShotDev& s, int tile, int L, int flags, float amp0, float amp1, int xcd, hipStream_t st);
+int launch_adj_pair(const ShotDev& s, int tile, int L, int flags, int xcd, hipStream_t st);
+// Compute units of the current device (0 if unknown).
+int device_cus();
 // Marching forms: one workgroup of nw waves (nw in {1, 2, 4}) per strip of
 // 64*nw rows x xw columns (xw even; strip tables start strips on even
 // columns and rows on multiples of 64*nw). Bitwise the same results as

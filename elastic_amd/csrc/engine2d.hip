@@ -210,10 +210,10 @@ int Engine::setup(const EngineCfg& cfg, const std::vector<ShotSpec>& shots,
     r.nstrip = nstrips(p.nz, p.nx, cfg_.txr);
   }
   // dt*source(L-1) for level L (explosive_source, W/source-mod.f90:47-53)
-  std::vector<float> amp(cfg_.nt, 0.f);
-  for (int L = 2; L <= cfg_.nt; ++L) amp[L - 1] = cfg_.dt * wavelet[L - 2];
+  amp_.assign(cfg_.nt, 0.f);
+  for (int L = 2; L <= cfg_.nt; ++L) amp_[L - 1] = cfg_.dt * wavelet[L - 2];
   STCHK(src_amp_.alloc(cfg_.nt * sizeof(float), "source amplitudes"));
-  HIPCHK(hipMemcpy(src_amp_.p, amp.data(), cfg_.nt * sizeof(float), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(src_amp_.p, amp_.data(), cfg_.nt * sizeof(float), hipMemcpyHostToDevice));
   if (cfg_.stack_nz > 0 && cfg_.stack_nx > 0) {
     STCHK(stack_.alloc((size_t)3 * cfg_.stack_nz * cfg_.stack_nx * sizeof(double), "stacked image"));
     HIPCHK(hipMemsetAsync(stack_.p, 0, stack_.bytes, st_));
@@ -495,6 +495,28 @@ int Engine::single_nbz(const Group& gr) const {
   return gr.shots.size() == 1 ? (specs_[gr.shots[0]].nz + TILE_Z - 1) / TILE_Z : 0;
 }
 
+// How many levels one launch of a group's forward run takes (mode as below):
+// PAIR_TILES two on tiles (kernel form 1: levels L >= 3 at the widths the
+// kernel has; Born scattering sources and the learned layer are per level),
+// PAIR_SMALL two on the tiles of elastic2d_pair.hip (one shot on a small grid).
+Engine::Pairs Engine::fwd_pairs(const Group& gr, int mode) const {
+  if (cfg_.labc_w && mode <= 3) return PAIR_NONE;
+  if (cfg_.tblock == 1) return mode != 5 && cfg_.txr <= 4 ? PAIR_TILES : PAIR_NONE;
+  return small_tile(gr, true, mode == 5) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
+}
+// The same of its adjoint run (no two-level form with the R/Src sponge; the
+// learned layer corrects every level).
+Engine::Pairs Engine::adj_pairs(const Group& gr) const {
+  if (cfg_.adj_abc == 2 || cfg_.labc_wa) return PAIR_NONE;
+  if (cfg_.tblock == 1) return cfg_.txr <= 4 ? PAIR_TILES : PAIR_NONE;
+  return small_tile(gr, false, false) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
+}
+// The tile of those launches, PAIR_ONE where one level a launch is faster.
+int Engine::small_tile(const Group& gr, bool forward, bool born) const {
+  if (cfg_.tblock != 0 || tile_code() != kSmallTile || gr.shots.size() != 1) return PAIR_ONE;
+  return pair_tile(specs_[gr.shots[0]].nz, specs_[gr.shots[0]].nx, forward, born);
+}
+
 // mode 0: imaging forward (migration model, snapshots); 1: record with the
 // true model (store); 2: record with the migration model (subtract);
 // 3: record with the migration model (store); 4: Born background (fp32
@@ -519,12 +541,11 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
   // source runs: imaging, data synthesis, modelling)
   const bool learn = cfg_.labc_w && mode <= 3;
   const LCell* lcells = learn ? d_lcells_.as<LCell>() + gr.lcell0 : nullptr;
-  // levels L >= 3 go two per launch (temporal blocking) where the kernel
-  // supports the tile width; Born scattering sources and the learned layer
-  // are per level
-  const bool pairs = cfg_.tblock == 1 && !born && !learn && cfg_.txr <= 4;
+  const Pairs pairs = fwd_pairs(gr, mode);
+  const int ptile = small_tile(gr, true, born);
+  const ShotDev& one = h_desc_[(size_t)variant * specs_.size() + gr.desc0];
   for (int L = first; L <= cfg_.nt;) {
-    const bool two = pairs && L >= 3 && L + 1 <= cfg_.nt;
+    const bool two = pairs != PAIR_NONE && (born || L >= 3) && L + 1 <= cfg_.nt;
     int fl = 0;
     if (cfg_.abc > 0 && (born || L >= 3)) fl |= F_K;  // level 2 of the source run is the bare injection
     if (!born) fl |= F_SRC;
@@ -544,7 +565,9 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
         if (two && L % cfg_.snap_every == 0) fl |= F_SNAP2;    // and of level L
       }
     }
-    if (two)
+    if (two && pairs == PAIR_SMALL)
+      STCHK(launch_fwd_pair(one, ptile, L, fl, amp_[L - 1], amp_[L], cfg_.xcd, st));
+    else if (two)
       STCHK(launch_fwd2(desc, tiles, gr.ntiles, L, fl, cfg_.txr, snap, cfg_.xcd, st));
     else if (march)
       STCHK(launch_fwdm(desc, strips, gr.fnstrips, L, fl, gr.fmarch_w, cfg_.march_nw, snap, cfg_.xcd, st));
@@ -587,12 +610,12 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
     STCHK(launch_fill(r.img.as<float>(), 3 * r.n2, 0.f, st));
     if (cfg_.comp) STCHK(launch_fill(r.imgc.as<float>(), 3 * r.n2, 0.f, st));
   }
-  // the two-level adjoint has no R/Src sponge form, and the learned layer
-  // corrects every level: one level per launch
-  const bool pairs = cfg_.tblock == 1 && cfg_.txr <= 4 && cfg_.adj_abc != 2 && !cfg_.labc_wa;
+  const Pairs pairs = adj_pairs(gr);
+  const int ptile = small_tile(gr, false, false);
+  const ShotDev& one = h_desc_[gr.desc0];
   const LCell* lcells = cfg_.labc_wa ? d_lcells_.as<LCell>() + gr.lcell0 : nullptr;
   for (int L = cfg_.nt; L >= 1;) {
-    const bool two = pairs && L - 1 >= 1;
+    const bool two = pairs != PAIR_NONE && L - 1 >= 1;
     int fl = A_INJ;
     if (cfg_.adj_abc && cfg_.abc > 0) fl |= A_K;
     if (cfg_.adj_abc == 2 && cfg_.abc > 0) fl |= A_KSRC;
@@ -601,7 +624,9 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
     if (L < cfg_.nt) fl |= A_NEXT;
     if (cfg_.comp) fl |= A_COMP;
     if (nt_stores()) fl |= A_NTS;
-    if (two)
+    if (two && pairs == PAIR_SMALL)
+      STCHK(launch_adj_pair(one, ptile, L, fl, cfg_.xcd, st));
+    else if (two)
       STCHK(launch_adj2(desc, tiles, gr.ntiles, L, fl, cfg_.txr, cfg_.snap_fmt, cfg_.xcd, st));
     else if (march)
       STCHK(launch_adjm(desc, strips, gr.nstrips, L, fl, gr.march_w, cfg_.march_nw, cfg_.snap_fmt, cfg_.xcd, st));
@@ -618,17 +643,16 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
   return OK;
 }
 
-// Step launches of one forward run of a mode / of one adjoint run (the
-// loops of enqueue_forward / enqueue_adjoint).
-long long Engine::fwd_launch_count(int mode) const {
-  const bool born = mode == 5;
-  const bool pairs = cfg_.tblock == 1 && !born && !(cfg_.labc_w && mode <= 3) && cfg_.txr <= 4;
+// Step launches of one forward run of a mode / of one adjoint run of a group
+// (the loops of enqueue_forward / enqueue_adjoint).
+long long Engine::fwd_launch_count(const Group& gr, int mode) const {
+  const bool born = mode == 5, pairs = fwd_pairs(gr, mode) != PAIR_NONE;
   long long n = 0;
-  for (int L = born ? 1 : 2; L <= cfg_.nt; ++n) L += (pairs && L >= 3 && L + 1 <= cfg_.nt) ? 2 : 1;
+  for (int L = born ? 1 : 2; L <= cfg_.nt; ++n) L += (pairs && (born || L >= 3) && L + 1 <= cfg_.nt) ? 2 : 1;
   return n;
 }
-long long Engine::adj_launch_count() const {
-  const bool pairs = cfg_.tblock == 1 && cfg_.txr <= 4 && cfg_.adj_abc != 2 && !cfg_.labc_wa;
+long long Engine::adj_launch_count(const Group& gr) const {
+  const bool pairs = adj_pairs(gr) != PAIR_NONE;
   long long n = 0;
   for (int L = cfg_.nt; L >= 1; ++n) L -= (pairs && L - 1 >= 1) ? 2 : 1;
   return n;
@@ -713,7 +737,7 @@ int Engine::model_data() {
       STCHK(launch_fill(res_[s].rec.as<float>(), (size_t)5 * cfg_.nt * std::max(specs_[s].nrx, 1), 0.f, st_));
     STCHK(enqueue_forward(g, 3, st_));
     for (int s : groups_[g].shots) tm_.fwd_cells += cells_of(specs_[s]) * (cfg_.nt - 1);
-    tm_.fwd_launches += fwd_launch_count(3);
+    tm_.fwd_launches += fwd_launch_count(groups_[g], 3);
     last_group_ = g;
   }
   HIPCHK(hipEventRecord(ev_[1], st_));
@@ -749,8 +773,8 @@ int Engine::migrate() {
     tm_.fwd_ms += a;
     tm_.adj_ms += b;
     tm_.total_ms += c;
-    tm_.fwd_launches += fwd_launch_count(0);
-    tm_.adj_launches += adj_launch_count();
+    tm_.fwd_launches += fwd_launch_count(groups_[g], 0);
+    tm_.adj_launches += adj_launch_count(groups_[g]);
     for (int s : groups_[g].shots) {
       tm_.fwd_cells += cells_of(specs_[s]) * (cfg_.nt - 1);
       tm_.adj_cells += cells_of(specs_[s]) * cfg_.nt;
@@ -787,7 +811,7 @@ int Engine::born(const std::vector<const float*>& dm) {
   float ms = 0;
   HIPCHK(hipEventElapsedTime(&ms, ev_[0], ev_[1]));
   tm_.fwd_ms = tm_.total_ms = ms;
-  tm_.fwd_launches = fwd_launch_count(5);
+  tm_.fwd_launches = fwd_launch_count(groups_[0], 5);
   last_group_ = 0;
   return OK;
 }

@@ -178,8 +178,12 @@ class Engine {
   int enqueue_forward(int g, int mode, hipStream_t st);
   int enqueue_adjoint(int g, hipStream_t st);
   int run_phase(int g, int which, hipStream_t st);
-  long long fwd_launch_count(int mode) const;
-  long long adj_launch_count() const;
+  enum Pairs { PAIR_NONE, PAIR_TILES, PAIR_SMALL };  // levels per step launch, see engine2d.hip
+  Pairs fwd_pairs(const Group& gr, int mode) const;
+  Pairs adj_pairs(const Group& gr) const;
+  int small_tile(const Group& gr, bool forward, bool born) const;
+  long long fwd_launch_count(const Group& gr, int mode) const;
+  long long adj_launch_count(const Group& gr) const;
   void destroy_graphs();
 
   EngineCfg cfg_;
@@ -194,6 +198,7 @@ class Engine {
   size_t arena_bytes_ = 0;
   DevBuf src_amp_, work_, d_desc_, d_tiles_, d_strips_, stack_, born_buf_, d_lcells_;
   std::vector<ShotDev> h_desc_;
+  std::vector<float> amp_;  // source terms by level, the host's copy of src_amp_
   hipStream_t st_ = nullptr;
   hipEvent_t ev_[4] = {};
   int last_group_ = -1;

@@ -8,13 +8,16 @@
 // for the interior (5 cells from every face), then the point source or the
 // receiver-plane injection, the receiver recording, the per-snapshot max-abs
 // of the source wavefield and, in the receiver pass, the image update.
-// Layout: (n1, n2, n3) = (z fastest, x, y slowest). A workgroup owns a 64 x 16
+// Layout: (n1, n2, n3) = (z fastest, x, y slowest); on the device each z-row is
+// padded so that the first interior cell, and with it every wave's row of 64,
+// starts on a cache line (see Layout). A workgroup owns a 64 x 16
 // tile of the (z, x) plane and marches along y over a chunk of planes; the
 // y-neighbours live in an 11-deep register queue, the (z, x) halo of the
 // current plane in LDS. Each step moves 16 algorithmic bytes per cell
 // (read p, p_prev, c; write p_next): HBM-bound.
 
 #include "../../include/acoustic3d.h"
+#include "buffer.hpp"
 #include "common.hpp"
 #include "engine2d.hpp"
 #include "hostcopy.hpp"
@@ -57,6 +60,8 @@ struct Ac3Args {
   const void* snap;          // source snapshot of this level (mode 1 image level)
   float snap_scale;
   int snap_bf16;
+  void* snap_out;            // snapshot of the current level p to write (mode 0)
+  const unsigned* snap_max;  // its max-abs (float bits)
   float* img;                // image (mode 1 image level)
   int ychunk;
 };
@@ -94,17 +99,48 @@ __device__ __forceinline__ T g1(const T* p, int i) {
 // operands) are issued before plane y is computed, so their latency hides
 // behind the arithmetic of the current plane. The plane tile is
 // double-buffered in LDS with one barrier per plane whose fences cover LDS
-// only, so those loads stay in flight across it; they are issued with
-// clamped indices and masked where the values are taken.
+// only, so those loads stay in flight across it.
+// A plane is addressed as a raw buffer, so the offsets of a thread's cells stay
+// the same through the march; what a plane needs besides (image, injected row)
+// is loaded at its start. us a step, 203 x 181 x 247 (bound by latency and
+// vector instructions) and 522^3 (bound by memory: the step moves 2.7 GB, 5.6
+// TB/s, of which 0.5 GB are halo lines fetched twice): through pointers 42 and
+// 526, with the image 60 and 970; now 33 and 480, 56 and 767.
 // The halo cells of a plane are loaded with the queue entry of the same
 // plane, five planes before it is computed: that is when the neighbouring
 // tiles load those cells as their own queue entries, so the second read of
 // each line is an L2 hit rather than a second fetch. Each thread keeps its
 // halo cells of the five planes ahead in a ring in LDS (slot = plane % 5)
 // that only it reads.
-template <bool IMG>
-__global__ __launch_bounds__(256) void k_ac3_step(const Ac3Args a) {
-  __shared__ float sh[2][ALX * ALZ];
+// What a step does besides: nothing, update the image (receiver pass at an
+// imaging level), or store the snapshot of the level it reads (source pass: the
+// level's max-abs is complete and its cells are at hand in the queue, so the
+// snapshot costs its own bytes only; a pass of its own read the field again).
+enum StepKind { STEP_PLAIN, STEP_IMAGE, STEP_SNAP };
+
+// The max-abs of a snapshot is kept in SMAX_SLOTS partial maxima, each on a cache
+// line of its own: thousands of waves that end together would queue at one
+// address (203 x 181 x 247: 66 us a step against 33 without the maximum).
+constexpr int SMAX_SLOTS = 32, SMAX_STRIDE = 32, SMAX_SNAP = SMAX_SLOTS * SMAX_STRIDE;
+__device__ __forceinline__ float snap_max(const unsigned* m) {
+  float v = __uint_as_float(m[(threadIdx.x & (SMAX_SLOTS - 1)) * SMAX_STRIDE]);
+#pragma unroll
+  for (int o = SMAX_SLOTS / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ float snap_inv(const unsigned* m) {
+  const float v = snap_max(m);
+  return v > 1e-30f ? 1.f / v : 0.f;  // subnormal maxima would overflow 1/v
+}
+__device__ __forceinline__ unsigned short snap_bf16(float v, float inv) {
+  unsigned u = __float_as_uint(v * inv);
+  u += 0x7fffu + ((u >> 16) & 1u);
+  return (unsigned short)(u >> 16);
+}
+
+template <int KIND>
+__global__ __launch_bounds__(256, 4) void k_ac3_step(const Ac3Args a) {
+  __shared__ float sh[2][ALX * ALZ + 1];  // the last one takes the threads without a halo cell
   __shared__ float hring[5][ANH][256];
   const int nbz = (a.n1 - 10 + AZ - 1) / AZ;
   const int nbx = (a.n2 - 10 + AX - 1) / AX;
@@ -124,94 +160,107 @@ __global__ __launch_bounds__(256) void k_ac3_step(const Ac3Args a) {
   const int tid = tz + AZ * ty;
   const int gz = z0 + tz;
   const bool zok = gz < a.n1 - AH;
-  // element offsets of one field fit in 32 bits (the host checks n < 2^31)
-  const int s2 = (int)a.s2, s3 = (int)a.s3;
-  constexpr bool imaging = IMG;  // receiver pass at an imaging level
-  // per-thread halo cells (plane independent): LDS slot (-1: none) and
-  // in-plane offset (-1: outside the grid, staged as zero)
-  int hoff[ANH], hlds[ANH];
+  const int s2 = (int)a.s2;
+  const unsigned plane = 4u * (unsigned)a.s3;  // bytes of a plane, which a buffer covers
+  constexpr bool imaging = KIND == STEP_IMAGE;
+  const float inv = KIND == STEP_SNAP && a.snap_bf16 ? snap_inv(a.snap_max) : 0.f;
+  auto at = [&](const float* f, int y) { return Buf(f + (long long)y * a.s3, plane); };
+  // per-thread halo cells (plane independent): LDS slot and byte
+  // offset in a plane (kOutside: outside the grid, staged as zero)
+  int hlds[ANH];
+  unsigned hoff[ANH];
 #pragma unroll
   for (int k = 0; k < ANH; ++k) {
     const int h = tid + 256 * k;
     int lx = 0, lz = 0;
-    hlds[k] = -1;
-    hoff[k] = -1;
+    hlds[k] = ALX * ALZ;
+    hoff[k] = kOutside;
     if (h < AHALO) {
       halo_cell(h, lx, lz);
       hlds[k] = lx * ALZ + lz;
       const int gx = x0 - AH + lx, g1v = z0 - AH + lz;
-      if (gx >= 0 && gx < a.n2 && g1v >= 0 && g1v < a.n1) hoff[k] = g1v + gx * s2;
+      if (gx >= 0 && gx < a.n2 && g1v >= 0 && g1v < a.n1) hoff[k] = 4u * (unsigned)(g1v + gx * s2);
     }
   }
-  int coff[ATXR];  // own columns (-1: outside the interior)
+  // own columns (kOutside: outside the interior, where every value is zero and
+  // nothing is written), and their sponge factors of row and column
+  unsigned coff[ATXR];
+  float kzx[ATXR];
+  auto sc = [](const float* p, int i) { return ((const __attribute__((address_space(4))) float*)p)[i]; };
+  const float kzv = (a.kz && zok) ? g1(a.kz, gz) : 1.f;
 #pragma unroll
   for (int j = 0; j < ATXR; ++j) {
     const int gx = x0 + ty * ATXR + j;
-    coff[j] = (zok && gx < a.n2 - AH) ? gz + gx * s2 : -1;
+    coff[j] = (zok && gx < a.n2 - AH) ? 4u * (unsigned)(gz + gx * s2) : kOutside;
+    kzx[j] = a.kz ? kzv * sc(a.kx, min(gx, a.n2 - 1)) : 1.f;
   }
   // register queue: q[k][j] = p at plane y-5+k
   float q[11][ATXR];
 #pragma unroll
-  for (int k = 0; k < 10; ++k)
+  for (int k = 0; k < 10; ++k) {
+    const Buf p = at(a.p, y0 - AH + k);
 #pragma unroll
-    for (int j = 0; j < ATXR; ++j) {
-      const bool ok = coff[j] >= 0;
-      const float v = g1(a.p, ok ? coff[j] + (y0 - AH + k) * s3 : 0);
-      q[k][j] = ok ? v : 0.f;
-    }
-  float hv[ANH], ppv[ATXR], cv[ATXR], snv[ATXR], imv[ATXR], qn[ATXR];
-  // raw loads of plane y (clamped indices; own-cell values are used only
-  // where coff >= 0, queue and halo values are masked where taken)
+    for (int j = 0; j < ATXR; ++j) q[k][j] = p.get(coff[j]);
+  }
+  float hv[ANH], ppv[ATXR], cv[ATXR], snv[ATXR], qn[ATXR];
+  // loads of plane y: own cells, and with the queue entry of plane y+5 its halo
   auto load_plane = [&](int y, float (&h)[ANH], float (&qv)[ATXR], float (&pv)[ATXR], float (&c)[ATXR],
-                        float (&sn)[ATXR], float (&im)[ATXR]) {
-    const int py = y * s3;
+                        float (&sn)[ATXR]) {
+    const Buf p5 = at(a.p, y + AH), pp = at(a.pp, y), cc = at(a.c, y);
 #pragma unroll
     for (int j = 0; j < ATXR; ++j) {
-      const int o = coff[j] >= 0 ? coff[j] + py : 0;
-      qv[j] = g1(a.p, coff[j] >= 0 ? o + AH * s3 : 0);
-      pv[j] = g1(static_cast<const float*>(a.pp), o);
-      c[j] = g1(a.c, o);
-      sn[j] = 0.f;
-      im[j] = 0.f;
-      if (imaging) {
-        sn[j] = a.snap_bf16 ? bf16_to_f(g1(static_cast<const unsigned short*>(a.snap), o)) * a.snap_scale
-                            : g1(static_cast<const float*>(a.snap), o);
-        im[j] = g1(static_cast<const float*>(a.img), o);
+      qv[j] = p5.get(coff[j]);
+      pv[j] = pp.get(coff[j]);
+      c[j] = cc.get(coff[j]);
+    }
+    if (imaging) {
+      const Buf sb(static_cast<const char*>(a.snap) + (long long)y * (a.snap_bf16 ? plane / 2 : plane), plane);
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j) {
+        sn[j] = a.snap_bf16 ? bf16_to_f(sb.get16(coff[j] / 2)) * a.snap_scale : sb.get(coff[j]);
       }
     }
-    // halo cells of plane y+5, with its queue entry
 #pragma unroll
-    for (int k = 0; k < ANH; ++k) h[k] = g1(a.p, hoff[k] >= 0 ? hoff[k] + py + AH * s3 : 0);
+    for (int k = 0; k < ANH; ++k) h[k] = p5.get(hoff[k]);
   };
   // halo cells of the first five planes into the ring
 #pragma unroll
   for (int j = 0; j < AH; ++j) {
-    const int py = (y0 + j) * s3;
+    const Buf p = at(a.p, y0 + j);
 #pragma unroll
-    for (int k = 0; k < ANH; ++k) {
-      const float v = g1(a.p, hoff[k] >= 0 ? hoff[k] + py : 0);
-      hring[(y0 + j) % 5][k][tid] = hoff[k] >= 0 ? v : 0.f;
-    }
+    for (int k = 0; k < ANH; ++k) hring[(y0 + j) % 5][k][tid] = p.get(hoff[k]);
   }
-  if (y0 < y1) load_plane(y0, hv, qn, ppv, cv, snv, imv);
+  if (y0 < y1) load_plane(y0, hv, qn, ppv, cv, snv);
   float mx = 0.f;
-  // sponge factors: kz of the thread's row (loop invariant), kx of the
-  // wave's columns and ky of the plane (wave-uniform, scalar loads)
-  const float kzv = (a.kz && zok) ? g1(a.kz, gz) : 1.f;
-  auto sc = [](const float* p, int i) { return ((const __attribute__((address_space(4))) float*)p)[i]; };
+  // receiver row: recorded (source pass), or injected from loads issued before
+  // the plane's arithmetic
+  const bool row = gz == a.zr && a.mode == 0 && a.rec_out;
+  const bool inject = a.mode != 0 && a.rec_in && a.zr >= z0 && a.zr < z0 + AZ;  // uniform over the workgroup
   for (int y = y0; y < y1; ++y) {
     const int bb = (y - y0) & 1;
     float* const sp = sh[bb];
+    // the image and the injected row: loaded here, not a plane ahead (registers)
+    float rv[ATXR], imv[ATXR];
+    if (imaging) {
+      const Buf ib = at(a.img, y);
 #pragma unroll
-    for (int j = 0; j < ATXR; ++j) q[10][j] = coff[j] >= 0 ? qn[j] : 0.f;
+      for (int j = 0; j < ATXR; ++j) imv[j] = ib.get(coff[j]);
+    }
+    if (inject) {
+      const Buf r(a.rec_in + (long long)y * a.n2, 4u * (unsigned)a.n2);
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j) rv[j] = r.get(gz == a.zr ? 4u * (unsigned)(x0 + ty * ATXR + j) : kOutside);
+    }
+#pragma unroll
+    for (int j = 0; j < ATXR; ++j) q[10][j] = qn[j];
 #pragma unroll
     for (int j = 0; j < ATXR; ++j) sp[(ty * ATXR + j + AH) * ALZ + tz + AH] = q[5][j];
     // this plane's halo cells from the ring; the slot then takes plane y+5's
     const int slot = y % 5;
 #pragma unroll
     for (int k = 0; k < ANH; ++k) {
-      if (hlds[k] >= 0) sp[hlds[k]] = hring[slot][k][tid];
-      hring[slot][k][tid] = hoff[k] >= 0 ? hv[k] : 0.f;
+      sp[hlds[k]] = hring[slot][k][tid];
+      hring[slot][k][tid] = hv[k];
     }
     // the tile of plane y is complete; plane y-1's buffer is free again
     // once every wave has passed this barrier
@@ -219,39 +268,56 @@ __global__ __launch_bounds__(256) void k_ac3_step(const Ac3Args a) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     // issue the next plane's loads before this plane's arithmetic
-    float hv2[ANH], pp2[ATXR], c2[ATXR], sn2[ATXR], im2[ATXR];
-    load_plane(y + 1 < y1 ? y + 1 : y, hv2, qn, pp2, c2, sn2, im2);
-    const int py = y * s3;
-    if (zok) {
-      const float kyv = a.kz ? sc(a.ky, y) : 1.f;
+    float hv2[ANH], pp2[ATXR], c2[ATXR], sn2[ATXR];
+    load_plane(y + 1 < y1 ? y + 1 : y, hv2, qn, pp2, c2, sn2);
+    const float kyv = a.kz ? sc(a.ky, y) : 1.f;
+    const Buf out = at(a.pp, y);
+    float v[ATXR];
+#pragma unroll
+    for (int j = 0; j < ATXR; ++j) {
+      const int p0 = (ty * ATXR + j + AH) * ALZ + tz + AH;
+      float lap = 3.f * W0 * q[5][j];
+      lap += W1 * ((sp[p0 + 1] + sp[p0 - 1]) + (sp[p0 + ALZ] + sp[p0 - ALZ]) + (q[6][j] + q[4][j]));
+      lap += W2 * ((sp[p0 + 2] + sp[p0 - 2]) + (sp[p0 + 2 * ALZ] + sp[p0 - 2 * ALZ]) + (q[7][j] + q[3][j]));
+      lap += W3 * ((sp[p0 + 3] + sp[p0 - 3]) + (sp[p0 + 3 * ALZ] + sp[p0 - 3 * ALZ]) + (q[8][j] + q[2][j]));
+      lap += W4 * ((sp[p0 + 4] + sp[p0 - 4]) + (sp[p0 + 4 * ALZ] + sp[p0 - 4 * ALZ]) + (q[9][j] + q[1][j]));
+      lap += W5 * ((sp[p0 + 5] + sp[p0 - 5]) + (sp[p0 + 5 * ALZ] + sp[p0 - 5 * ALZ]) + (q[10][j] + q[0][j]));
+      v[j] = kzx[j] * kyv * (2.f * q[5][j] - ppv[j] + cv[j] * lap);
+    }
+    if (a.mode == 0 && y == a.sy) {
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j)
+        if (gz == a.sz && x0 + ty * ATXR + j == a.sx) v[j] += a.amp;
+    }
+    if (inject) {
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j) v[j] = gz == a.zr ? v[j] + rv[j] : v[j];
+    }
+    if (row) {
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j)
+        if (coff[j] != kOutside) a.rec_out[(long long)y * a.n2 + x0 + ty * ATXR + j] = v[j];
+    }
+#pragma unroll
+    for (int j = 0; j < ATXR; ++j) out.put(coff[j], 0, v[j]);
+    if (KIND == STEP_SNAP) {
+      const Buf so(static_cast<char*>(a.snap_out) + (long long)y * (a.snap_bf16 ? plane / 2 : plane), plane);
 #pragma unroll
       for (int j = 0; j < ATXR; ++j) {
-        const int lxo = ty * ATXR + j;
-        const int gx = x0 + lxo;
-        if (coff[j] < 0) continue;
-        const int p0 = (lxo + AH) * ALZ + tz + AH;
-        float lap = 3.f * W0 * q[5][j];
-        lap += W1 * ((sp[p0 + 1] + sp[p0 - 1]) + (sp[p0 + ALZ] + sp[p0 - ALZ]) + (q[6][j] + q[4][j]));
-        lap += W2 * ((sp[p0 + 2] + sp[p0 - 2]) + (sp[p0 + 2 * ALZ] + sp[p0 - 2 * ALZ]) + (q[7][j] + q[3][j]));
-        lap += W3 * ((sp[p0 + 3] + sp[p0 - 3]) + (sp[p0 + 3 * ALZ] + sp[p0 - 3 * ALZ]) + (q[8][j] + q[2][j]));
-        lap += W4 * ((sp[p0 + 4] + sp[p0 - 4]) + (sp[p0 + 4 * ALZ] + sp[p0 - 4 * ALZ]) + (q[9][j] + q[1][j]));
-        lap += W5 * ((sp[p0 + 5] + sp[p0 - 5]) + (sp[p0 + 5 * ALZ] + sp[p0 - 5 * ALZ]) + (q[10][j] + q[0][j]));
-        const int gi = coff[j] + py;
-        const float kk = a.kz ? kzv * sc(a.kx, gx) * kyv : 1.f;
-        float v = kk * (2.f * q[5][j] - ppv[j] + cv[j] * lap);
-        if (a.mode == 0) {
-          if (gz == a.sz && gx == a.sx && y == a.sy) v += a.amp;
-        } else if (a.rec_in && gz == a.zr) {
-          v += a.rec_in[(long long)y * a.n2 + gx];
-        }
-        a.pp[gi] = v;
-        if (a.mode == 0) {
-          if (a.rec_out && gz == a.zr) a.rec_out[(long long)y * a.n2 + gx] = v;
-          mx = fmaxf(mx, fabsf(v));
-        } else if (imaging) {
-          a.img[gi] = imv[j] + snv[j] * v;
-        }
+        if (a.snap_bf16)
+          so.put16(coff[j] / 2, snap_bf16(q[5][j], inv));
+        else
+          so.put(coff[j], 0, q[5][j]);
       }
+    }
+    if (imaging) {
+      const Buf io = at(a.img, y);
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j) io.put(coff[j], 0, imv[j] + snv[j] * v[j]);
+    }
+    if (a.smax) {
+#pragma unroll
+      for (int j = 0; j < ATXR; ++j) mx = coff[j] != kOutside ? fmaxf(mx, fabsf(v[j])) : mx;
     }
 #pragma unroll
     for (int k = 0; k < 10; ++k)
@@ -264,30 +330,38 @@ __global__ __launch_bounds__(256) void k_ac3_step(const Ac3Args a) {
       ppv[j] = pp2[j];
       cv[j] = c2[j];
       snv[j] = sn2[j];
-      imv[j] = im2[j];
     }
   }
   if (a.mode == 0 && a.smax) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if (tz == 0) atomicMax(a.smax, __float_as_uint(mx));
+    if (tz == 0) atomicMax(a.smax + ((blockIdx.x * AWY + ty) & (SMAX_SLOTS - 1)) * SMAX_STRIDE, __float_as_uint(mx));
   }
 }
 
-// Snapshot of one level: bf16 with the level's max-abs scale, or fp32 copy.
+// Snapshot of the last level (no later step reads it): bf16 with the level's
+// max-abs scale, or fp32 copy.
 __global__ void k_ac3_snap(const float* p, void* out, size_t n, const unsigned* smax, int bf16) {
-  const float m = __uint_as_float(*smax);
-  const float inv = m > 1e-30f ? 1.f / m : 0.f;  // subnormal maxima would overflow 1/m
+  const float inv = snap_inv(smax);
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x) {
-    if (bf16) {
-      unsigned u = __float_as_uint(p[i] * inv);
-      u += 0x7fffu + ((u >> 16) & 1u);
-      static_cast<unsigned short*>(out)[i] = (unsigned short)(u >> 16);
-    } else {
+    if (bf16)
+      static_cast<unsigned short*>(out)[i] = snap_bf16(p[i], inv);
+    else
       static_cast<float*>(out)[i] = p[i];
-    }
   }
+}
+
+// The max-abs of every snapshot.
+__global__ void k_ac3_scales(const unsigned* smax, float* out) {
+  const float v = snap_max(smax + (size_t)blockIdx.x * SMAX_SNAP);
+  if (threadIdx.x == 0) out[blockIdx.x] = v;
+}
+
+// Rows of n1 cells, contiguous on one side and ld apart on the other.
+__global__ void k_ac3_rows(const float* in, float* out, int n1, long long rows, int ld_in, int ld_out) {
+  for (long long r = blockIdx.x * (long long)blockDim.y + threadIdx.y; r < rows; r += (long long)gridDim.x * blockDim.y)
+    for (int z = threadIdx.x; z < n1; z += blockDim.x) out[r * ld_out + z] = in[r * ld_in + z];
 }
 
 __global__ void k_fill3(float* p, size_t n) {
@@ -335,7 +409,7 @@ int resident_workgroups() {
     int dev = 0, cus = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_ac3_step<false>, AZ * AWY, 0) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_ac3_step<STEP_PLAIN>, AZ * AWY, 0) != hipSuccess ||
         cus * per <= 0)
       return 1024;
     return cus * per;
@@ -350,7 +424,7 @@ int resident_workgroups() {
 // source-pass step: 203 x 181 x 247 (44 tiles) 64 planes 115 us, 12 planes
 // 42 us; 266^3 64 planes 115 us, 16 planes (one whole round) 59 us; 64^3 64
 // planes 94 us, 8 planes 18 us. At 522^3 (256 tiles), where memory bounds the
-// step, 20 to 128 planes take 530 to 558 us.
+// step, 64 to 128 planes take 1 to 9% more or less.
 int planes_per_workgroup(int tiles, int n) {
   const int resident = resident_workgroups();
   long long best = -1;
@@ -376,7 +450,16 @@ using namespace erm;
 
 struct ac3d {
   ac3d_cfg_t cfg{};
-  size_t n = 0;
+  size_t n = 0;         // cells
+  // Device layout of a field: cell (z, x, y) at lead + z + ld (x + n2 y). With
+  // lead 27 and ld a multiple of 64 the first interior cell of every row (z = 5)
+  // lies on a 128-byte line, so a wave's row is two lines instead of three; a
+  // snapshot starts 32 elements later (slead), which does the same for its
+  // 16-bit rows (522^3: 10% fewer L2 requests, step 565 -> 526 us, with the image
+  // 1064 -> 970). Where memory or 32-bit offsets do not allow it, rows are
+  // contiguous.
+  int lead = 0, slead = 0, ld = 0;
+  size_t np = 0, ns = 0;  // elements of a field and of a snapshot
   long long plane = 0;
   int ychunk = 0;  // planes per step workgroup
   DevBuf c, c_alt, k, f0, f1, rec, rec_tmp, snap, smax, img, amp_h_dummy;
@@ -385,6 +468,10 @@ struct ac3d {
   hipStream_t st = nullptr;
   hipEvent_t ev[2] = {};
   double timings[6] = {0, 0, 0, 0, 0, 0};
+  void* snap_at(int k) const {  // snapshot k, as the step kernel indexes it
+    const size_t esz = cfg.snap_prec == 1 ? 2 : 4;
+    return snap.as<char>() + ((size_t)k * ns + slead) * esz;
+  }
   ~ac3d() {
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
@@ -393,12 +480,13 @@ struct ac3d {
 };
 
 static int ac3_launch(ac3d* a, const float* p, float* pp, const float* c, int mode, int level, bool record,
-                      bool inject, unsigned* smax, const void* snap, float scale, float* img) {
+                      bool inject, unsigned* smax, const void* snap, float scale, float* img,
+                      void* snap_out = nullptr, const unsigned* snap_max = nullptr) {
   const ac3d_cfg_t& g = a->cfg;
   Ac3Args x{};
   x.n1 = g.n1; x.n2 = g.n2; x.n3 = g.n3;
-  x.s2 = g.n1;
-  x.s3 = (long long)g.n1 * g.n2;
+  x.s2 = a->ld;
+  x.s3 = (long long)a->ld * g.n2;
   x.p = p; x.pp = pp; x.c = c;
   if (g.abc > 0) {
     x.kz = a->k.as<float>();
@@ -416,25 +504,45 @@ static int ac3_launch(ac3d* a, const float* p, float* pp, const float* c, int mo
   x.snap_scale = scale;
   x.snap_bf16 = g.snap_prec == 1;
   x.img = img;
+  x.snap_out = snap_out;
+  x.snap_max = snap_max;
   x.ychunk = a->ychunk;
   const int nbz = (g.n1 - 10 + AZ - 1) / AZ, nbx = (g.n2 - 10 + AX - 1) / AX;
   const int nby = (g.n3 - 10 + x.ychunk - 1) / x.ychunk;
   if (mode == 1 && img)
-    hipLaunchKernelGGL(k_ac3_step<true>, dim3(nbz * nbx * nby), dim3(AZ, AWY), 0, a->st, x);
+    hipLaunchKernelGGL(k_ac3_step<STEP_IMAGE>, dim3(nbz * nbx * nby), dim3(AZ, AWY), 0, a->st, x);
+  else if (snap_out)
+    hipLaunchKernelGGL(k_ac3_step<STEP_SNAP>, dim3(nbz * nbx * nby), dim3(AZ, AWY), 0, a->st, x);
   else
-    hipLaunchKernelGGL(k_ac3_step<false>, dim3(nbz * nbx * nby), dim3(AZ, AWY), 0, a->st, x);
+    hipLaunchKernelGGL(k_ac3_step<STEP_PLAIN>, dim3(nbz * nbx * nby), dim3(AZ, AWY), 0, a->st, x);
   HIPCHK(hipGetLastError());
   return OK;
+}
+
+// Rows between the caller's layout and the device's; the source field of the
+// passes, which begin with a fill of their own, carries the contiguous side.
+static int ac3_rows(ac3d* a, const float* in, float* out, int ld_in, int ld_out) {
+  const long long rows = a->plane;
+  hipLaunchKernelGGL(k_ac3_rows, dim3((unsigned)std::min<long long>((rows + 3) / 4, 65536)), dim3(64, 4), 0, a->st, in,
+                     out, a->cfg.n1, rows, ld_in, ld_out);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(a->st));
+  return OK;
+}
+static int ac3_upload(ac3d* a, const float* host, float* dev) {
+  if (a->ld == a->cfg.n1) return copy_to_device(dev, host, a->n * 4);
+  STCHK(copy_to_device(a->f0.p, host, a->n * 4));
+  return ac3_rows(a, a->f0.as<float>(), dev + a->lead, a->cfg.n1, a->ld);
 }
 
 // Source pass: levels 1..nt with the model c; records the receiver plane
 // (subtracting when sub) and, with snapshots, stores every j-th level.
 static int ac3_source_pass(ac3d* a, const float* c, int record, int sub, int snaps) {
   const ac3d_cfg_t& g = a->cfg;
-  float* p = a->f0.as<float>();
-  float* pp = a->f1.as<float>();
-  STCHK(fill0(p, a->n, a->st));
-  STCHK(fill0(pp, a->n, a->st));
+  STCHK(fill0(a->f0.as<float>(), a->np, a->st));
+  STCHK(fill0(a->f1.as<float>(), a->np, a->st));
+  float* p = a->f0.as<float>() + a->lead;
+  float* pp = a->f1.as<float>() + a->lead;
   float* rec_dst = nullptr;
   if (record) {
     if (sub) {
@@ -445,17 +553,18 @@ static int ac3_source_pass(ac3d* a, const float* c, int record, int sub, int sna
   }
   const int j = g.snap_every;
   const int nsnap = g.nt / j;
-  if (snaps) HIPCHK(hipMemsetAsync(a->smax.p, 0, sizeof(unsigned) * std::max(nsnap, 1), a->st));
+  if (snaps) HIPCHK(hipMemsetAsync(a->smax.p, 0, sizeof(unsigned) * SMAX_SNAP * std::max(nsnap, 1), a->st));
   for (int t = 1; t <= g.nt; ++t) {
     const bool sl = snaps && t % j == 0;
-    unsigned* sm = sl ? a->smax.as<unsigned>() + (t / j - 1) : nullptr;
-    STCHK(ac3_launch(a, p, pp, c, 0, t, record != 0, false, sm, nullptr, 0.f, nullptr));
-    if (sl) {
-      const size_t esz = g.snap_prec == 1 ? 2 : 4;
-      char* dst = a->snap.as<char>() + (size_t)(t / j - 1) * a->n * esz;
-      size_t blocks = std::min<size_t>((a->n + 255) / 256, 65536);
-      hipLaunchKernelGGL(k_ac3_snap, dim3((unsigned)blocks), dim3(256), 0, a->st, pp, (void*)dst, a->n, sm,
-                         g.snap_prec == 1);
+    unsigned* sm = sl ? a->smax.as<unsigned>() + (size_t)(t / j - 1) * SMAX_SNAP : nullptr;
+    // the snapshot of the level this step reads
+    const int k = snaps && t > 1 && (t - 1) % j == 0 ? (t - 1) / j - 1 : -1;
+    STCHK(ac3_launch(a, p, pp, c, 0, t, record != 0, false, sm, nullptr, 0.f, nullptr, k < 0 ? nullptr : a->snap_at(k),
+                     k < 0 ? nullptr : a->smax.as<unsigned>() + (size_t)k * SMAX_SNAP));
+    if (sl && t == g.nt) {
+      size_t blocks = std::min<size_t>((a->np + 255) / 256, 65536);
+      hipLaunchKernelGGL(k_ac3_snap, dim3((unsigned)blocks), dim3(256), 0, a->st, pp, a->snap_at(t / j - 1),
+                         a->np - a->lead, sm, g.snap_prec == 1);
       HIPCHK(hipGetLastError());
     }
     std::swap(p, pp);
@@ -497,6 +606,25 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
     return E_ARG;
   }
   a->plane = (long long)g.n2 * g.n3;
+  const int nsnap = std::max(g.nt / g.snap_every, 1);
+  const size_t esz = g.snap_prec == 1 ? 2 : 4;
+  a->ld = g.n1;
+  a->np = a->ns = a->n;
+  {
+    const int ld = round_up(27 + g.n1, 64);
+    const size_t np = (size_t)ld * a->plane, ns = np + 64;
+    const size_t need = 5 * np * 4 + (size_t)nsnap * ns * esz + 2 * (size_t)g.nt * a->plane * 4;
+    size_t freeb = 0, totb = 0;
+    HIPCHK(hipMemGetInfo(&freeb, &totb));
+    const char* pad = getenv("RTM_AC3_PAD");  // 0: contiguous rows (experiments)
+    if (np < (size_t)1 << 31 && need < freeb / 10 * 9 && !(pad && atoi(pad) == 0)) {
+      a->ld = ld;
+      a->lead = 27;
+      a->slead = 59;
+      a->np = np;
+      a->ns = ns;
+    }
+  }
   // RTM_AC3_YCHUNK overrides the planes per workgroup (experiments)
   const char* fixed = getenv("RTM_AC3_YCHUNK");
   a->ychunk = fixed && atoi(fixed) > 0
@@ -504,21 +632,20 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
                   : planes_per_workgroup(((g.n1 - 10 + AZ - 1) / AZ) * ((g.n2 - 10 + AX - 1) / AX), g.n3 - 10);
   HIPCHK(hipStreamCreateWithFlags(&a->st, hipStreamNonBlocking));
   for (auto& e : a->ev) HIPCHK(hipEventCreate(&e));
-  STCHK(a->c.alloc(a->n * 4, "velocity term"));
-  STCHK(copy_to_device(a->c.p, c, a->n * 4));
+  STCHK(a->c.alloc(a->np * 4, "velocity term"));
+  STCHK(a->f0.alloc(a->np * 4, "wavefield"));
+  STCHK(a->f1.alloc(a->np * 4, "wavefield"));
+  STCHK(ac3_upload(a.get(), c, a->c.as<float>()));
   STCHK(a->k.alloc((size_t)(g.n1 + g.n2 + g.n3) * 4, "sponge"));
   std::vector<float> k1 = taper(g.n1, g.abc), k2 = taper(g.n2, g.abc), k3 = taper(g.n3, g.abc);
   HIPCHK(hipMemcpy(a->k.p, k1.data(), g.n1 * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(a->k.as<float>() + g.n1, k2.data(), g.n2 * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(a->k.as<float>() + g.n1 + g.n2, k3.data(), g.n3 * 4, hipMemcpyHostToDevice));
-  STCHK(a->f0.alloc(a->n * 4, "wavefield"));
-  STCHK(a->f1.alloc(a->n * 4, "wavefield"));
   STCHK(a->rec.alloc((size_t)g.nt * a->plane * 4, "receiver data"));
   STCHK(fill0(a->rec.as<float>(), (size_t)g.nt * a->plane, a->st));
-  STCHK(a->img.alloc(a->n * 4, "image"));
-  const int nsnap = std::max(g.nt / g.snap_every, 1);
-  STCHK(a->snap.alloc((size_t)nsnap * a->n * (g.snap_prec == 1 ? 2 : 4), "snapshots"));
-  STCHK(a->smax.alloc(sizeof(unsigned) * nsnap, "snapshot scales"));
+  STCHK(a->img.alloc(a->np * 4, "image"));
+  STCHK(a->snap.alloc((size_t)nsnap * a->ns * esz, "snapshots"));
+  STCHK(a->smax.alloc(sizeof(unsigned) * (SMAX_SNAP + 1) * nsnap, "snapshot scales"));
   a->amp.assign(amp, amp + g.nt);
   HIPCHK(hipStreamSynchronize(a->st));
   *out = a.release();
@@ -531,14 +658,14 @@ RTM_EXPORT int ac3d_model_data(ac3d* a, const float* c_true) {
   // else the migration-model data
   HIPCHK(hipEventRecord(a->ev[0], a->st));
   if (c_true) {
-    STCHK(a->c_alt.alloc(a->n * 4, "true model"));
-    STCHK(copy_to_device(a->c_alt.p, c_true, a->n * 4));
+    STCHK(a->c_alt.alloc(a->np * 4, "true model"));
+    STCHK(ac3_upload(a, c_true, a->c_alt.as<float>()));
     if (!a->rec_tmp.p) STCHK(a->rec_tmp.alloc((size_t)a->cfg.nt * a->plane * 4, "receiver scratch"));
-    STCHK(ac3_source_pass(a, a->c_alt.as<float>(), 1, 0, 0));
-    STCHK(ac3_source_pass(a, a->c.as<float>(), 1, 1, 0));
+    STCHK(ac3_source_pass(a, a->c_alt.as<float>() + a->lead, 1, 0, 0));
+    STCHK(ac3_source_pass(a, a->c.as<float>() + a->lead, 1, 1, 0));
     a->c_alt.release();
   } else {
-    STCHK(ac3_source_pass(a, a->c.as<float>(), 1, 0, 0));
+    STCHK(ac3_source_pass(a, a->c.as<float>() + a->lead, 1, 0, 0));
   }
   HIPCHK(hipEventRecord(a->ev[1], a->st));
   HIPCHK(hipStreamSynchronize(a->st));
@@ -552,35 +679,34 @@ RTM_EXPORT int ac3d_migrate(ac3d* a) {
   if (!a) { set_error("null handle"); return E_ARG; }
   const ac3d_cfg_t& g = a->cfg;
   HIPCHK(hipEventRecord(a->ev[0], a->st));
-  STCHK(ac3_source_pass(a, a->c.as<float>(), 0, 0, 1));
+  STCHK(ac3_source_pass(a, a->c.as<float>() + a->lead, 0, 0, 1));
   HIPCHK(hipEventRecord(a->ev[1], a->st));
   HIPCHK(hipStreamSynchronize(a->st));
   float ms_src = 0;
   HIPCHK(hipEventElapsedTime(&ms_src, a->ev[0], a->ev[1]));
   const int j = g.snap_every;
   const int nsnap = g.nt / j;
-  std::vector<unsigned> sm(std::max(nsnap, 1));
-  HIPCHK(hipMemcpy(sm.data(), a->smax.p, sizeof(unsigned) * sm.size(), hipMemcpyDeviceToHost));
-  a->scales.resize(sm.size());
-  for (size_t i = 0; i < sm.size(); ++i) {
-    float f;
-    std::memcpy(&f, &sm[i], 4);
-    a->scales[i] = f;
+  a->scales.assign(std::max(nsnap, 1), 0.f);
+  if (nsnap > 0) {
+    float* scales = reinterpret_cast<float*>(a->smax.as<unsigned>() + (size_t)nsnap * SMAX_SNAP);
+    hipLaunchKernelGGL(k_ac3_scales, dim3(nsnap), dim3(64), 0, a->st, a->smax.as<unsigned>(), scales);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(a->st));
+    HIPCHK(hipMemcpy(a->scales.data(), scales, sizeof(float) * nsnap, hipMemcpyDeviceToHost));
   }
   // receiver pass, levels nt..1
-  float* q = a->f0.as<float>();
-  float* qq = a->f1.as<float>();
-  STCHK(fill0(q, a->n, a->st));
-  STCHK(fill0(qq, a->n, a->st));
-  STCHK(fill0(a->img.as<float>(), a->n, a->st));
+  STCHK(fill0(a->f0.as<float>(), a->np, a->st));
+  STCHK(fill0(a->f1.as<float>(), a->np, a->st));
+  STCHK(fill0(a->img.as<float>(), a->np, a->st));
+  float* q = a->f0.as<float>() + a->lead;
+  float* qq = a->f1.as<float>() + a->lead;
   HIPCHK(hipEventRecord(a->ev[0], a->st));
-  const size_t esz = g.snap_prec == 1 ? 2 : 4;
   for (int t = g.nt; t >= 1; --t) {
     const bool il = t % j == 0;
-    const void* sp = il ? a->snap.as<char>() + (size_t)(t / j - 1) * a->n * esz : nullptr;
+    const void* sp = il ? a->snap_at(t / j - 1) : nullptr;
     const float sc = il ? a->scales[t / j - 1] : 0.f;
-    STCHK(ac3_launch(a, q, qq, a->c.as<float>(), 1, t, false, true, nullptr, sp, sc,
-                     il ? a->img.as<float>() : nullptr));
+    STCHK(ac3_launch(a, q, qq, a->c.as<float>() + a->lead, 1, t, false, true, nullptr, sp, sc,
+                     il ? a->img.as<float>() + a->lead : nullptr));
     std::swap(q, qq);
   }
   HIPCHK(hipEventRecord(a->ev[1], a->st));
@@ -608,7 +734,9 @@ RTM_EXPORT int ac3d_get_data(ac3d* a, float* rec) {
 RTM_EXPORT int ac3d_get_image(ac3d* a, float* img) {
   if (!a || !img) { set_error("null argument"); return E_ARG; }
   HIPCHK(hipStreamSynchronize(a->st));
-  return copy_to_host(img, a->img.p, a->n * 4);
+  if (a->ld == a->cfg.n1) return copy_to_host(img, a->img.p, a->n * 4);
+  STCHK(ac3_rows(a, a->img.as<float>() + a->lead, a->f0.as<float>(), a->ld, a->cfg.n1));
+  return copy_to_host(img, a->f0.p, a->n * 4);
 }
 
 RTM_EXPORT int ac3d_get_snapshot_scales(ac3d* a, float* out, int n) {

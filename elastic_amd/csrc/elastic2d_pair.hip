@@ -22,6 +22,7 @@
 //
 // Every cell of both levels gets exactly the arithmetic of k_fwd / k_adj, so
 // results are bitwise those of two one-level launches.
+#include "buffer.hpp"
 #include "elastic2d_device.hpp"
 
 #include <cstdlib>
@@ -44,24 +45,6 @@ struct PairArgs {
   float* imgc;
   const float* dm;
 };
-
-// Fields are read and written as raw buffers: the base is a scalar descriptor,
-// the field a scalar offset and the cell one vector register for all arrays
-// (through pointers the compiler forms a 64-bit vector address per access, a
-// seventh of the kernel's vector instructions); an offset past the buffer reads
-// zero and writes nothing, which masks cells outside the grid.
-struct Buf {
-  __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ Buf(const float* p, unsigned floats)
-      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, 4u * floats, 0x00020000)) {}
-  __device__ __forceinline__ float get(unsigned cell, unsigned field) const {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, cell, field, 0));
-  }
-  __device__ __forceinline__ void put(unsigned cell, unsigned field, float v) const {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, cell, field, 0);
-  }
-};
-constexpr unsigned kOutside = 0x80000000u;  // past every buffer: launches take fields of at most kPairCells cells
 
 // OCC: waves a SIMD is to hold (512 / OCC registers; Born modelling would spill).
 template <int TZ_, int TX_, int NT_, int CX_, int OCC_>
@@ -177,15 +160,15 @@ __global__ __launch_bounds__(T::NT, BORN ? 4 : T::OCC) void k_fwd_pair(float* le
   float *const s1 = lds.s1, *const s0 = lds.s0;
   const int ldz = (nz + 31) / 32 * 32, n2 = ldz * nx;
   const unsigned fs = 4u * n2;  // bytes of a field
-  const Buf x2(lev + ((L + 2) & 3) * 5 * n2, 5 * n2), y1(lev + ((L + 3) & 3) * 5 * n2, 5 * n2);
-  const Buf out0(lev + (L & 3) * 5 * n2, 5 * n2), out1(lev + ((L + 1) & 3) * 5 * n2, 5 * n2);
-  const Buf co(coef, 5 * n2), ks(kfac, nz + nx);
+  const Buf x2(lev + ((L + 2) & 3) * 5 * n2, 5 * fs), y1(lev + ((L + 3) & 3) * 5 * n2, 5 * fs);
+  const Buf out0(lev + (L & 3) * 5 * n2, 5 * fs), out1(lev + ((L + 1) & 3) * 5 * n2, 5 * fs);
+  const Buf co(coef, 5 * fs), ks(kfac, 4u * (nz + nx));
   const PairCells<T> k(nz, nx, ldz, ntiles, nbz, flags);
 
   float st[T::NIT][5], bs[BORN ? T::NIT : 1][2];
   // Born: background Vx, Vz of levels L, L+1 and L+2 (past the last one: zero)
   const bool has2 = BORN && L + 2 <= a.nt;
-  const Buf bg(a.snap + (long long)(L - 1) * 2 * n2, BORN ? (has2 ? 6 : 4) * n2 : 0);
+  const Buf bg(a.snap + (long long)(L - 1) * 2 * n2, BORN ? (has2 ? 6 : 4) * fs : 0);
 #pragma unroll
   for (int j = 0; j < T::NIT; ++j) {
     const unsigned gi = staged<T>(k, j, nz, nx, ldz);
@@ -199,7 +182,7 @@ __global__ __launch_bounds__(T::NT, BORN ? 4 : T::OCC) void k_fwd_pair(float* le
   float v[CX][5], m[CX][5], kx[CX], b1[CX][2], b2[CX][2], d[CX][3];
   const bool sponge = flags & F_K;
   const float kz = sponge ? ks.get(4u * k.gz, 0) : 1.f;
-  const Buf dm(a.dm, BORN ? 3 * n2 : 0);
+  const Buf dm(a.dm, BORN ? 3 * fs : 0);
 #pragma unroll
   for (int i = 0; i < CX; ++i) {
     kx[i] = sponge ? ks.get(4u * (k.gx + i), 4u * nz) : 1.f;
@@ -294,7 +277,7 @@ __global__ __launch_bounds__(T::NT, BORN ? 4 : T::OCC) void k_fwd_pair(float* le
       record(a, L + 1, k.gx + i, flags, w[i]);
     }
     if (flags & P_HIST) {
-      const Buf h(a.snap + (long long)(L - 1) * 2 * n2, 4 * n2);
+      const Buf h(a.snap + (long long)(L - 1) * 2 * n2, 4 * fs);
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         h.put(go[i], f * fs, v[i][f]);
@@ -302,7 +285,7 @@ __global__ __launch_bounds__(T::NT, BORN ? 4 : T::OCC) void k_fwd_pair(float* le
       }
     }
     if (flags & F_SNAP) {  // of level L-1
-      const Buf h(a.snap + (long long)a.k0 * 4 * n2, 4 * n2);
+      const Buf h(a.snap + (long long)a.k0 * 4 * n2, 4 * fs);
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         h.put(go[i], f * fs, y[i][f]);
@@ -310,7 +293,7 @@ __global__ __launch_bounds__(T::NT, BORN ? 4 : T::OCC) void k_fwd_pair(float* le
       }
     }
     if (flags & F_SNAP2) {  // of level L
-      const Buf h(a.snap + (long long)a.k1 * 4 * n2, 4 * n2);
+      const Buf h(a.snap + (long long)a.k1 * 4 * n2, 4 * fs);
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         h.put(go[i], f * fs, v[i][f]);
@@ -380,9 +363,9 @@ __global__ __launch_bounds__(T::NT, T::OCC) void k_adj_pair(float* lev, const fl
   float *const s1 = lds.s1, *const s0 = lds.s0, *const sv = lds.sv;
   const int ldz = (nz + 31) / 32 * 32, n2 = ldz * nx;
   const unsigned fs = 4u * n2;  // bytes of a field
-  const Buf x2(lev + ((L + 2) & 3) * 5 * n2, 5 * n2), y1(lev + ((L + 1) & 3) * 5 * n2, 5 * n2);
-  const Buf out0(lev + (L & 3) * 5 * n2, 5 * n2), out1(lev + ((L + 3) & 3) * 5 * n2, 5 * n2);
-  const Buf co(coef, 5 * n2), ks(kfac, nz + nx);
+  const Buf x2(lev + ((L + 2) & 3) * 5 * n2, 5 * fs), y1(lev + ((L + 1) & 3) * 5 * n2, 5 * fs);
+  const Buf out0(lev + (L & 3) * 5 * n2, 5 * fs), out1(lev + ((L + 3) & 3) * 5 * n2, 5 * fs);
+  const Buf co(coef, 5 * fs), ks(kfac, 4u * (nz + nx));
   const PairCells<T> k(nz, nx, ldz, ntiles, nbz, flags);
 
   float st[T::NIT][5];
@@ -413,12 +396,12 @@ __global__ __launch_bounds__(T::NT, T::OCC) void k_adj_pair(float* lev, const fl
   // imaging operands: source Vx, Vz of level L (g0) and L-1 (g1), of level L+1
   // or the differences at the own cells (gn), the images
   const bool hist = flags & P_HIST, imaging = flags & (A_IMG | A_IMG2), next = flags & A_NEXT;
-  const Buf img(a.img, 3 * n2), imgc(a.imgc, (flags & A_COMP) ? 3 * n2 : 0);
+  const Buf img(a.img, 3 * fs), imgc(a.imgc, (flags & A_COMP) ? 3 * fs : 0);
   float g0[CX][2], g1[CX][2], gn[CX][2], im[CX][3], imc[CX][3];
   if (imaging) {
     // history: levels L-1, L and L+1 (past the last one: zero); else the
     // snapshot serves whichever level is imaged
-    const Buf h(hist ? a.snap + (long long)(L - 2) * 2 * n2 : a.snap + (long long)a.k0 * 4 * n2, (hist && next ? 6 : 4) * n2);
+    const Buf h(hist ? a.snap + (long long)(L - 2) * 2 * n2 : a.snap + (long long)a.k0 * 4 * n2, (hist && next ? 6 : 4) * fs);
 #pragma unroll
     for (int i = 0; i < CX; ++i) {
 #pragma unroll

@@ -91,13 +91,25 @@ enum : int {
                 // level imaged is K T(L) for L >= 3, T(2), R(1)
 };
 
+// Flag of every step launch: the tiles (and the columns of a marching strip)
+// in the opposite order. Levels alternate, so that a launch begins with the
+// cells the one before it ended with, which are still in the 256 MB memory-side
+// cache; in one direction a working set beyond it is evicted before it is read
+// again.
+enum : int { STEP_REV = 1 << 14 };
+
 // Workgroups are dispatched round-robin over the 8 XCDs; renumber them so
 // each XCD receives a contiguous range of tiles (shot-major, column-major),
 // which keeps neighbouring tiles -- and their shared halos -- in one L2.
-__device__ __forceinline__ int xcd_tile(int L, int N) {
+__device__ __forceinline__ int xcd_tile(int L, int N, bool rev = false) {
   const int q = N >> 3, r = N & 7;
-  const int x = L & 7, pos = L >> 3;
+  const int x = L & 7, n = x < r ? q + 1 : q;
+  const int pos = rev ? n - 1 - (L >> 3) : L >> 3;
   return (x < r) ? x * (q + 1) + pos : r * (q + 1) + (x - r) * q + pos;
+}
+// The tile (or strip) of workgroup L of N.
+__device__ __forceinline__ int step_tile(int L, int N, int xcd, bool rev) {
+  return xcd ? xcd_tile(L, N, rev) : rev ? N - 1 - L : L;
 }
 
 // Tile geometry: 64 z-cells (one wave64 along the fast axis) by 4*TXR
@@ -144,6 +156,8 @@ int launch_fwd_pair(const ShotDev& s, int tile, int L, int flags, float amp0, fl
 int launch_adj_pair(const ShotDev& s, int tile, int L, int flags, int xcd, hipStream_t st);
 // Compute units of the current device (0 if unknown).
 int device_cus();
+// The marching forms read the five fields of a level through one buffer.
+inline bool march_addressable(long long n2) { return 20 * n2 < (1LL << 31); }
 // Marching forms: one workgroup of nw waves (nw in {1, 2, 4}) per strip of
 // 64*nw rows x xw columns (xw even; strip tables start strips on even
 // columns and rows on multiples of 64*nw). Bitwise the same results as

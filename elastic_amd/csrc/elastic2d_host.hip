@@ -203,11 +203,11 @@ static int op3(int nt, int nz, int nx, const float* const* in, float* const* out
   d.nz = nz; d.nx = nx; d.ldz = ldz; d.nt = nt; d.n2 = n2;
   d.lev = hp; d.lev_stride = n2; d.fstride = (long long)nt * n2; d.lev_mod = nt; d.lev_off = 0;
   d.coef = cf.as<float>();
-  const int width = single_shot_txr(SNAP_HIST);
-  const int txr = tile_code(width, default_tblock() == 2 ? 2 : 0, SNAP_HIST);
   // kernel form 2 (RTM_TBLOCK=2): strips of RTM_MARCH_W columns marching
   // along x (form 3 marches the forward only: tiles here)
-  const bool march = default_tblock() == 2;
+  const bool march = default_tblock() == 2 && march_addressable(n2);
+  const int width = single_shot_txr(SNAP_HIST);
+  const int txr = tile_code(width, march ? 2 : 0, SNAP_HIST);
   const int mw = default_march_w(), mnw = default_march_nw();
   if (!march && width != 1 && width != 2 && width != 4 && width != 8) {
     set_error("unsupported tile width %d", width);

@@ -11,6 +11,13 @@
 // cell-update: 5 fields read at level L-1, 5 at L-2, 5 written, 5
 // coefficients).
 //
+// Steps of a working set beyond the 256 MB memory-side cache run their tiles in
+// alternating order (STEP_REV) over a ring of two levels, the new level in place
+// of the one before the last: us a level, forward / adjoint, 7 shots of 890 x
+// 690..1290 139 / 200 -> 124 / 181 with the order
+// -> 116 / 172 with the ring of two as well; 14 of them with bfloat16 snapshots
+// 226 / 237 (levels not imaged) -> 200 / 220.
+//
 // The reference operators (W/rtmlib-mod.f90:200-633) all reduce to two
 // staggered differences along either axis:
 //   S+ f(i) = sum_k c_k (f[i+6-k] - f[i-5+k])   (D, E, F, G, Az, Bx)
@@ -20,6 +27,7 @@
 // coefficient-weighted products, which the adjoint kernel forms while it
 // stages the halo.
 
+#include "buffer.hpp"
 #include "elastic2d_device.hpp"
 
 namespace erm {
@@ -66,13 +74,19 @@ struct SnapQ {
   __device__ static float dec(unsigned short h) { return SNAP == SNAP_F16 ? dq_f16(h) : dq_bf16(h); }
 };
 
+// Fields are accessed as raw buffers (buffer.hpp): the adjoint tile of width 1
+// takes 68 registers instead of 78 and 461 vector instructions instead of 530
+// (12 shots of 200 x 400: 45.6 -> 42.9 us a level), that of width 2 4 waves a
+// SIMD instead of 3 (52 -> 44 us). The marching kernels, which memory bounds,
+// have a third to a half fewer vector instructions and the same times.
+
 // The tile of this workgroup. A launch over one shot (nbz: its tiles along z)
 // works it out from the workgroup's number, which is one dependent memory
 // latency less than the table's entry (about 0.5 us of a 5 us launch on small
 // grids); several shots share a table.
 template <int TX>
-__device__ __forceinline__ TileRef tile_of(const TileRef* tiles, int ntiles, int xcd, int nbz) {
-  const int b = xcd ? xcd_tile(blockIdx.x, ntiles) : (int)blockIdx.x;
+__device__ __forceinline__ TileRef tile_of(const TileRef* tiles, int ntiles, int xcd, int nbz, int flags) {
+  const int b = step_tile(blockIdx.x, ntiles, xcd, flags & STEP_REV);
   if (nbz == 0) return tiles[b];
   const int bx = b / nbz;
   return TileRef{0, (b - bx * nbz) * TILE_Z, bx * TX, b};
@@ -103,7 +117,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
   constexpr int NIT = (T::N + T::NT - 1) / T::NT;  // staged cells per thread
   static_assert(!BORN || SNAP == SNAP_HIST, "Born sources come from the fp32 history");
   __shared__ float sh[BORN ? 7 : 5][T::N];
-  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz);
+  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz, flags);
   const ShotDev& S = shots[tr.shot];
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   // offsets inside one field are 32-bit (5 * n2 < 2^31, checked by the
@@ -118,6 +132,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
   const int tz = threadIdx.x, ty = threadIdx.y;
   const int tid = tz + T::TZ * ty;
 
+  auto field = [&](const float* p) { return Buf(p, 4u * (unsigned)n2); };
   // Every global load of this thread is issued before the first LDS store or
   // barrier: the staged tile of level L-1 (flat over tile + halo so all
   // lanes stay busy) and the own-cell operands (level L-2, coefficients).
@@ -128,9 +143,9 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
     const int lx = c / T::LZ, lz = c - lx * T::LZ;
     const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
     const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
-    const int gi = gz + ldz * gx;
+    const unsigned o = in ? 4u * (unsigned)(gz + ldz * gx) : kOutside;
 #pragma unroll
-    for (int f = 0; f < 5; ++f) st[k][f] = gldm(y1 + f * fs, gi, in);
+    for (int f = 0; f < 5; ++f) st[k][f] = field(y1 + f * fs).get(o);
   }
   // Born: the background Vx, Vz of level L over the tile and its halo, of the
   // next level at the own cells, and the model perturbation
@@ -144,9 +159,9 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
       const int lx = c / T::LZ, lz = c - lx * T::LZ;
       const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
       const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
-      const int gi = gz + ldz * gx;
-      bs[k][0] = gldm(bg, gi, in);
-      bs[k][1] = gldm(bg + n2, gi, in);
+      const unsigned o = in ? 4u * (unsigned)(gz + ldz * gx) : kOutside;
+      bs[k][0] = field(bg).get(o);
+      bs[k][1] = field(bg + n2).get(o);
     }
   }
   const int gz = z0 + tz;
@@ -162,18 +177,18 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
   for (int j = 0; j < TXR; ++j) {
     const int gx = x0 + ty * TXR + j;
     const bool ok = zok && gx < nx;
-    const int gi = gz + ldz * gx;
+    const unsigned o = ok ? 4u * (unsigned)(gz + ldz * gx) : kOutside;
     kx[j] = sponge ? gldu(S.kx, __builtin_amdgcn_readfirstlane(min(gx, nx - 1))) : 1.f;
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
-      ox[j][f] = gld(x2 + f * fs, ok ? gi : 0);
-      oc[j][f] = gld(coef + f * n2, ok ? gi : 0);
+      ox[j][f] = field(x2 + f * fs).get(o);
+      oc[j][f] = field(coef + f * n2).get(o);
     }
     if (BORN) {
 #pragma unroll
-      for (int a = 0; a < 2; ++a) bn[j][a] = gld(bg + (bnext ? 2 + a : a) * n2, ok ? gi : 0);
+      for (int a = 0; a < 2; ++a) bn[j][a] = field(bg + (bnext ? 2 + a : a) * n2).get(o);
 #pragma unroll
-      for (int a = 0; a < 3; ++a) bd[j][a] = gld(S.dm + a * n2, ok ? gi : 0);
+      for (int a = 0; a < 3; ++a) bd[j][a] = field(S.dm + a * n2).get(o);
     }
   }
 #pragma unroll
@@ -245,7 +260,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
       for (int f = 0; f < 5; ++f) gst_nt(out + f * fs, gi, v[f]);
     } else {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) gst(out + f * fs, gi, v[f]);
+      for (int f = 0; f < 5; ++f) field(out + f * fs).put(4u * (unsigned)gi, 0, v[f]);
     }
     if ((flags & (F_REC | F_RECSUB)) && gz == S.zr && gx >= S.rx0 && gx < S.rx0 + S.nrx) {
       float* r = S.rec + (long long)(L - 1) * S.nrx + (gx - S.rx0);
@@ -260,8 +275,8 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_fwd(const ShotDev* __restrict__
     }
     if (SNAP == SNAP_HIST && (flags & F_SNAP)) {
       float* h = static_cast<float*>(S.snap) + (long long)(L - 1) * 2 * (long long)n2;
-      gst(h, gi, v[0]);
-      gst(h + n2, gi, v[1]);
+      field(h).put(4u * (unsigned)gi, 0, v[0]);
+      field(h + n2).put(4u * (unsigned)gi, 0, v[1]);
     }
     if (SNAP != SNAP_HIST) {
       sv[0][j] = sh[0][p];
@@ -697,34 +712,6 @@ struct SrcView {
     const int strip = (gz >> 6) + nbz * (gx >> sw);
     return SnapQ<SNAP>::dec(q[a][gi]) * sc[a][strip];
   }
-  // an element as loaded (clamped index), decoded and masked by value():
-  // loads and their use can be a column apart
-  struct Raw {
-    float v;
-    unsigned short h;
-    bool in;
-  };
-  __device__ __forceinline__ void load(int a, int gi, int gz, int gx, bool in, Raw& r) const {
-    r.in = in;
-    if (SNAP == SNAP_HIST || SNAP == SNAP_F32) {
-      r.v = gld(f[a], in ? gi : 0);
-    } else {
-      r.h = gld(q[a], in ? gi : 0);
-      r.v = gld(sc[a], in ? (gz >> 6) + nbz * (gx >> sw) : 0);
-    }
-  }
-  __device__ __forceinline__ float value(const Raw& r) const {
-    if (SNAP == SNAP_HIST || SNAP == SNAP_F32) return r.in ? r.v : 0.f;
-    return r.in ? SnapQ<SNAP>::dec(r.h) * r.v : 0.f;
-  }
-  // The element alone (16-bit formats: the scale comes from scale_u).
-  __device__ __forceinline__ void load_q(int a, int gi, bool in, Raw& r) const {
-    r.in = in;
-    if (SNAP == SNAP_HIST || SNAP == SNAP_F32)
-      r.v = gld(f[a], in ? gi : 0);
-    else
-      r.h = gld(q[a], in ? gi : 0);
-  }
   // 16-bit formats: the scale of the strip of 64-row block zb and column gx,
   // read through the constant address space, so that a wave-uniform block and
   // column make it one scalar load into a scalar register.
@@ -732,11 +719,7 @@ struct SrcView {
     if (SNAP == SNAP_HIST || SNAP == SNAP_F32) return 1.f;
     return ((const __attribute__((address_space(4))) float*)sc[a])[zb + nbz * (gx >> sw)];
   }
-  __device__ __forceinline__ float value_s(const Raw& r, float s) const {
-    if (SNAP == SNAP_HIST || SNAP == SNAP_F32) return r.in ? r.v : 0.f;
-    return r.in ? SnapQ<SNAP>::dec(r.h) * s : 0.f;
-  }
-  // the same as a branch-free global load, zero where !in
+  // array a at an element by a branch-free global load, zero where !in
   __device__ __forceinline__ float getm(int a, int gi, int gz, int gx, bool in) const {
     if (SNAP == SNAP_HIST || SNAP == SNAP_F32) return gldm(f[a], gi, in);
     const int strip = in ? (gz >> 6) + nbz * (gx >> sw) : 0;
@@ -769,7 +752,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
   constexpr bool kEarly = SNAP == SNAP_HIST || SNAP == SNAP_F32;
   constexpr bool kSmall = kEarly && WY != TILE_WY;
   __shared__ float sh[kSmall ? 7 : 5][T::N];
-  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz);
+  const TileRef tr = tile_of<T::TX>(tiles, ntiles, xcd, nbz, flags);
   const ShotDev& S = shots[tr.shot];
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   const long long fs = S.fstride;
@@ -782,6 +765,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
   const int tz = threadIdx.x, ty = threadIdx.y;
   const int tid = tz + T::TZ * ty;
 
+  auto field = [&](const float* p) { return Buf(p, 4u * (unsigned)n2); };
   // Staged tile: coefficient-weighted products of level L+1 (flat over tile +
   // halo); own-cell operands are loaded before the barrier as well.
   float st[NIT][5];
@@ -791,24 +775,12 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
     const int lx = c / T::LZ, lz = c - lx * T::LZ;
     const int gx = x0 - T::H + lx, gz = z0 - T::H + lz;
     const bool in = c < T::N && gx >= 0 && gx < nx && gz >= 0 && gz < nz;
-    // With the fp32 history out-of-range cells issue no loads; with
-    // decimated snapshots the loads are branch-free (clamped index, masked
-    // products). Each form measured faster for its format with four waves; in
-    // the first form a cell's loads end before the next cell's begin, so the
-    // eight-wave tile takes the second one.
-    float p0 = 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f, p4 = 0.f;
-    if (SNAP != SNAP_HIST || kSmall || in) {
-      const int gi = in ? gz + ldz * gx : 0;
-      const float vx = gld(y1, gi), vz = gld(y1 + fs, gi), xx = gld(y1 + 2 * fs, gi), zz = gld(y1 + 3 * fs, gi),
-                  xz = gld(y1 + 4 * fs, gi);
-      const float m1x = gld(coef, gi), m1z = gld(coef + n2, gi), m2 = gld(coef + 2 * n2, gi),
-                  m3 = gld(coef + 3 * n2, gi), m2m3 = gld(coef + 4 * n2, gi);
-      p0 = in ? fmaf(m2m3, xx, m2 * zz) : 0.f;
-      p1 = in ? fmaf(m2, xx, m2m3 * zz) : 0.f;
-      p2 = in ? m3 * xz : 0.f;
-      p3 = in ? m1x * vx : 0.f;
-      p4 = in ? m1z * vz : 0.f;
-    }
+    const unsigned o = in ? 4u * (unsigned)(gz + ldz * gx) : kOutside;  // products outside are zero
+    const float vx = field(y1).get(o), vz = field(y1 + fs).get(o), xx = field(y1 + 2 * fs).get(o),
+                zz = field(y1 + 3 * fs).get(o), xz = field(y1 + 4 * fs).get(o);
+    const float m1x = field(coef).get(o), m1z = field(coef + n2).get(o), m2 = field(coef + 2 * n2).get(o),
+                m3 = field(coef + 3 * n2).get(o), m2m3 = field(coef + 4 * n2).get(o);
+    const float p0 = fmaf(m2m3, xx, m2 * zz), p1 = fmaf(m2, xx, m2m3 * zz), p2 = m3 * xz, p3 = m1x * vx, p4 = m1z * vz;
     st[k][0] = p0;
     st[k][1] = p1;
     st[k][2] = p2;
@@ -826,15 +798,15 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
   for (int j = 0; j < TXR; ++j) {
     const int gx = x0 + ty * TXR + j;
     const bool ok = zok && gx < nx;
-    const int gi = gz + ldz * gx;
+    const unsigned o = ok ? 4u * (unsigned)(gz + ldz * gx) : kOutside;
 #pragma unroll
-    for (int f = 0; f < 5; ++f) b[j][f] = gld(x2 + f * fs, ok ? gi : 0);  // used where ok only
+    for (int f = 0; f < 5; ++f) b[j][f] = field(x2 + f * fs).get(o);
     kx[j] = sponge ? gldu(S.kx, __builtin_amdgcn_readfirstlane(min(gx, nx - 1))) : 1.f;
     // the level's own content (drop-in form) or the receiver row, added after
     // the barrier: nothing waits for it here
     if (flags & A_XIN) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) inj[j][f] = gld(out + f * fs, ok ? gi : 0);
+      for (int f = 0; f < 5; ++f) inj[j][f] = field(out + f * fs).get(o);
     } else if (tile_row) {
       const bool in = row && gx >= S.rx0 && gx < S.rx0 + S.nrx;
       const float* r = S.rec + (long long)(L - 1) * S.nrx + (in ? gx - S.rx0 : 0);
@@ -860,8 +832,9 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
       const int gx = x0 - T::H + lx, gz2 = z0 - T::H + lz;
       const bool in = c < T::N && gx >= 0 && gx < nx && gz2 >= 0 && gz2 < nz;
       const int gi = gz2 + ldz * gx;
-      sx[k][0] = sv.getm(0, gi, gz2, gx, in);
-      sx[k][1] = sv.getm(1, gi, gz2, gx, in);
+      const unsigned o = in ? 4u * (unsigned)gi : kOutside;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) sx[k][a] = kEarly ? field(sv.f[a]).get(o) : sv.getm(a, gi, gz2, gx, in);
     }
     const bool next = flags & A_NEXT;
 #pragma unroll
@@ -869,12 +842,14 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
       const int gx = x0 + ty * TXR + j;
       const bool ok = zok && gx < nx;
       const int gi = gz + ldz * gx;
-      nt2[j][0] = next ? sv.getm(2, gi, gz, gx, ok) : 0.f;  // arrays 2, 3 exist below the last level only
-      nt2[j][1] = next ? sv.getm(3, gi, gz, gx, ok) : 0.f;
+      const unsigned o = ok ? 4u * (unsigned)gi : kOutside;
+#pragma unroll
+      for (int a = 0; a < 2; ++a)  // arrays 2, 3 exist below the last level only
+        nt2[j][a] = !next ? 0.f : kEarly ? field(sv.f[2 + a]).get(o) : sv.getm(2 + a, gi, gz, gx, ok);
 #pragma unroll
       for (int a = 0; a < 3; ++a) {  // used where ok only
-        im[j][a] = gld(S.img + a * n2, ok ? gi : 0);
-        imc[j][a] = (flags & A_COMP) ? gld(S.imgc + a * n2, ok ? gi : 0) : 0.f;
+        im[j][a] = field(S.img + a * n2).get(o);
+        imc[j][a] = (flags & A_COMP) ? field(S.imgc + a * n2).get(o) : 0.f;
       }
     }
   };
@@ -933,7 +908,7 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
       for (int f = 0; f < 5; ++f) gst_nt(out + f * fs, gi, v[f]);
     } else {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) gst(out + f * fs, gi, v[f]);
+      for (int f = 0; f < 5; ++f) field(out + f * fs).put(4u * (unsigned)gi, 0, v[f]);
     }
 #pragma unroll
     for (int f = 0; f < 5; ++f) o[j][f] = ksrc && L >= 3 ? (v[f] * kz) * kx[j] : v[f];
@@ -1000,12 +975,12 @@ __global__ __launch_bounds__(TILE_Z * WY) void k_adj(const ShotDev* __restrict__
       for (int a = 0; a < 3; ++a) {
         float sa = im[j][a], ca = imc[j][a];
         neumaier(sa, ca, t[a]);
-        gst(img + a * n2, gi, sa);
-        gst(imgc + a * n2, gi, ca);
+        field(img + a * n2).put(4u * (unsigned)gi, 0, sa);
+        field(imgc + a * n2).put(4u * (unsigned)gi, 0, ca);
       }
     } else {
 #pragma unroll
-      for (int a = 0; a < 3; ++a) gst(img + a * n2, gi, im[j][a] + t[a]);
+      for (int a = 0; a < 3; ++a) field(img + a * n2).put(4u * (unsigned)gi, 0, im[j][a] + t[a]);
     }
   }
 }
@@ -1497,15 +1472,17 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   const long long fs = S.fstride;
   const int n2 = (int)S.n2;
-  float* const out = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L);
-  const float* const x2 = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L - 2);
-  const float* const y1 = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L - 1);
-  const float* const coef = S.coef;
-  const float* const bsrc = S.bsrc;
+  float* const outp = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L);
+  const Fields<false> out(outp, fs, n2), x2(lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L - 2), fs, n2),
+      y1(lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L - 1), fs, n2), coef(S.coef, n2, n2), bsrc(S.bsrc, n2, n2);
   const int z0 = tr.z0, xb = tr.x0, xe = min(tr.x0 + xw, nx);
   const int ncol = xe - xb, xs = DIR > 0 ? xb : xe - 1;  // columns, first column of the march
   const MarchLane<NW> m(z0, nz);
   const int gz = m.gz;
+  // byte offsets: own row and halo row (kOutside where there is none), and a
+  // column (outside unless ok, which is wave-uniform)
+  const unsigned zo = m.zok ? 4u * (unsigned)gz : kOutside, ho = m.hok ? 4u * (unsigned)m.hz : kOutside;
+  auto xo = [&](int gx, bool ok) { return ok ? 4u * (unsigned)(ldz * gx) : kOutside; };
   const bool born = BORN;  // Born sources (F_BORN) in their own instance: 10 fewer live registers
 
   // queues: sigma_xx (S-x), sigma_xz (S+x), Vx (S+x), Vz (S-x). The
@@ -1517,11 +1494,11 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
   for (int i = 0; i < 11; ++i) {
     const int k = DIR > 0 ? i : 10 - i;
     const int gx = xs + DIR * (k - 5);
-    const bool in = m.zok && gx >= 0 && gx < nx;
-    qa[k] = gldm(y1 + 2 * fs, gz + ldz * gx, in);
-    qb[k] = gldm(y1 + 4 * fs, gz + ldz * gx, in);
-    qc[k] = gldm(y1, gz + ldz * gx, in);
-    qd[k] = gldm(y1 + fs, gz + ldz * gx, in);
+    const unsigned o = add_sat(zo, xo(gx, gx >= 0 && gx < nx));
+    qa[k] = y1.get(2, o);
+    qb[k] = y1.get(4, o);
+    qc[k] = y1.get(0, o);
+    qd[k] = y1.get(1, o);
     // Halo rows of sigma_xz, Vx, Vz: lanes 0..9 of the first wave load their
     // halo row of a column when the column enters the queues, the step at
     // which the strips above and below load those rows as their own (so the
@@ -1530,35 +1507,31 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
     // the lane that writes an entry reads it. sigma_zz is not queued: its
     // halo rows come with the centre column's own loads.
     if (k >= 5 && m.lane < 10) {
-      const bool hin = m.hok && k - 5 < ncol;
-      const int ih = m.hz + ldz * gx;
-      hring[k - 5][0][m.lane] = gldm(y1 + 4 * fs, ih, hin);
-      hring[k - 5][1][m.lane] = gldm(y1, ih, hin);
-      hring[k - 5][2][m.lane] = gldm(y1 + fs, ih, hin);
+      const unsigned oh = add_sat(ho, xo(gx, k - 5 < ncol));
+      hring[k - 5][0][m.lane] = y1.get(4, oh);
+      hring[k - 5][1][m.lane] = y1.get(0, oh);
+      hring[k - 5][2][m.lane] = y1.get(1, oh);
     }
   }
   // Operands of a column: centre sigma_zz, halo rows of the LDS fields, own
-  // cell level L-2 (+ Born sources) and coefficients. Loads are issued with
-  // clamped indices and masked where the values are taken, so that nothing
-  // waits for them before the next column.
+  // cell level L-2 (+ Born sources) and coefficients; nothing waits for them
+  // before the next column.
   struct Col {
     float zz, h, o[5], c[5], bs[5];
   };
   auto load_col = [&](int gx, bool more, Col& v) {
-    const int ic = m.zok && more ? gz + ldz * gx : 0;
-    const int ih = m.hok && more ? m.hz + ldz * gx : 0;
-    v.zz = gld(y1 + 3 * fs, ic);
-    v.h = gld(y1 + 3 * fs, ih);
+    const unsigned x = xo(gx, more), o = add_sat(zo, x);
+    v.zz = y1.get(3, o);
+    v.h = y1.get(3, add_sat(ho, x));
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
-      v.o[f] = gld(x2 + f * fs, ic);
-      v.c[f] = gld(coef + f * n2, ic);
-      v.bs[f] = born ? gld(bsrc + f * n2, ic) : 0.f;
+      v.o[f] = x2.get(f, o);
+      v.c[f] = coef.get(f, o);
+      v.bs[f] = born ? bsrc.get(f, o) : 0.f;
     }
   };
   Col cur;
   load_col(xs, true, cur);
-  bool cur_h = m.hok;  // halo values of the current column are valid
   const float kz = ((flags & F_K) && m.zok) ? gld(S.kz, gz) : 1.f;
   float svp[4] = {0.f, 0.f, 0.f, 0.f};  // previous column's snapshot values (16-bit formats)
 
@@ -1566,23 +1539,21 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
     const int x = xs + DIR * st;
     const bool more = st + 1 < ncol;
     const int xq = x + 6 * DIR;  // column entering the queues
-    const bool qok = m.zok && more && xq >= 0 && xq < nx;
-    const int iq = qok ? gz + ldz * xq : 0;
-    const float na = gld(y1 + 2 * fs, iq), nb = gld(y1 + 4 * fs, iq), nc = gld(y1, iq), nd = gld(y1 + fs, iq);
+    const unsigned oq = add_sat(zo, xo(xq, more && xq >= 0 && xq < nx));
+    const float na = y1.get(2, oq), nb = y1.get(4, oq), nc = y1.get(0, oq), nd = y1.get(1, oq);
     // halo rows of the column entering the queues (centre at step st + 6)
-    const bool hq = m.hok && st + 6 < ncol;
-    const int ihq = hq ? m.hz + ldz * xq : 0;
-    const float hb = gld(y1 + 4 * fs, ihq), hc = gld(y1, ihq), hd = gld(y1 + fs, ihq);
+    const unsigned ohq = add_sat(ho, xo(xq, st + 6 < ncol));
+    const float hb = y1.get(4, ohq), hc = y1.get(0, ohq), hd = y1.get(1, ohq);
     Col nxt;
     load_col(x + DIR, more, nxt);
 
     const int b = st & 1;
-    col[b][0][m.lane + 5] = m.zok ? cur.zz : 0.f;
+    col[b][0][m.lane + 5] = cur.zz;
     col[b][1][m.lane + 5] = qb[5];
     col[b][2][m.lane + 5] = qc[5];
     col[b][3][m.lane + 5] = qd[5];
     if (m.lane < 10) {
-      col[b][0][m.hs] = cur_h ? cur.h : 0.f;
+      col[b][0][m.hs] = cur.h;
 #pragma unroll
       for (int f = 0; f < 3; ++f) col[b][f + 1][m.hs] = hring[st % 7][f][m.lane];
     }
@@ -1627,10 +1598,10 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
       }
       if (flags & F_NTS) {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) gst_nt(out + f * fs, gi, v[f]);
+        for (int f = 0; f < 5; ++f) gst_nt(outp + f * fs, gi, v[f]);
       } else {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) gst(out + f * fs, gi, v[f]);
+        for (int f = 0; f < 5; ++f) out.put(f, 4u * (unsigned)gi, v[f]);
       }
       if ((flags & (F_REC | F_RECSUB)) && gz == S.zr && gx >= S.rx0 && gx < S.rx0 + S.nrx) {
         float* r = S.rec + (long long)(L - 1) * S.nrx + (gx - S.rx0);
@@ -1645,8 +1616,9 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
       }
       if (SNAP == SNAP_HIST && (flags & F_SNAP)) {
         float* h = static_cast<float*>(S.snap) + (long long)(L - 1) * 2 * (long long)n2;
-        gst(h, gi, v[0]);
-        gst(h + n2, gi, v[1]);
+        const Buf hb(h, 8u * (unsigned)n2);
+        hb.put(4u * (unsigned)gi, 0, v[0]);
+        hb.put(4u * (unsigned)gi, 4u * (unsigned)n2, v[1]);
       }
       if (SNAP != SNAP_HIST) {
         sv[0] = qc[5];
@@ -1690,18 +1662,17 @@ __device__ __forceinline__ void fwdm_strip(const ShotDev& S, const TileRef& tr, 
 #pragma unroll
       for (int a = 0; a < 4; ++a) svp[a] = sv[a];
     }
-    push(qa, qok ? na : 0.f);
-    push(qb, qok ? nb : 0.f);
-    push(qc, qok ? nc : 0.f);
-    push(qd, qok ? nd : 0.f);
+    push(qa, na);
+    push(qb, nb);
+    push(qc, nc);
+    push(qd, nd);
     if (m.lane < 10) {
       float* r = &hring[(st + 6) % 7][0][m.lane];
-      r[0] = hq ? hb : 0.f;
-      r[10] = hq ? hc : 0.f;
-      r[20] = hq ? hd : 0.f;
+      r[0] = hb;
+      r[10] = hc;
+      r[20] = hd;
     }
     cur = nxt;
-    cur_h = m.hok && more;
   }
 }
 
@@ -1712,11 +1683,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     int xcd) {
   __shared__ float col[2][4][MarchCol<NW>::MZ];  // sigma_zz, sigma_xz, Vx, Vz of the centre column
   __shared__ float hring[7][3][10];              // sigma_xz, Vx, Vz of the halo rows of the next six columns
-  const TileRef tr = strips[xcd ? xcd_tile(blockIdx.x, nstrips) : (int)blockIdx.x];
+  const TileRef tr = strips[step_tile(blockIdx.x, nstrips, xcd, flags & STEP_REV)];
   // neighbouring strips march in opposite directions, so the columns they
   // share (a strip's priming columns) are read by both at the same end of
   // their marches, close in time, and come from L2 for the second
-  if (((tr.x0 / xw) & 1) == 0)
+  if (((tr.x0 / xw) & 1) == ((flags & STEP_REV) ? 1 : 0))
     fwdm_strip<SNAP, BORN, 1, NW>(shots[tr.shot], tr, L, flags, xw, col, hring);
   else
     fwdm_strip<SNAP, BORN, -1, NW>(shots[tr.shot], tr, L, flags, xw, col, hring);
@@ -1735,21 +1706,40 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
   const int nz = S.nz, nx = S.nx, ldz = S.ldz;
   const long long fs = S.fstride;
   const int n2 = (int)S.n2;
-  float* const out = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L);
-  const float* const x2 = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L + 2);
-  const float* const y1 = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L + 1);
-  const float* const coef = S.coef;
+  float* const outp = lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L);
+  const Fields<XIN> out(outp, fs, n2), x2(lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L + 2), fs, n2),
+      y1(lev_ptr(S.lev, S.lev_stride, S.lev_mod, S.lev_off, L + 1), fs, n2);
+  const Fields<false> coef(S.coef, n2, n2);
   const int z0 = tr.z0, xb = tr.x0, xe = min(tr.x0 + xw, nx);
   const int ncol = xe - xb, xs = DIR > 0 ? xb : xe - 1;  // columns, first column of the march
   const MarchLane<NW> m(z0, nz);
   const int gz = m.gz;
+  const unsigned zo = m.zok ? 4u * (unsigned)gz : kOutside, ho = m.hok ? 4u * (unsigned)m.hz : kOutside;
+  auto xo = [&](int gx, bool ok) { return ok ? 4u * (unsigned)(ldz * gx) : kOutside; };
   // the drop-in form has no imaging, injection or sponge; PROP: the
   // instance for levels that are not imaged (no imaging code or registers)
   const bool imaging = !XIN && !PROP && (flags & A_IMG);
   const bool next = flags & A_NEXT;
   constexpr bool comp = !XIN && COMP;  // compensated image sums (A_COMP), an instance of its own
   constexpr bool xin = XIN;
+  // source arrays 0 to 3 (see SrcView), back to back, as stored; at the last
+  // level of the history arrays 2, 3 lie past the buffer
+  constexpr bool f32 = SNAP == SNAP_HIST || SNAP == SNAP_F32;
   const SrcView<SNAP> sv(S, L);
+  const Buf src(f32 ? (const void*)sv.f[0] : (const void*)sv.q[0],
+                (f32 ? 4u : 2u) * (unsigned)n2 * (SNAP == SNAP_HIST && !next ? 2u : 4u));
+  struct Src {
+    float v;
+    unsigned short h;
+  };
+  auto load_src = [&](int a, unsigned o, Src& r) {
+    if (f32)
+      r.v = src.get(o, a * 4u * (unsigned)n2);
+    else
+      r.h = src.get16(o / 2, a * 2u * (unsigned)n2);
+  };
+  auto value = [&](const Src& r, float scale) { return f32 ? r.v : SnapQ<SNAP>::dec(r.h) * scale; };
+  const Buf img(S.img, 12u * (unsigned)n2), imgc(S.imgc, comp ? 12u * (unsigned)n2 : 0);
   // 64-row blocks of the 16-bit snapshot scales: the wave's own rows (clamped
   // for a wave wholly below the grid) and the halo rows above and below the
   // strip; all wave-uniform, so their scales are scalar loads
@@ -1757,21 +1747,21 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
   const int zbt = max((z0 >> 6) - 1, 0), zbb = min((z0 >> 6) + NW, S.snap_nbz - 1);
   auto cx = [&](int gx) { return min(max(gx, 0), nx - 1); };
 
-  // the ten level-(L+1) operands at element i (clamped index), as loaded
+  // the ten level-(L+1) operands at offset o, as loaded (zero outside)
   struct Raw {
     float vx, vz, xx, zz, xz, m1x, m1z, m2, m3, m2m3;
   };
-  auto raw = [&](int i, Raw& w) {
-    w.vx = gld(y1, i);
-    w.vz = gld(y1 + fs, i);
-    w.xx = gld(y1 + 2 * fs, i);
-    w.zz = gld(y1 + 3 * fs, i);
-    w.xz = gld(y1 + 4 * fs, i);
-    w.m1x = gld(coef, i);
-    w.m1z = gld(coef + n2, i);
-    w.m2 = gld(coef + 2 * n2, i);
-    w.m3 = gld(coef + 3 * n2, i);
-    w.m2m3 = gld(coef + 4 * n2, i);
+  auto raw = [&](unsigned o, Raw& w) {
+    w.vx = y1.get(0, o);
+    w.vz = y1.get(1, o);
+    w.xx = y1.get(2, o);
+    w.zz = y1.get(3, o);
+    w.xz = y1.get(4, o);
+    w.m1x = coef.get(0, o);
+    w.m1z = coef.get(1, o);
+    w.m2 = coef.get(2, o);
+    w.m3 = coef.get(3, o);
+    w.m2m3 = coef.get(4, o);
   };
 
   // Halo rows: lanes 0..9 of the first wave load their halo row of a column
@@ -1782,31 +1772,31 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
   // later. Only the lane that writes an entry reads it.
   struct Halo {
     Raw w;
-    typename SrcView<SNAP>::Raw s[2];
+    Src s[2];
     float sc[2][2];  // 16-bit scales of the source values: above, below
   };
   auto load_halo = [&](int gx, bool in, Halo& h) {
-    const int ih = in ? m.hz + ldz * gx : 0;
-    raw(ih, h.w);
+    const unsigned o = add_sat(ho, xo(gx, in));
+    raw(o, h.w);
     if (imaging) {
 #pragma unroll
       for (int a = 0; a < 2; ++a) {
-        sv.load_q(a, ih, in, h.s[a]);
+        load_src(a, o, h.s[a]);
         h.sc[a][0] = sv.scale_u(a, zbt, cx(gx));
         h.sc[a][1] = sv.scale_u(a, zbb, cx(gx));
       }
     }
   };
-  auto put_halo = [&](int slot, bool in, const Halo& h) {
+  auto put_halo = [&](int slot, const Halo& h) {
     if (m.lane < 10) {
       float* r = &hring[slot][0][m.lane];
-      r[0] = in ? fmaf(h.w.m2, h.w.xx, h.w.m2m3 * h.w.zz) : 0.f;
-      r[10] = in ? h.w.m3 * h.w.xz : 0.f;
-      r[20] = in ? h.w.m1x * h.w.vx : 0.f;
-      r[30] = in ? h.w.m1z * h.w.vz : 0.f;
+      r[0] = fmaf(h.w.m2, h.w.xx, h.w.m2m3 * h.w.zz);
+      r[10] = h.w.m3 * h.w.xz;
+      r[20] = h.w.m1x * h.w.vx;
+      r[30] = h.w.m1z * h.w.vz;
       if (imaging) {
-        r[40] = sv.value_s(h.s[0], m.lane < 5 ? h.sc[0][0] : h.sc[0][1]);
-        r[50] = sv.value_s(h.s[1], m.lane < 5 ? h.sc[1][0] : h.sc[1][1]);
+        r[40] = value(h.s[0], m.lane < 5 ? h.sc[0][0] : h.sc[0][1]);
+        r[50] = value(h.s[1], m.lane < 5 ? h.sc[1][0] : h.sc[1][1]);
       }
     }
   };
@@ -1819,64 +1809,61 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
   for (int i = 0; i < 11; ++i) {
     const int k = DIR > 0 ? i : 10 - i;
     const int gx = xs + DIR * (k - 5);
-    const bool in = m.zok && gx >= 0 && gx < nx;
+    const unsigned o = add_sat(zo, xo(gx, gx >= 0 && gx < nx));
     Raw w;
-    raw(in ? gz + ldz * gx : 0, w);
-    q0[k] = in ? fmaf(w.m2m3, w.xx, w.m2 * w.zz) : 0.f;
-    q2[k] = in ? w.m3 * w.xz : 0.f;
-    q3[k] = in ? w.m1x * w.vx : 0.f;
-    q4[k] = in ? w.m1z * w.vz : 0.f;
-    if (k >= 5) d1[k - 5] = in ? fmaf(w.m2, w.xx, w.m2m3 * w.zz) : 0.f;
+    raw(o, w);
+    q0[k] = fmaf(w.m2m3, w.xx, w.m2 * w.zz);
+    q2[k] = w.m3 * w.xz;
+    q3[k] = w.m1x * w.vx;
+    q4[k] = w.m1z * w.vz;
+    if (k >= 5) d1[k - 5] = fmaf(w.m2, w.xx, w.m2m3 * w.zz);
     if (imaging) {
-      s0q[k] = sv.getm(0, gz + ldz * gx, gz, gx, in);
-      s1q[k] = sv.getm(1, gz + ldz * gx, gz, gx, in);
+      Src s0, s1;
+      load_src(0, o, s0);
+      load_src(1, o, s1);
+      s0q[k] = value(s0, sv.scale_u(0, zbw, cx(gx)));
+      s1q[k] = value(s1, sv.scale_u(1, zbw, cx(gx)));
     } else {
       s0q[k] = s1q[k] = 0.f;
     }
     if (k >= 5) {  // the strip's first six columns: halo rows into ring slots 0..5
-      const bool hin = m.hok && k - 5 < ncol;
       Halo h;
-      load_halo(gx, hin, h);
-      put_halo(k - 5, hin, h);
+      load_halo(gx, k - 5 < ncol, h);
+      put_halo(k - 5, h);
     }
   }
   const bool row = !XIN && (flags & A_INJ) && gz == S.zr;
-  // Operands of a column, loaded with clamped indices and masked where they
-  // are taken: own cell (level L+2, the level's own content for the drop-in
+  // Operands of a column: own cell (level L+2, the level's own content for the drop-in
   // form, the injected receivers), imaging operands.
   struct Col {
     float b[5], add[5];  // level L+2; the level's own content (drop-in form) or the injected receivers
-    typename SrcView<SNAP>::Raw nt2[2];
+    Src nt2[2];
     float ntsc[2];  // their 16-bit scales
     float im[3], imc[3];
   };
   auto load_col = [&](int gx, bool more, Col& c) {
-    const int ic = m.zok && more ? gz + ldz * gx : 0;
+    const unsigned o = add_sat(zo, xo(gx, more));
     const bool inj = row && more && gx >= S.rx0 && gx < S.rx0 + S.nrx;
     const float* r = S.rec + (long long)(L - 1) * S.nrx + (inj ? gx - S.rx0 : 0);
     const long long rs = (long long)S.nt * S.nrx;
 #pragma unroll
     for (int f = 0; f < 5; ++f) {
-      c.b[f] = gld(x2 + f * fs, ic);
+      c.b[f] = x2.get(f, o);
       if (xin)
-        c.add[f] = gld(out + f * fs, ic);
+        c.add[f] = out.get(f, o);
       else
         c.add[f] = row ? gld(r + f * rs, 0) : 0.f;
     }
     if (imaging) {
-      if (next) {  // arrays 2, 3 exist only below the last level
-        sv.load_q(2, ic, m.zok && more, c.nt2[0]);
-        sv.load_q(3, ic, m.zok && more, c.nt2[1]);
-        c.ntsc[0] = sv.scale_u(2, zbw, cx(gx));
-        c.ntsc[1] = sv.scale_u(3, zbw, cx(gx));
-      } else {
-        c.nt2[0].in = c.nt2[1].in = false;
-        c.ntsc[0] = c.ntsc[1] = 0.f;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) {
+        load_src(2 + a, o, c.nt2[a]);  // used below the last level only
+        c.ntsc[a] = sv.scale_u(2 + a, zbw, cx(gx));
       }
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        c.im[a] = gld(S.img + a * n2, ic);
-        c.imc[a] = comp ? gld(S.imgc + a * n2, ic) : 0.f;
+        c.im[a] = img.get(o, a * 4u * (unsigned)n2);
+        c.imc[a] = comp ? imgc.get(o, a * 4u * (unsigned)n2) : 0.f;
       }
     }
   };
@@ -1893,22 +1880,20 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
     const int x = xs + DIR * st;
     const bool more = st + 1 < ncol;
     const int xq = x + 6 * DIR;  // column entering the queues
-    const bool qok = m.zok && more && xq >= 0 && xq < nx;
-    const int iq = qok ? gz + ldz * xq : 0;
+    const unsigned oq = add_sat(zo, xo(xq, more && xq >= 0 && xq < nx));
     Raw nr;
-    raw(iq, nr);
-    typename SrcView<SNAP>::Raw ns0, ns1;
+    raw(oq, nr);
+    Src ns0, ns1;
     float nsc0 = 0.f, nsc1 = 0.f;
     if (imaging) {
-      sv.load_q(0, iq, qok, ns0);
-      sv.load_q(1, iq, qok, ns1);
+      load_src(0, oq, ns0);
+      load_src(1, oq, ns1);
       nsc0 = sv.scale_u(0, zbw, cx(xq));
       nsc1 = sv.scale_u(1, zbw, cx(xq));
     }
     // halo rows of the column entering the queues (centre at step st + 6)
-    const bool hq = m.hok && st + 6 < ncol;
     Halo nh;
-    load_halo(xq, hq, nh);
+    load_halo(xq, st + 6 < ncol, nh);
     load_col(x + DIR, more, nxt);
 
     const int b = st & 1;
@@ -1964,10 +1949,10 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
       for (int f = 0; f < 5; ++f) vi[f] = ksrc && L >= 3 ? (v[f] * kz) * kx : v[f];
       if (flags & A_NTS) {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) gst_nt(out + f * fs, gi, v[f]);
+        for (int f = 0; f < 5; ++f) gst_nt(outp + f * fs, gi, v[f]);
       } else {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) gst(out + f * fs, gi, v[f]);
+        for (int f = 0; f < 5; ++f) out.put(f, 4u * (unsigned)gi, v[f]);
       }
       if (imaging) {
         // the imaging arithmetic is fused only where written (fmaf), so
@@ -1976,11 +1961,11 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
         float s1 = 0.f, s2 = 0.f;
         if (next) {
           if (SNAP == SNAP_HIST) {  // arrays 2, 3 are Vx, Vz of level L+1
-            s1 = inv_dt * (sv.value_s(cur.nt2[0], cur.ntsc[0]) - s0q[5]);
-            s2 = inv_dt * (sv.value_s(cur.nt2[1], cur.ntsc[1]) - s1q[5]);
+            s1 = inv_dt * (value(cur.nt2[0], cur.ntsc[0]) - s0q[5]);
+            s2 = inv_dt * (value(cur.nt2[1], cur.ntsc[1]) - s1q[5]);
           } else {
-            s1 = inv_dt * sv.value_s(cur.nt2[0], cur.ntsc[0]);
-            s2 = inv_dt * sv.value_s(cur.nt2[1], cur.ntsc[1]);
+            s1 = inv_dt * value(cur.nt2[0], cur.ntsc[0]);
+            s2 = inv_dt * value(cur.nt2[1], cur.ntsc[1]);
           }
         }
         float s4 = 0.f, s5 = 0.f, s6 = 0.f;
@@ -2000,27 +1985,27 @@ __device__ __forceinline__ void adjm_strip(const ShotDev& S, const TileRef& tr, 
           for (int a = 0; a < 3; ++a) {
             float sa = cur.im[a], ca = cur.imc[a];
             neumaier(sa, ca, t[a]);
-            gst(S.img + a * n2, gi, sa);
-            gst(S.imgc + a * n2, gi, ca);
+            img.put(4u * (unsigned)gi, a * 4u * (unsigned)n2, sa);
+            imgc.put(4u * (unsigned)gi, a * 4u * (unsigned)n2, ca);
           }
         } else {
 #pragma unroll
-          for (int a = 0; a < 3; ++a) gst(S.img + a * n2, gi, cur.im[a] + t[a]);
+          for (int a = 0; a < 3; ++a) img.put(4u * (unsigned)gi, a * 4u * (unsigned)n2, cur.im[a] + t[a]);
         }
       }
     }
-    push(q0, qok ? fmaf(nr.m2m3, nr.xx, nr.m2 * nr.zz) : 0.f);
-    push(q2, qok ? nr.m3 * nr.xz : 0.f);
-    push(q3, qok ? nr.m1x * nr.vx : 0.f);
-    push(q4, qok ? nr.m1z * nr.vz : 0.f);
+    push(q0, fmaf(nr.m2m3, nr.xx, nr.m2 * nr.zz));
+    push(q2, nr.m3 * nr.xz);
+    push(q3, nr.m1x * nr.vx);
+    push(q4, nr.m1z * nr.vz);
 #pragma unroll
     for (int k = 0; k < 5; ++k) d1[k] = d1[k + 1];
-    d1[5] = qok ? fmaf(nr.m2, nr.xx, nr.m2m3 * nr.zz) : 0.f;
+    d1[5] = fmaf(nr.m2, nr.xx, nr.m2m3 * nr.zz);
     if (imaging) {
-      push(s0q, sv.value_s(ns0, nsc0));
-      push(s1q, sv.value_s(ns1, nsc1));
+      push(s0q, value(ns0, nsc0));
+      push(s1q, value(ns1, nsc1));
     }
-    put_halo((st + 6) % 7, hq, nh);
+    put_halo((st + 6) % 7, nh);
     cur_inj = row && more && x + DIR >= S.rx0 && x + DIR < S.rx0 + S.nrx;
   };
   Col alt;
@@ -2035,9 +2020,9 @@ __device__ __forceinline__ void adjm_kernel(const ShotDev* __restrict__ shots, c
                                             int nstrips, int L, int flags, int xw, int xcd) {
   __shared__ float col[2][6][MarchCol<NW>::MZ];  // P1, P2, P3, P4, source Vx, source Vz of the centre column
   __shared__ float hring[7][6][10];              // the same for the halo rows of the next six columns
-  const TileRef tr = strips[xcd ? xcd_tile(blockIdx.x, nstrips) : (int)blockIdx.x];
+  const TileRef tr = strips[step_tile(blockIdx.x, nstrips, xcd, flags & STEP_REV)];
   // neighbouring strips march in opposite directions (see k_fwdm)
-  if (((tr.x0 / xw) & 1) == 0)
+  if (((tr.x0 / xw) & 1) == ((flags & STEP_REV) ? 1 : 0))
     adjm_strip<SNAP, 1, NW, XIN, COMP, PROP>(shots[tr.shot], tr, L, flags, xw, col, hring);
   else
     adjm_strip<SNAP, -1, NW, XIN, COMP, PROP>(shots[tr.shot], tr, L, flags, xw, col, hring);

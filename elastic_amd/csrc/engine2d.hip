@@ -160,6 +160,8 @@ int Engine::setup(const EngineCfg& cfg, const std::vector<ShotSpec>& shots,
     }
   }
   if (cfg_.snap_fmt == SNAP_HIST && cfg_.snap_every != 1) cfg_.snap_fmt = SNAP_F32;
+  for (const ShotSpec& p : shots)
+    if (cfg_.tblock >= 2 && !march_addressable((long long)device_ldz(p.nz) * p.nx)) cfg_.tblock = 0;  // the same results
   HIPCHK(hipStreamCreateWithFlags(&st_, hipStreamNonBlocking));
   for (auto& e : ev_) HIPCHK(hipEventCreate(&e));
   res_.resize(shots.size());
@@ -427,7 +429,8 @@ int Engine::set_learned(const unsigned char* w) {
   cfg_.labc_w = w;
   const int rc = build_lcells();
   if (rc != OK) cfg_.labc_w = cfg_.labc_wa = nullptr;
-  return rc;
+  const int rd = refill_desc();
+  return rc != OK ? rc : rd;
 }
 
 int Engine::set_learned_adjoint(const unsigned char* w) {
@@ -439,7 +442,8 @@ int Engine::set_learned_adjoint(const unsigned char* w) {
   cfg_.labc_wa = w;
   const int rc = build_lcells();
   if (rc != OK) cfg_.labc_w = cfg_.labc_wa = nullptr;
-  return rc;
+  const int rd = refill_desc();
+  return rc != OK ? rc : rd;
 }
 
 // Descriptors of group g (variant 0: migration coefficients; 1: true
@@ -456,9 +460,9 @@ int Engine::fill_desc(int g, bool true_model, bool born_mode) {
     ShotDev d{};
     d.nz = p.nz; d.nx = p.nx; d.ldz = r.ldz; d.nt = cfg_.nt; d.n2 = r.n2;
     d.lev = ring_of(s);
-    // slot of level L = (L + kRing) % kRing: non-negative for the levels -1
+    // slot of level L = (L + kRing) % slots: non-negative for the levels -1
     // and 0 that the first steps read
-    d.lev_stride = 5 * r.n2; d.fstride = r.n2; d.lev_mod = kRing; d.lev_off = kRing;
+    d.lev_stride = 5 * r.n2; d.fstride = r.n2; d.lev_mod = ring_slots(gr); d.lev_off = kRing;
     if (true_model && !r.coef_true.p) { set_error("no true model set"); return E_ARG; }
     d.coef = true_model ? r.coef_true.as<float>() : r.coef.as<float>();
     d.kz = r.kfac.p ? r.kfac.as<float>() : nullptr;
@@ -511,6 +515,28 @@ Engine::Pairs Engine::adj_pairs(const Group& gr) const {
   if (cfg_.tblock == 1) return cfg_.txr <= 4 ? PAIR_TILES : PAIR_NONE;
   return small_tile(gr, false, false) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
 }
+// Slots of a group's level ring in use. One level a launch needs two: a step
+// reads the level it replaces at its own cells only, and one set of fields less
+// passes through the memory-side cache. Two levels a launch write beside the
+// two they read, and the learned layer reads both levels before the one it
+// corrects.
+int Engine::ring_slots(const Group& gr) const {
+  const bool one = cfg_.tblock != 1 && !cfg_.labc_w && !cfg_.labc_wa && small_tile(gr, true, false) == PAIR_ONE &&
+                   small_tile(gr, true, true) == PAIR_ONE && small_tile(gr, false, false) == PAIR_ONE;
+  return one ? 2 : kRing;
+}
+
+// Descriptors again, after the slots in use may have changed.
+int Engine::refill_desc() {
+  for (int g = 0; g < (int)groups_.size(); ++g) {
+    STCHK(fill_desc(g, false, false));
+    bool true_model = true;
+    for (int s : groups_[g].shots) true_model = true_model && res_[s].coef_true.p;
+    if (true_model) STCHK(fill_desc(g, true, false));
+  }
+  return OK;
+}
+
 // The tile of those launches, PAIR_ONE where one level a launch is faster.
 int Engine::small_tile(const Group& gr, bool forward, bool born) const {
   if (cfg_.tblock != 0 || tile_code() != kSmallTile || gr.shots.size() != 1) return PAIR_ONE;
@@ -531,7 +557,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
   const int nbz = single_nbz(gr);
   const int snap = (mode == 0) ? cfg_.snap_fmt : SNAP_HIST;
   for (int s : gr.shots) {
-    STCHK(launch_fill(ring_of(s), (size_t)5 * kRing * res_[s].n2, 0.f, st));
+    STCHK(launch_fill(ring_of(s), (size_t)5 * ring_slots(gr) * res_[s].n2, 0.f, st));
     if ((mode == 0 && cfg_.snap_fmt == SNAP_HIST) || mode == 4)
       STCHK(launch_fill(reinterpret_cast<float*>(snap_of(s)), 2 * res_[s].n2, 0.f, st));  // level 1
   }
@@ -557,6 +583,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
     if (mode == 2) fl |= F_RECSUB;
     if (mode == 4) fl |= F_SNAP;
     if (nt_stores()) fl |= F_NTS;
+    if (L & 1) fl |= STEP_REV;
     if (mode == 0) {
       if (cfg_.snap_fmt == SNAP_HIST) {
         fl |= F_SNAP;
@@ -581,7 +608,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
           Lm / cfg_.movie_every <= cfg_.movie_n) {
         const int s = gr.shots[0];
         const long long k = Lm / cfg_.movie_every - 1;
-        const float* lev = ring_of(s) + (size_t)(Lm % kRing) * 5 * res_[s].n2;
+        const float* lev = ring_of(s) + (size_t)(Lm % ring_slots(gr)) * 5 * res_[s].n2;
         for (int f = 0; f < 5; ++f)
           HIPCHK(hipMemcpy2DAsync(cfg_.movie + ((size_t)k * 5 + f) * cfg_.movie_nz * cfg_.movie_nx,
                                   cfg_.movie_nz * sizeof(float),
@@ -606,7 +633,7 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
   const int nbz = single_nbz(gr);
   for (size_t k = 0; k < gr.shots.size(); ++k) {
     Res& r = res_[gr.shots[k]];
-    STCHK(launch_fill(ring_of(gr.shots[k]), (size_t)5 * kRing * r.n2, 0.f, st));
+    STCHK(launch_fill(ring_of(gr.shots[k]), (size_t)5 * ring_slots(gr) * r.n2, 0.f, st));
     STCHK(launch_fill(r.img.as<float>(), 3 * r.n2, 0.f, st));
     if (cfg_.comp) STCHK(launch_fill(r.imgc.as<float>(), 3 * r.n2, 0.f, st));
   }
@@ -624,6 +651,7 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
     if (L < cfg_.nt) fl |= A_NEXT;
     if (cfg_.comp) fl |= A_COMP;
     if (nt_stores()) fl |= A_NTS;
+    if (L & 1) fl |= STEP_REV;
     if (two && pairs == PAIR_SMALL)
       STCHK(launch_adj_pair(one, ptile, L, fl, cfg_.xcd, st));
     else if (two)
@@ -839,8 +867,8 @@ int Engine::get_last_levels(int shot, float* last10) {
   const size_t nn = (size_t)p.nz * p.nx;
   const int nt = cfg_.nt;
   for (int lv = 0; lv < 2; ++lv) {
-    const int L = nt - 1 + lv;  // levels nt-1, nt (slot L % kRing)
-    STCHK(fetch_fields(last10 + 5 * lv * nn, 5, p.nz, p.nx, r.ldz, base + (size_t)(L % kRing) * 5 * r.n2, r.n2,
+    const int L = nt - 1 + lv;  // levels nt-1, nt (slot L % ring_slots)
+    STCHK(fetch_fields(last10 + 5 * lv * nn, 5, p.nz, p.nx, r.ldz, base + (size_t)(L % ring_slots(gr)) * 5 * r.n2, r.n2,
                        nullptr, st_));
   }
   return OK;

@@ -182,6 +182,8 @@ class Engine {
   Pairs fwd_pairs(const Group& gr, int mode) const;
   Pairs adj_pairs(const Group& gr) const;
   int small_tile(const Group& gr, bool forward, bool born) const;
+  int ring_slots(const Group& gr) const;
+  int refill_desc();
   long long fwd_launch_count(const Group& gr, int mode) const;
   long long adj_launch_count(const Group& gr) const;
   void destroy_graphs();

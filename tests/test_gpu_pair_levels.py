@@ -44,6 +44,31 @@ def test_pairs(hip, monkeypatch, nz, nx, tile):
             _same(monkeypatch, tile, lambda: [hip.born(s, coefs, wav, dm)])
 
 
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("tile", TILES)
+def test_one_shot_batch(hip, monkeypatch, tile, graph):
+    """Synthesized data (the second run subtracts from the record) and migrations
+    of a one-shot batch, twice, the second time from the captured graphs."""
+    nz, nx, nt = 61, 77, 33
+    s, coefs, wav, rng = _setup(hip, nz, nx, nt)
+    true = [np.asfortranarray(c * np.float32(1.05)) for c in coefs]
+    spec = dict(nz=nz, nx=nx, xs=nx // 2, zs=nz // 2, zr=20, rx0=1, nrx=nx - 2)
+
+    def run():
+        b = hip.Batch(nt, 10.0, 1e-3, [spec], [coefs], wav, abc=6, adj_abc=1, txr=1, use_graph=graph)
+        b.set_true_model([true])
+        out = []
+        for _ in range(2):
+            b.synthesize()
+            out.append(b.get_data(0))
+            b.migrate()
+            out += list(b.image(0))
+        b.close()
+        return out
+
+    _same(monkeypatch, tile, run)
+
+
 @pytest.mark.parametrize("nt", [1, 2, 3, 4])
 def test_few_levels(hip, monkeypatch, nt):
     s, coefs, wav, rng = _setup(hip, 40, 30, nt)

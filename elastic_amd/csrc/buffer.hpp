@@ -24,6 +24,9 @@ struct Buf {
   __device__ __forceinline__ void put(unsigned cell, unsigned array, float v) const {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, cell, array, 0);
   }
+  __device__ __forceinline__ void put_nt(unsigned cell, unsigned array, float v) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, cell, array, 2);
+  }
   __device__ __forceinline__ void put16(unsigned cell, unsigned short v) const {
     __builtin_amdgcn_raw_buffer_store_b16(v, r, cell, 0, 0);
   }

@@ -732,7 +732,8 @@ int Engine::set_true_model(const std::vector<const float*>& coef5_true) {
   if (coef5_true.size() != specs_.size()) { set_error("true-model list size mismatch"); return E_ARG; }
   for (size_t s = 0; s < specs_.size(); ++s) {
     Res& r = res_[s];
-    STCHK(r.coef_true.alloc(5 * r.n2 * sizeof(float), "true-model coefficients"));
+    // kept from one true model to the next: captured launches hold its address
+    if (!r.coef_true.p) STCHK(r.coef_true.alloc(5 * r.n2 * sizeof(float), "true-model coefficients"));
     STCHK(fill_masked_coefs(coef5_true[s], specs_[s].nz, specs_[s].nx, r.ldz, r.coef_true.as<float>(), st_));
   }
   for (int g = 0; g < (int)groups_.size(); ++g) STCHK(fill_desc(g, true, false));

@@ -1,0 +1,38 @@
+"""A batch whose true model is set again between syntheses: the second data set
+is that of the second model, also when the launches are replayed from graphs
+captured with the first one, with one and with several shots a group and with
+one and two levels a launch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("pair", ["0", "1"])
+@pytest.mark.parametrize("shots", [1, 2])
+def test_true_model_set_again(hip, monkeypatch, shots, pair):
+    nz, nx, nt = 61, 77, 33
+    monkeypatch.setenv("RTM_PAIR", pair)
+    rng = np.random.default_rng(shots)
+    coefs = [np.asfortranarray(c * rng.uniform(0.5, 1.0, (nz, nx)), np.float32) for c in (1e-7, 1e-7, 1e6, 1e6, 3e6)]
+    models = [[np.asfortranarray(c * np.float32(f)) for c in coefs] for f in (1.05, 0.9, 1.02)]
+    wav = rng.standard_normal(nt).astype(np.float32)
+    spec = dict(nz=nz, nx=nx, xs=nx // 2, zs=nz // 2, zr=20, rx0=1, nrx=nx - 2)
+
+    def batch(graph):
+        return hip.Batch(nt, 10.0, 1e-3, [spec] * shots, [coefs] * shots, wav, abc=6, adj_abc=1, txr=1, use_graph=graph)
+
+    def data(b, model):
+        b.set_true_model([model] * shots)
+        b.synthesize()
+        return [b.get_data(i) for i in range(shots)]
+
+    kept = batch(1)
+    for model in models:
+        print("true model again", shots, pair, flush=True)
+        fresh = batch(0)
+        want = data(fresh, model)
+        fresh.close()
+        for g, w in zip(data(kept, model), want):
+            assert np.array_equal(g, w) and np.abs(w).max() > 0
+    kept.close()

@@ -383,6 +383,10 @@ int Engine::build_groups() {
     }
     g.ntiles = (int)tiles.size() - g.tile0;
     if (!march) g.nstrips = 0;
+    g.ftile = small_tile(g, true, false);
+    g.btile = small_tile(g, true, true);
+    g.atile = small_tile(g, false, false);
+    g.slots = ring_slots(g);
     G_ = std::max(G_, (int)g.shots.size());
     groups_.push_back(g);
   }
@@ -462,7 +466,7 @@ int Engine::fill_desc(int g, bool true_model, bool born_mode) {
     d.lev = ring_of(s);
     // slot of level L = (L + kRing) % slots: non-negative for the levels -1
     // and 0 that the first steps read
-    d.lev_stride = 5 * r.n2; d.fstride = r.n2; d.lev_mod = ring_slots(gr); d.lev_off = kRing;
+    d.lev_stride = 5 * r.n2; d.fstride = r.n2; d.lev_mod = gr.slots; d.lev_off = kRing;
     if (true_model && !r.coef_true.p) { set_error("no true model set"); return E_ARG; }
     d.coef = true_model ? r.coef_true.as<float>() : r.coef.as<float>();
     d.kz = r.kfac.p ? r.kfac.as<float>() : nullptr;
@@ -506,14 +510,14 @@ int Engine::single_nbz(const Group& gr) const {
 Engine::Pairs Engine::fwd_pairs(const Group& gr, int mode) const {
   if (cfg_.labc_w && mode <= 3) return PAIR_NONE;
   if (cfg_.tblock == 1) return mode != 5 && cfg_.txr <= 4 ? PAIR_TILES : PAIR_NONE;
-  return small_tile(gr, true, mode == 5) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
+  return (mode == 5 ? gr.btile : gr.ftile) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
 }
 // The same of its adjoint run (no two-level form with the R/Src sponge; the
 // learned layer corrects every level).
 Engine::Pairs Engine::adj_pairs(const Group& gr) const {
   if (cfg_.adj_abc == 2 || cfg_.labc_wa) return PAIR_NONE;
   if (cfg_.tblock == 1) return cfg_.txr <= 4 ? PAIR_TILES : PAIR_NONE;
-  return small_tile(gr, false, false) != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
+  return gr.atile != PAIR_ONE ? PAIR_SMALL : PAIR_NONE;
 }
 // Slots of a group's level ring in use. One level a launch needs two: a step
 // reads the level it replaces at its own cells only, and one set of fields less
@@ -521,14 +525,15 @@ Engine::Pairs Engine::adj_pairs(const Group& gr) const {
 // two they read, and the learned layer reads both levels before the one it
 // corrects.
 int Engine::ring_slots(const Group& gr) const {
-  const bool one = cfg_.tblock != 1 && !cfg_.labc_w && !cfg_.labc_wa && small_tile(gr, true, false) == PAIR_ONE &&
-                   small_tile(gr, true, true) == PAIR_ONE && small_tile(gr, false, false) == PAIR_ONE;
+  const bool one = cfg_.tblock != 1 && !cfg_.labc_w && !cfg_.labc_wa && gr.ftile == PAIR_ONE && gr.btile == PAIR_ONE &&
+                   gr.atile == PAIR_ONE;
   return one ? 2 : kRing;
 }
 
 // Descriptors again, after the slots in use may have changed.
 int Engine::refill_desc() {
   for (int g = 0; g < (int)groups_.size(); ++g) {
+    groups_[g].slots = ring_slots(groups_[g]);
     STCHK(fill_desc(g, false, false));
     bool true_model = true;
     for (int s : groups_[g].shots) true_model = true_model && res_[s].coef_true.p;
@@ -538,6 +543,7 @@ int Engine::refill_desc() {
 }
 
 // The tile of those launches, PAIR_ONE where one level a launch is faster.
+// Asked once per group: the ring's slots go by it.
 int Engine::small_tile(const Group& gr, bool forward, bool born) const {
   if (cfg_.tblock != 0 || tile_code() != kSmallTile || gr.shots.size() != 1) return PAIR_ONE;
   return pair_tile(specs_[gr.shots[0]].nz, specs_[gr.shots[0]].nx, forward, born);
@@ -557,7 +563,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
   const int nbz = single_nbz(gr);
   const int snap = (mode == 0) ? cfg_.snap_fmt : SNAP_HIST;
   for (int s : gr.shots) {
-    STCHK(launch_fill(ring_of(s), (size_t)5 * ring_slots(gr) * res_[s].n2, 0.f, st));
+    STCHK(launch_fill(ring_of(s), (size_t)5 * gr.slots * res_[s].n2, 0.f, st));
     if ((mode == 0 && cfg_.snap_fmt == SNAP_HIST) || mode == 4)
       STCHK(launch_fill(reinterpret_cast<float*>(snap_of(s)), 2 * res_[s].n2, 0.f, st));  // level 1
   }
@@ -568,7 +574,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
   const bool learn = cfg_.labc_w && mode <= 3;
   const LCell* lcells = learn ? d_lcells_.as<LCell>() + gr.lcell0 : nullptr;
   const Pairs pairs = fwd_pairs(gr, mode);
-  const int ptile = small_tile(gr, true, born);
+  const int ptile = born ? gr.btile : gr.ftile;
   const ShotDev& one = h_desc_[(size_t)variant * specs_.size() + gr.desc0];
   for (int L = first; L <= cfg_.nt;) {
     const bool two = pairs != PAIR_NONE && (born || L >= 3) && L + 1 <= cfg_.nt;
@@ -608,7 +614,7 @@ int Engine::enqueue_forward(int g, int mode, hipStream_t st) {
           Lm / cfg_.movie_every <= cfg_.movie_n) {
         const int s = gr.shots[0];
         const long long k = Lm / cfg_.movie_every - 1;
-        const float* lev = ring_of(s) + (size_t)(Lm % ring_slots(gr)) * 5 * res_[s].n2;
+        const float* lev = ring_of(s) + (size_t)(Lm % gr.slots) * 5 * res_[s].n2;
         for (int f = 0; f < 5; ++f)
           HIPCHK(hipMemcpy2DAsync(cfg_.movie + ((size_t)k * 5 + f) * cfg_.movie_nz * cfg_.movie_nx,
                                   cfg_.movie_nz * sizeof(float),
@@ -633,12 +639,12 @@ int Engine::enqueue_adjoint(int g, hipStream_t st) {
   const int nbz = single_nbz(gr);
   for (size_t k = 0; k < gr.shots.size(); ++k) {
     Res& r = res_[gr.shots[k]];
-    STCHK(launch_fill(ring_of(gr.shots[k]), (size_t)5 * ring_slots(gr) * r.n2, 0.f, st));
+    STCHK(launch_fill(ring_of(gr.shots[k]), (size_t)5 * gr.slots * r.n2, 0.f, st));
     STCHK(launch_fill(r.img.as<float>(), 3 * r.n2, 0.f, st));
     if (cfg_.comp) STCHK(launch_fill(r.imgc.as<float>(), 3 * r.n2, 0.f, st));
   }
   const Pairs pairs = adj_pairs(gr);
-  const int ptile = small_tile(gr, false, false);
+  const int ptile = gr.atile;
   const ShotDev& one = h_desc_[gr.desc0];
   const LCell* lcells = cfg_.labc_wa ? d_lcells_.as<LCell>() + gr.lcell0 : nullptr;
   for (int L = cfg_.nt; L >= 1;) {
@@ -868,8 +874,8 @@ int Engine::get_last_levels(int shot, float* last10) {
   const size_t nn = (size_t)p.nz * p.nx;
   const int nt = cfg_.nt;
   for (int lv = 0; lv < 2; ++lv) {
-    const int L = nt - 1 + lv;  // levels nt-1, nt (slot L % ring_slots)
-    STCHK(fetch_fields(last10 + 5 * lv * nn, 5, p.nz, p.nx, r.ldz, base + (size_t)(L % ring_slots(gr)) * 5 * r.n2, r.n2,
+    const int L = nt - 1 + lv;  // levels nt-1, nt (slot L % slots)
+    STCHK(fetch_fields(last10 + 5 * lv * nn, 5, p.nz, p.nx, r.ldz, base + (size_t)(L % gr.slots) * 5 * r.n2, r.n2,
                        nullptr, st_));
   }
   return OK;

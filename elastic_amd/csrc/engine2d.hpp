@@ -166,6 +166,8 @@ class Engine {
     int fstrip0 = 0, fnstrips = 0;  // slice of the strip table for the marching forward
     int fmarch_w = 0;               // its strip width
     int desc0 = 0;              // first descriptor
+    int ftile = PAIR_ONE, btile = PAIR_ONE, atile = PAIR_ONE;  // tiles of two levels a launch: forward, Born, adjoint
+    int slots = kRing;          // slots of the level ring in use, as the descriptors have them
     int lcell0 = 0, nlband = 0, nlrim = 0;  // slice of the learned layer's cell table
     hipGraphExec_t gfwd = nullptr, gadj = nullptr, gsyn = nullptr;
   };

@@ -1,7 +1,7 @@
-"""A batch whose true model is set again between syntheses: the second data set
-is that of the second model, also when the launches are replayed from graphs
-captured with the first one, with one and with several shots a group and with
-one and two levels a launch."""
+"""Batches whose settings change between runs. The true model is set again between
+syntheses: the second data set is that of the second model, also when the
+launches are replayed from graphs captured with the first one, with one and
+with several shots a group and with one and two levels a launch."""
 import numpy as np
 import pytest
 
@@ -36,3 +36,28 @@ def test_true_model_set_again(hip, monkeypatch, shots, pair):
         for g, w in zip(data(kept, model), want):
             assert np.array_equal(g, w) and np.abs(w).max() > 0
     kept.close()
+
+
+@pytest.mark.parametrize("created,run", [("-1", "0"), ("0", "-1"), ("3", "0"), ("0", "3")])
+def test_levels_a_launch_are_the_batchs_own(hip, monkeypatch, created, run):
+    """How many levels a launch takes, and with it the ring of levels, is decided
+    when a batch is created: a run under another RTM_PAIR (-1: the rule) gives the
+    same images."""
+    nz, nx = 61, 77
+    spec = dict(nz=nz, nx=nx, xs=nx // 2, zs=nz // 2, zr=20, rx0=1, nrx=nx - 2)
+    rng = np.random.default_rng(3)
+    coefs = [np.asfortranarray(c * rng.uniform(0.5, 1.0, (nz, nx)), np.float32) for c in (1e-7, 1e-7, 1e6, 1e6, 3e6)]
+    for nt in (32, 33, 34, 35):
+        print("levels a launch", created, run, nt, flush=True)
+        rec = rng.standard_normal((5, nx - 2, nt)).astype(np.float32)
+        wav = rng.standard_normal(nt).astype(np.float32)
+        monkeypatch.setenv("RTM_PAIR", created)
+        b = hip.Batch(nt, 10.0, 1e-3, [spec], [coefs], wav, abc=6, adj_abc=1, txr=1)
+        b.set_data(0, rec)
+        b.migrate()
+        want = b.image(0)
+        monkeypatch.setenv("RTM_PAIR", run)
+        b.migrate()
+        for w, g in zip(want, b.image(0)):
+            assert np.array_equal(g, w) and np.abs(w).max() > 0
+        b.close()

@@ -55,6 +55,12 @@ static std::string tune_key(const EngineCfg& c, const std::vector<ShotSpec>& sp)
   return buf;
 }
 
+// 16-bit snapshots are scaled per strip of the tile's width, so the images go by
+// it (by about 1e-3): timings must not choose it, and only width 2 (which the
+// marching forms share) is a candidate. Cached choices obey the same rule: a
+// file may hold another one's.
+static bool width_allowed(const EngineCfg& c, int txr) { return c.snap_fmt <= SNAP_F32 || txr == 2; }
+
 static void load_file_cache() {
   static bool done = false;
   if (done) return;
@@ -95,7 +101,7 @@ int autotune_txr(const EngineCfg& cfg, const std::vector<ShotSpec>& shots, const
     std::lock_guard<std::mutex> lk(g_tune_mu);
     load_file_cache();
     auto it = g_tune_cache.find(key);
-    if (use_cache && it != g_tune_cache.end()) {
+    if (use_cache && it != g_tune_cache.end() && width_allowed(cfg, it->second & 15)) {
       *best = it->second & 15;
       *best_tblock = (it->second >> 4) & 15;
       if (best_march_w && (it->second >> 8) > 0) *best_march_w = it->second >> 8;
@@ -155,10 +161,7 @@ int autotune_txr(const EngineCfg& cfg, const std::vector<ShotSpec>& shots, const
   };
   for (int i = 0; i < 8; ++i) {
     t[i] = -1;
-    // 16-bit snapshots are scaled per strip of the tile's width, so the images
-    // go by it (by about 1e-3): timings must not choose it, and only width 2
-    // (which the marching forms share) is a candidate
-    if (c.snap_fmt > SNAP_F32 && cand[i][0] != 2) continue;
+    if (!width_allowed(c, cand[i][0])) continue;
     if (i < 7) {
       STCHK(time_form(cand[i][0], cand[i][1], &t[i]));
     } else {

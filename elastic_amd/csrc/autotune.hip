@@ -159,8 +159,13 @@ int autotune_txr(const EngineCfg& cfg, const std::vector<ShotSpec>& shots, const
     *ms = std::min(t1, e.timing().total_ms);
     return OK;
   };
+  // the engine runs tiles where a grid is too large to march: no candidate then
+  const bool marches = std::all_of(shots.begin(), shots.end(), [](const ShotSpec& p) {
+    return march_addressable((long long)device_ldz(p.nz) * p.nx);
+  });
   for (int i = 0; i < 8; ++i) {
     t[i] = -1;
+    if (i == 7 && !marches) continue;
     if (!width_allowed(c, cand[i][0])) continue;
     if (i < 7) {
       STCHK(time_form(cand[i][0], cand[i][1], &t[i]));

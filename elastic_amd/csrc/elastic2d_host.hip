@@ -912,8 +912,8 @@ RTM_EXPORT int rtm_batch_create(rtm_batch** out, const rtm_batch_cfg_t* cfg, int
   b->nt = cfg->nt;
   if (tune) STCHK(autotune_txr(ec, sp, cf, wavelet, &ec.txr, &ec.tblock, nullptr, true, &ec.march_w));
   b->txr = ec.txr;
-  b->tblock = ec.tblock;
   STCHK(b->eng.setup(ec, sp, cf, wavelet));
+  b->tblock = b->eng.tblock();
   b->march_w = b->eng.first_march_w();
   *out = b.release();
   return OK;

@@ -141,6 +141,8 @@ class Engine {
     const int w = cfg_.tblock == 3 ? groups_[0].fmarch_w : groups_[0].march_w;
     return w > 0 ? w : cfg_.march_w;
   }
+  // kernel form the engine runs (tiles where a grid is too large to march)
+  int tblock() const { return cfg_.tblock; }
   int group_size() const { return G_; }
   int ngroups() const { return (int)groups_.size(); }
 

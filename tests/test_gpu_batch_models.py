@@ -61,3 +61,18 @@ def test_levels_a_launch_are_the_batchs_own(hip, monkeypatch, created, run):
         for w, g in zip(want, b.image(0)):
             assert np.array_equal(g, w) and np.abs(w).max() > 0
         b.close()
+
+
+@pytest.mark.parametrize("nx,form", [(10355, 2), (10357, 0)])
+def test_reported_form_of_large_grids(hip, monkeypatch, nx, form):
+    """The marching forms take grids of up to 2^31 / 20 cells (columns of 10368
+    rows: 10356); a batch that asked for one on a larger grid says that it runs
+    tiles."""
+    nz = 10368
+    print("large grid", nz, nx, flush=True)
+    monkeypatch.setenv("RTM_TBLOCK", "2")
+    field = np.zeros((nz, nx), np.float32, order="F")
+    spec = dict(nz=nz, nx=nx, xs=20, zs=20, zr=20, rx0=0, nrx=4)
+    b = hip.Batch(2, 10.0, 1e-3, [spec], [[field] * 5], np.ones(2, np.float32), txr=2, snap_every=2)
+    assert b.tblock == form
+    b.close()

@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <map>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -11,28 +12,45 @@ namespace erm {
 
 namespace {
 
-// Streams of the copy threads: one set per process, on the device of its last
-// use, used by one call at a time (concurrent calls share one link anyway).
-std::mutex g_lanes_mu;
-std::vector<hipStream_t> g_lanes;
-int g_lanes_dev = -1;
+// Idle streams of the copy threads, by device. A call takes those it finds,
+// creates the rest and gives them back, so calls at the same time (also on other
+// devices) have streams of their own and wait for nothing but the link.
+std::mutex g_idle_mu;
+std::map<int, std::vector<hipStream_t>> g_idle;
 
-void drop_lanes() {
-  for (hipStream_t s : g_lanes) (void)hipStreamDestroy(s);
-  g_lanes.clear();
-  g_lanes_dev = -1;
-}
+// The streams of one call.
+struct Lanes {
+  int dev;
+  std::vector<hipStream_t> st;
+  bool sound = true;  // false: a lane failed, its stream may hold work
 
-int get_lanes(int n, int dev) {
-  if (g_lanes_dev != dev) drop_lanes();
-  g_lanes_dev = dev;
-  while ((int)g_lanes.size() < n) {
-    hipStream_t s;
-    HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    g_lanes.push_back(s);
+  explicit Lanes(int device) : dev(device) {}
+  int get(int n) {
+    st.reserve(n);
+    {
+      std::lock_guard<std::mutex> lock(g_idle_mu);
+      std::vector<hipStream_t>& idle = g_idle[dev];
+      for (; (int)st.size() < n && !idle.empty(); idle.pop_back()) st.push_back(idle.back());
+      idle.reserve(kLanes);  // giving back does not allocate
+    }
+    while ((int)st.size() < n) {
+      hipStream_t s;
+      HIPCHK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+      st.push_back(s);
+    }
+    return OK;
   }
-  return OK;
-}
+  ~Lanes() {
+    if (!sound)
+      for (hipStream_t s : st) (void)hipStreamSynchronize(s);
+    if (sound) {
+      std::lock_guard<std::mutex> lock(g_idle_mu);
+      std::vector<hipStream_t>& idle = g_idle[dev];
+      for (; !st.empty() && (int)idle.size() < kLanes; st.pop_back()) idle.push_back(st.back());
+    }
+    for (hipStream_t s : st) (void)hipStreamDestroy(s);
+  }
+};
 
 int copy(void* dst, const void* src, size_t n, hipMemcpyKind kind) {
   if (n == 0) return OK;
@@ -58,12 +76,12 @@ int with_copy_lanes(int n, const std::function<int(int, hipStream_t)>& work) {
   n = std::min(std::max(n, 1), kLanes);
   int dev = 0;
   HIPCHK(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lock(g_lanes_mu);
-  STCHK(get_lanes(n, dev));
+  Lanes lanes(dev);
+  STCHK(lanes.get(n));
   std::vector<int> rc(n, OK);
   std::vector<std::string> msg(n);
   auto run = [&](int k) {
-    rc[k] = hipSetDevice(dev) == hipSuccess ? work(k, g_lanes[k]) : E_HIP;
+    rc[k] = hipSetDevice(dev) == hipSuccess ? work(k, lanes.st[k]) : E_HIP;
     if (rc[k] != OK) msg[k] = last_error();  // the message is the thread's own
   };
   std::vector<std::thread> th;
@@ -77,6 +95,7 @@ int with_copy_lanes(int n, const std::function<int(int, hipStream_t)>& work) {
   for (std::thread& t : th) t.join();
   for (int k = 0; k < n; ++k)
     if (rc[k] != OK) {
+      lanes.sound = false;
       set_error("%s", msg[k].c_str());
       return rc[k];
     }
@@ -84,8 +103,13 @@ int with_copy_lanes(int n, const std::function<int(int, hipStream_t)>& work) {
 }
 
 void release_copy_lanes() {
-  std::lock_guard<std::mutex> lock(g_lanes_mu);
-  drop_lanes();
+  std::map<int, std::vector<hipStream_t>> idle;
+  {
+    std::lock_guard<std::mutex> lock(g_idle_mu);
+    idle.swap(g_idle);
+  }
+  for (auto& d : idle)
+    for (hipStream_t s : d.second) (void)hipStreamDestroy(s);
 }
 
 int copy_to_device(void* dst, const void* src, size_t n) { return copy(dst, src, n, hipMemcpyHostToDevice); }

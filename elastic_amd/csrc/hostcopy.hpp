@@ -28,9 +28,10 @@ constexpr int kCopyThreads = 6;
 int copy_to_device(void* dst, const void* src, size_t n);
 int copy_to_host(void* dst, const void* src, size_t n);
 
-// Runs work(k, stream) for k = 0..n-1 on n threads, each with a stream of its
-// own; the streams are kept for the next call (at most kLanes, one user at a
-// time) until release_copy_lanes(). Where a thread cannot be started its work
+// Runs work(k, stream) for k = 0..n-1 on n threads (at most kLanes), each with a
+// stream of its own. Calls may run at the same time, on one device or several;
+// idle streams, at most kLanes a device, are kept for the next calls until
+// release_copy_lanes(). Where a thread cannot be started its work
 // runs on the calling thread after the others. Returns the first error.
 constexpr int kLanes = 8;
 int with_copy_lanes(int n, const std::function<int(int, hipStream_t)>& work);

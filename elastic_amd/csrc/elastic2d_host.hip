@@ -6,10 +6,8 @@
 
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -17,6 +15,7 @@
 #include "../../include/rtmlib_modC.h"
 #include "engine2d.hpp"
 #include "hostcopy.hpp"
+#include "op3_chunks.hpp"
 
 namespace erm {
 
@@ -50,113 +49,6 @@ static int snap_fmt_of(int prec, int every) {
 // ---------------------------------------------------------------------------
 // Drop-in adjoint on full (nz,nx,nt) histories, W/rtmlib-modC.c:120-253, from
 // the histories in[f] into out[f] (the same arrays: in place).
-//
-// The host link bounds it: every level goes up and comes down once. The
-// histories pass in chunks of levels, from the top; each chunk's pieces go up
-// from several threads, whichever completes a chunk launches its steps, and
-// finished levels come down from other threads while later ones go up (the
-// link carries both directions at once). 390 x 690 x 100 levels (1.08 GB both
-// ways): 51 ms one after the
-// other from one thread, 19 to 22 ms like this.
-namespace {
-struct Op3Run {
-  int nt, nup;
-  size_t n2;
-  const float* const* in;
-  float* const* out;
-  float* dev;                         // field f of level L at dev + (f*nt + L)*n2
-  int chunk;                          // levels per chunk; chunk 0 ends at level nt
-  int nchunk;
-  std::function<int(int)> step;       // launches the step of a level
-  hipStream_t st;
-  std::vector<hipEvent_t> ev;         // 2c: before, 2c+1: after the steps of chunk c
-  std::mutex mu;
-  std::condition_variable cv;
-  std::vector<size_t> left;           // bytes of chunk c still to go up
-  size_t up_task = 0, down_task = 0;  // next tasks, chunk by chunk
-  int launched = 0;                   // chunks whose steps are queued
-  bool failed = false;
-
-  int hi(int c) const { return nt - c * chunk; }
-  int lo(int c) const { return std::max(0, hi(c) - chunk); }
-  size_t field_bytes(int c, bool down) const {
-    // in place the top two levels are as they were
-    const int h = down && in[0] == out[0] ? std::min(hi(c), nt - 2) : hi(c);
-    return h > lo(c) ? (size_t)(h - lo(c)) * n2 * sizeof(float) : 0;
-  }
-  size_t pieces() const { return ((size_t)chunk * n2 * sizeof(float) + kCopyPiece - 1) / kCopyPiece; }
-  size_t tasks() const { return (size_t)nchunk * 5 * pieces(); }
-  // task -> chunk, field and bytes [o, o+m) of the chunk's run of that field
-  bool piece(size_t task, bool down, int* c, int* f, size_t* o, size_t* m) const {
-    const size_t np = pieces();
-    *c = (int)(task / (5 * np));
-    *f = (int)(task / np % 5);
-    *o = task % np * kCopyPiece;
-    const size_t n = field_bytes(*c, down);
-    *m = *o < n ? std::min(kCopyPiece, n - *o) : 0;
-    return *m > 0;
-  }
-  char* at(float* base, int c, size_t o) const { return reinterpret_cast<char*>(base + (size_t)lo(c) * n2) + o; }
-
-  // with mu held: queues the steps of every chunk that is complete
-  int advance() {
-    while (launched < nchunk && left[launched] == 0) {
-      const int c = launched;
-      HIPCHK(hipEventRecord(ev[2 * c], st));
-      for (int L = std::min(hi(c), nt - 2) - 1; L >= lo(c); --L) STCHK(step(L));
-      HIPCHK(hipEventRecord(ev[2 * c + 1], st));
-      ++launched;
-      cv.notify_all();
-    }
-    return OK;
-  }
-  int up(hipStream_t lane) {
-    for (;;) {
-      int c, f;
-      size_t o, m;
-      {
-        std::lock_guard<std::mutex> lk(mu);
-        if (failed || up_task == tasks()) return OK;
-        if (!piece(up_task++, false, &c, &f, &o, &m)) continue;
-      }
-      HIPCHK(hipMemcpyAsync(at(dev + (size_t)f * nt * n2, c, o), at(const_cast<float*>(in[f]), c, o), m,
-                            hipMemcpyHostToDevice, lane));
-      HIPCHK(hipStreamSynchronize(lane));
-      std::lock_guard<std::mutex> lk(mu);
-      left[c] -= m;
-      STCHK(advance());
-    }
-  }
-  int down(hipStream_t lane) {
-    for (;;) {
-      int c, f;
-      size_t o, m;
-      {
-        std::unique_lock<std::mutex> lk(mu);
-        if (failed || down_task == tasks()) return OK;
-        if (!piece(down_task++, true, &c, &f, &o, &m)) continue;
-        cv.wait(lk, [&] { return failed || launched > c; });
-        if (failed) return OK;
-      }
-      HIPCHK(hipStreamWaitEvent(lane, ev[2 * c + 1], 0));
-      HIPCHK(hipMemcpyAsync(at(out[f], c, o), at(dev + (size_t)f * nt * n2, c, o), m, hipMemcpyDeviceToHost, lane));
-      HIPCHK(hipStreamSynchronize(lane));
-    }
-  }
-  // thread k: the first nup upload until all is up, then download too
-  int work(int k, hipStream_t lane) {
-    int rc = k < nup ? up(lane) : OK;
-    if (rc == OK) rc = down(lane);
-    if (rc != OK) {
-      std::lock_guard<std::mutex> lk(mu);
-      failed = true;
-      cv.notify_all();
-    }
-    return rc;
-  }
-};
-}  // namespace
-
 static int op3(int nt, int nz, int nx, const float* const* in, float* const* out, const float* const* coefs) {
   if (nz < 12 || nx < 12) {
     set_error("grid %d x %d too small: the 10th-order operators need nz, nx >= 12", nz, nx);
@@ -226,12 +118,8 @@ static int op3(int nt, int nz, int nx, const float* const* in, float* const* out
   HIPCHK(hipStreamSynchronize(st));
   Op3Run run;
   run.nt = nt; run.n2 = (size_t)n2; run.in = in; run.out = out; run.dev = hp; run.st = st;
-  const size_t total = 5 * (size_t)nt * n2 * sizeof(float), level = 5 * (size_t)n2 * sizeof(float);
-  // chunks of about 16 MB, at most 256 of them; the first holds a stepped level
-  run.chunk = (int)std::max<size_t>({(kCopyPiece * 4 + level - 1) / level, ((size_t)nt + 255) / 256, 3});
-  run.nchunk = (nt + run.chunk - 1) / run.chunk;
-  run.left.resize(run.nchunk);
-  for (int c = 0; c < run.nchunk; ++c) run.left[c] = 5 * run.field_bytes(c, false);
+  const size_t total = 5 * (size_t)nt * n2 * sizeof(float);
+  run.split();
   run.step = [&](int it) -> int {
     if (march)
       return launch_adjm(dd.as<ShotDev>(), dt.as<TileRef>(), (int)tiles.size(), it, A_XIN, mw, mnw, SNAP_HIST,

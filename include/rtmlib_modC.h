@@ -57,8 +57,8 @@ int rtm_op3_hip(int nt, int nz, int nx, int zrec, float *Vx0, float *Vz0, float 
 
 /* rtm_op3_hip from five histories (Vx, Vz, sxx, szz, sxz) into five others,
  * for callers that keep their input: the result is written once instead of the
- * input being copied first. hist and out must not overlap, except that all of
- * out may be hist (in place). coefs: m1_x, m1_z, aux_m2, aux_m3, aux_m2m3. */
+ * input being copied first. hist and out must not overlap, except that any
+ * out[f] may be hist[f] (that field in place). coefs: m1_x, m1_z, aux_m2, aux_m3, aux_m2m3. */
 int rtm_op3_hip_to(int nt, int nz, int nx, const float *const *hist, float *const *out,
                    const float *const *coefs);
 

@@ -142,7 +142,6 @@ static int op3(int nt, int nz, int nx, const float* const* in, float* const* out
     run.nup = 1;
     STCHK(run.work(0, st));
   } else {
-    run.nup = kLanes / 2;
     const int rc = with_copy_lanes(kLanes, [&](int k, hipStream_t lane) { return run.work(k, lane); });
     if (rc != OK) (void)hipStreamSynchronize(st);  // steps in flight use this call's buffers
     STCHK(rc);

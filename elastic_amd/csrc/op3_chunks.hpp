@@ -5,7 +5,8 @@
 // from several threads, whichever completes a chunk launches its steps, and
 // finished levels come down from other threads while later ones go up (the
 // link carries both directions at once). 390 x 690 x 100 levels (1.08 GB both
-// ways): 51 ms one after the other from one thread, 19 to 22 ms like this.
+// ways): 51 ms one after the other from one thread, 19 to 22 ms like this; 21 to 25
+// in place, where the levels come down after the last step (see split()).
 #pragma once
 
 #include <algorithm>
@@ -35,6 +36,7 @@ struct Op3Run {
   size_t up_task = 0, down_task = 0;  // next tasks, chunk by chunk
   int launched = 0;                   // chunks whose steps are queued
   bool failed = false;
+  bool hold = false;                  // results wait for the last step
 
   // chunks of about 16 MB, at most 256 of them; the first holds a stepped level
   void split() {
@@ -43,6 +45,14 @@ struct Op3Run {
     nchunk = (nt + chunk - 1) / chunk;
     left.resize(nchunk);
     for (int c = 0; c < nchunk; ++c) left[c] = 5 * field_bytes(c, 0, false);
+    // A result that goes into an input: nothing is written until every step has
+    // run, so that a call that fails on the way leaves the caller's histories as
+    // they were.
+    const std::less<const float*> before;
+    for (int f = 0; f < 5; ++f)
+      for (int g = 0; g < 5; ++g)
+        hold |= before(out[f], in[g] + (size_t)nt * n2) && before(in[g], out[f] + (size_t)nt * n2);
+    nup = hold ? kLanes : kLanes / 2;
   }
   int hi(int c) const { return nt - c * chunk; }
   int lo(int c) const { return std::max(0, hi(c) - chunk); }
@@ -102,10 +112,14 @@ struct Op3Run {
         std::unique_lock<std::mutex> lk(mu);
         if (failed || down_task == tasks()) return OK;
         if (!piece(down_task++, true, &c, &f, &o, &m)) continue;
-        cv.wait(lk, [&] { return failed || launched > c; });
+        const int last = hold ? nchunk - 1 : c;
+        cv.wait(lk, [&] { return failed || launched > last; });
         if (failed) return OK;
       }
-      HIPCHK(hipStreamWaitEvent(lane, ev[2 * c + 1], 0));
+      if (hold)
+        HIPCHK(hipEventSynchronize(ev[2 * nchunk - 1]));
+      else
+        HIPCHK(hipStreamWaitEvent(lane, ev[2 * c + 1], 0));
       HIPCHK(hipMemcpyAsync(at(out[f], c, o), at(dev + (size_t)f * nt * n2, c, o), m, hipMemcpyDeviceToHost, lane));
       HIPCHK(hipStreamSynchronize(lane));
     }

@@ -54,7 +54,6 @@ static int run(int nt, size_t n2, unsigned alias, bool threads, int fail_level, 
   for (int i = 0; i < 2 * r.nchunk; ++i) r.ev.push_back(new int(0));
   int rc;
   if (threads) {
-    r.nup = kLanes / 2;
     rc = with_copy_lanes(kLanes, [&](int k, hipStream_t lane) { return r.work(k, lane); });
   } else {
     hipStream_t lane;
@@ -88,6 +87,27 @@ int main() {
         }
       }
   }
+  // a step or a copy up that fails leaves histories that are worked on in place as
+  // they were: the first step, one on the way, the last; copies of every chunk
+  for (bool threads : {false, true})
+    for (unsigned alias : {31u, 1u}) {
+      const int nt = 61;
+      const size_t n2 = 30000;
+      const History given = start(nt, n2);
+      History in, out;
+      for (int level : {nt - 3, nt / 2, 0}) {
+        CHECK(run(nt, n2, alias, threads, level, in, out) == E_HIP);
+        CHECK(std::string(last_error()) == "level " + std::to_string(level));
+        CHECK(in == given);
+      }
+      for (int copy : {0, 7, 10, 14}) {  // 15 go up: five fields of three chunks
+        host_hip::copies = 0;
+        host_hip::fail_copy = copy;
+        CHECK(run(nt, n2, alias, threads, -1, in, out) == E_HIP);
+        host_hip::fail_copy = -1;
+        CHECK(in == given);
+      }
+    }
   std::printf("OK\n");
   return 0;
 }

@@ -21,8 +21,10 @@
 #include "common.hpp"
 #include "engine2d.hpp"
 #include "hostcopy.hpp"
+#include "layout.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -519,20 +521,45 @@ static int ac3_launch(ac3d* a, const float* p, float* pp, const float* c, int mo
   return OK;
 }
 
-// Rows between the caller's layout and the device's; the source field of the
-// passes, which begin with a fill of their own, carries the contiguous side.
-static int ac3_rows(ac3d* a, const float* in, float* out, int ld_in, int ld_out) {
-  const long long rows = a->plane;
-  hipLaunchKernelGGL(k_ac3_rows, dim3((unsigned)std::min<long long>((rows + 3) / 4, 65536)), dim3(64, 4), 0, a->st, in,
-                     out, a->cfg.n1, rows, ld_in, ld_out);
+// Rows between the caller's layout and the device's.
+static int ac3_rows(const float* in, float* out, int n1, long long rows, int ld_in, int ld_out, hipStream_t st) {
+  hipLaunchKernelGGL(k_ac3_rows, dim3((unsigned)std::min<long long>((rows + 3) / 4, 65536)), dim3(64, 4), 0, st, in, out,
+                     n1, rows, ld_in, ld_out);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipStreamSynchronize(a->st));
   return OK;
 }
+// To the device: the source field of the passes, which begin with a fill of their
+// own, carries the contiguous side.
 static int ac3_upload(ac3d* a, const float* host, float* dev) {
   if (a->ld == a->cfg.n1) return copy_to_device(dev, host, a->n * 4);
   STCHK(copy_to_device(a->f0.p, host, a->n * 4));
-  return ac3_rows(a, a->f0.as<float>(), dev + a->lead, a->cfg.n1, a->ld);
+  STCHK(ac3_rows(a->f0.as<float>(), dev + a->lead, a->cfg.n1, a->plane, a->cfg.n1, a->ld, a->st));
+  HIPCHK(hipStreamSynchronize(a->st));
+  return OK;
+}
+// From the device, where a run may be using the fields: through scratch of its
+// own. Large arrays in pieces of whole rows, a piece of each copy thread at a time.
+static int ac3_fetch(ac3d* a, const float* dev, float* host) {
+  const int n1 = a->cfg.n1;
+  const size_t row = (size_t)n1 * 4;
+  const long long most = std::max<long long>(kCopyPiece / row, 1), pieces = (a->plane + most - 1) / most;
+  const int lanes = (int)std::min<long long>(pieces, kCopyThreads);
+  DevBuf t;
+  if (a->n * 4 < kLargeToHost || t.alloc(lanes * most * row, "scratch") != OK) {
+    (void)hipGetLastError();  // no scratch: fetch_fields does without
+    return fetch_fields(host, 1, n1, (int)a->plane, a->ld, dev, 0, nullptr, a->st);
+  }
+  std::atomic<long long> next{0};
+  return with_copy_lanes(lanes, [&](int lane, hipStream_t st) -> int {
+    float* const s = t.as<float>() + lane * most * n1;
+    for (long long k = next++; k < pieces; k = next++) {
+      const long long r0 = k * most, rows = std::min(most, a->plane - r0);
+      STCHK(ac3_rows(dev + r0 * a->ld, s, n1, rows, a->ld, n1, st));
+      HIPCHK(hipMemcpyAsync(host + r0 * n1, s, rows * row, hipMemcpyDeviceToHost, st));
+      HIPCHK(hipStreamSynchronize(st));
+    }
+    return OK;
+  });
 }
 
 // Source pass: levels 1..nt with the model c; records the receiver plane
@@ -735,8 +762,7 @@ RTM_EXPORT int ac3d_get_image(ac3d* a, float* img) {
   if (!a || !img) { set_error("null argument"); return E_ARG; }
   HIPCHK(hipStreamSynchronize(a->st));
   if (a->ld == a->cfg.n1) return copy_to_host(img, a->img.p, a->n * 4);
-  STCHK(ac3_rows(a, a->img.as<float>() + a->lead, a->f0.as<float>(), a->ld, a->cfg.n1));
-  return copy_to_host(img, a->f0.p, a->n * 4);
+  return ac3_fetch(a, a->img.as<float>() + a->lead, img);
 }
 
 RTM_EXPORT int ac3d_get_snapshot_scales(ac3d* a, float* out, int n) {

@@ -458,10 +458,10 @@ struct ac3d {
   // lies on a 128-byte line, so a wave's row is two lines instead of three; a
   // snapshot starts 32 elements later (slead), which does the same for its
   // 16-bit rows (522^3: 10% fewer L2 requests, step 565 -> 526 us, with the image
-  // 1064 -> 970). Where memory or 32-bit offsets do not allow it, rows are
-  // contiguous.
+  // 1064 -> 970). Where that takes much memory or 32-bit offsets do not allow it,
+  // rows are contiguous (lead 0).
   int lead = 0, slead = 0, ld = 0;
-  size_t np = 0, ns = 0;  // elements of a field and of a snapshot
+  size_t np = 0;  // elements of a field and of a snapshot
   long long plane = 0;
   int ychunk = 0;  // planes per step workgroup
   DevBuf c, c_alt, k, f0, f1, rec, rec_tmp, snap, smax, img, amp_h_dummy;
@@ -472,7 +472,7 @@ struct ac3d {
   double timings[6] = {0, 0, 0, 0, 0, 0};
   void* snap_at(int k) const {  // snapshot k, as the step kernel indexes it
     const size_t esz = cfg.snap_prec == 1 ? 2 : 4;
-    return snap.as<char>() + ((size_t)k * ns + slead) * esz;
+    return snap.as<char>() + ((size_t)k * np + slead) * esz;
   }
   ~ac3d() {
     for (auto& e : ev)
@@ -531,7 +531,7 @@ static int ac3_rows(const float* in, float* out, int n1, long long rows, int ld_
 // To the device: the source field of the passes, which begin with a fill of their
 // own, carries the contiguous side.
 static int ac3_upload(ac3d* a, const float* host, float* dev) {
-  if (a->ld == a->cfg.n1) return copy_to_device(dev, host, a->n * 4);
+  if (a->ld == a->cfg.n1) return copy_to_device(dev + a->lead, host, a->n * 4);
   STCHK(copy_to_device(a->f0.p, host, a->n * 4));
   STCHK(ac3_rows(a->f0.as<float>(), dev + a->lead, a->cfg.n1, a->plane, a->cfg.n1, a->ld, a->st));
   HIPCHK(hipStreamSynchronize(a->st));
@@ -589,9 +589,10 @@ static int ac3_source_pass(ac3d* a, const float* c, int record, int sub, int sna
     STCHK(ac3_launch(a, p, pp, c, 0, t, record != 0, false, sm, nullptr, 0.f, nullptr, k < 0 ? nullptr : a->snap_at(k),
                      k < 0 ? nullptr : a->smax.as<unsigned>() + (size_t)k * SMAX_SNAP));
     if (sl && t == g.nt) {
-      size_t blocks = std::min<size_t>((a->np + 255) / 256, 65536);
-      hipLaunchKernelGGL(k_ac3_snap, dim3((unsigned)blocks), dim3(256), 0, a->st, pp, a->snap_at(t / j - 1),
-                         a->np - a->lead, sm, g.snap_prec == 1);
+      const size_t cells = (size_t)a->ld * a->plane;
+      size_t blocks = std::min<size_t>((cells + 255) / 256, 65536);
+      hipLaunchKernelGGL(k_ac3_snap, dim3((unsigned)blocks), dim3(256), 0, a->st, pp, a->snap_at(t / j - 1), cells, sm,
+                         g.snap_prec == 1);
       HIPCHK(hipGetLastError());
     }
     std::swap(p, pp);
@@ -636,20 +637,24 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
   const int nsnap = std::max(g.nt / g.snap_every, 1);
   const size_t esz = g.snap_prec == 1 ? 2 : 4;
   a->ld = g.n1;
-  a->np = a->ns = a->n;
+  a->np = a->n;
   {
-    const int ld = round_up(27 + g.n1, 64);
-    const size_t np = (size_t)ld * a->plane, ns = np + 64;
-    const size_t need = 5 * np * 4 + (size_t)nsnap * ns * esz + 2 * (size_t)g.nt * a->plane * 4;
+    const int ld = round_up(g.n1, 64);
+    const size_t np = (size_t)ld * a->plane + 64;
+    const size_t fixed = 2 * (size_t)g.nt * a->plane * 4, cell = 5 * 4 + (size_t)nsnap * esz;
     size_t freeb = 0, totb = 0;
     HIPCHK(hipMemGetInfo(&freeb, &totb));
-    const char* pad = getenv("RTM_AC3_PAD");  // 0: contiguous rows (experiments)
-    if (np < (size_t)1 << 31 && need < freeb / 10 * 9 && !(pad && atoi(pad) == 0)) {
+    // Padding is to cost little memory, which other handles may be counting on:
+    // at most a third more than contiguous rows take, and at most a sixteenth of
+    // what is free. RTM_AC3_PAD (tests): 0 contiguous rows, 1 padded ones.
+    const char* pad = getenv("RTM_AC3_PAD");
+    const bool fits = np * cell + fixed < freeb / 10 * 9;
+    const bool little = 3LL * ld <= 4LL * g.n1 && (np - a->n) * cell <= freeb / 16;
+    if (np < (size_t)1 << 31 && fits && (pad ? atoi(pad) != 0 : little)) {
       a->ld = ld;
       a->lead = 27;
       a->slead = 59;
       a->np = np;
-      a->ns = ns;
     }
   }
   // RTM_AC3_YCHUNK overrides the planes per workgroup (experiments)
@@ -671,7 +676,7 @@ RTM_EXPORT int ac3d_create(ac3d** out, const ac3d_cfg_t* cfg, const float* c, co
   STCHK(a->rec.alloc((size_t)g.nt * a->plane * 4, "receiver data"));
   STCHK(fill0(a->rec.as<float>(), (size_t)g.nt * a->plane, a->st));
   STCHK(a->img.alloc(a->np * 4, "image"));
-  STCHK(a->snap.alloc((size_t)nsnap * a->ns * esz, "snapshots"));
+  STCHK(a->snap.alloc((size_t)nsnap * a->np * esz, "snapshots"));
   STCHK(a->smax.alloc(sizeof(unsigned) * (SMAX_SNAP + 1) * nsnap, "snapshot scales"));
   a->amp.assign(amp, amp + g.nt);
   HIPCHK(hipStreamSynchronize(a->st));
@@ -761,7 +766,7 @@ RTM_EXPORT int ac3d_get_data(ac3d* a, float* rec) {
 RTM_EXPORT int ac3d_get_image(ac3d* a, float* img) {
   if (!a || !img) { set_error("null argument"); return E_ARG; }
   HIPCHK(hipStreamSynchronize(a->st));
-  if (a->ld == a->cfg.n1) return copy_to_host(img, a->img.p, a->n * 4);
+  if (a->ld == a->cfg.n1) return copy_to_host(img, a->img.as<float>() + a->lead, a->n * 4);
   return ac3_fetch(a, a->img.as<float>() + a->lead, img);
 }
 

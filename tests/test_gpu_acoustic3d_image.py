@@ -1,6 +1,7 @@
 """Images of 3D acoustic handles read back: rows of every padding, in one piece
 and in pieces by several threads, and while another thread migrates on the same
 handle, which neither sees nor disturbs the run."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -49,3 +50,30 @@ def test_image_read_during_a_migration(hip):
     assert reads > 1
     assert np.array_equal(g.image(), want) and np.abs(want).max() > 0
     g.close()
+
+
+def _free(hip):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.load().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+# rows that a padded layout would lengthen most, and one that it lengthens by a quarter
+@pytest.mark.parametrize("n1", [11, 38, 41, 66, 102])
+def test_padding_takes_little_memory(hip, n1):
+    """A handle takes at most a third more device memory than contiguous rows
+    would (and what the allocator rounds up)."""
+    n2, n3, nt, j = 150, 160, 40, 1
+    rows = n2 * n3
+    # velocity term, two fields, image and a snapshot a level; the record
+    contiguous = 4 * n1 * rows * (4 + nt // j) + 4 * nt * rows
+    warm = _handle(hip, (40, 40, 40), 3)
+    warm.migrate()
+    free0 = _free(hip)
+    g = hip.Acoustic3D(np.full((n1, n2, n3), 0.08, np.float32, order="F"), np.ones(nt, np.float32), (5, 70, 80), 5, abc=0,
+                       snap_every=j, snap_prec="fp32")
+    used = free0 - _free(hip)
+    print("acoustic memory", n1, used / contiguous, flush=True)
+    assert used <= contiguous * 4 / 3 + 2**26
+    g.close()
+    warm.close()

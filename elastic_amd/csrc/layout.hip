@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdlib>
 #include <vector>
 
 namespace erm {
@@ -89,7 +90,8 @@ __global__ void k_clear_flag(int* flag) { *flag = 0; }
 unsigned blocks_of(size_t n) { return (unsigned)std::min<size_t>((n + 255) / 256, 16384); }
 
 // Scratch of `want` bytes, at least `least`, at most kScratch (or least), with
-// 256 bytes behind it for the flag. False: none is to be had.
+// 256 bytes behind it for the flag. False: none is to be had (RTM_SCRATCH=0, for
+// tests: as if).
 struct Scratch {
   DevBuf b;
   size_t bytes = 0;
@@ -98,6 +100,8 @@ struct Scratch {
     bytes = std::max(std::min(want, kScratch), least);
     bytes = (bytes + 255) / 256 * 256;
     void* p = nullptr;
+    const char* e = getenv("RTM_SCRATCH");
+    if (e && atoi(e) == 0) return false;
     if (hipMalloc(&p, bytes + 256) != hipSuccess) {
       (void)hipGetLastError();
       return false;

@@ -105,7 +105,7 @@ __device__ __forceinline__ T g1(const T* p, int i) {
 // A plane is addressed as a raw buffer, so the offsets of a thread's cells stay
 // the same through the march; what a plane needs besides (image, injected row)
 // is loaded at its start. us a step, 203 x 181 x 247 (bound by latency and
-// vector instructions) and 522^3 (bound by memory: the step moves 2.7 GB, 5.6
+// vector instructions) and 522^3 (bound by memory: the step moves 2.6 GB, 5.4
 // TB/s, of which 0.5 GB are halo lines fetched twice): through pointers 42 and
 // 526, with the image 60 and 970; now 33 and 480, 56 and 767.
 // The halo cells of a plane are loaded with the queue entry of the same
@@ -404,7 +404,7 @@ std::vector<float> taper(int n, int abc) {
   return k;
 }
 
-// Step workgroups resident at once on the current device (109 VGPRs without
+// Step workgroups resident at once on the current device (122 VGPRs without
 // imaging: 4 waves per SIMD, so 4 workgroups a CU, 1024 on the chip).
 int resident_workgroups() {
   static const int n = [] {
@@ -419,14 +419,15 @@ int resident_workgroups() {
   return n;
 }
 
-// Planes a workgroup marches along y. A plane costs a workgroup about 1.7 us
+// Planes a workgroup marches along y. A plane costs a workgroup about 1.2 us
 // whatever the grid (the latency of its loads), and a chunk some six planes
 // more for its first loads, so the step takes (rounds of resident workgroups)
 // x (planes + 6): the number of chunks that minimises it. Both sides,
-// source-pass step: 203 x 181 x 247 (44 tiles) 64 planes 115 us, 12 planes
-// 42 us; 266^3 64 planes 115 us, 16 planes (one whole round) 59 us; 64^3 64
-// planes 94 us, 8 planes 18 us. At 522^3 (256 tiles), where memory bounds the
-// step, 64 to 128 planes take 1 to 9% more or less.
+// source-pass step: 203 x 181 x 247 (44 tiles) 64 planes 83 us, 11 planes (the
+// rule's) 35 us; 266^3 (64 tiles) 64 planes 83 us, 16 planes (the rule's, one
+// whole round) 52, 8 planes (two) 50; 64^3 (4 tiles) 64 planes 67 us, 8 planes 13,
+// one plane (the rule's) 5.8. At 522^3 (256 tiles), where memory bounds the step,
+// 128 planes (the rule's) 483 us, 103 494, 86 488, 64 504, 32 506.
 int planes_per_workgroup(int tiles, int n) {
   const int resident = resident_workgroups();
   long long best = -1;

@@ -50,7 +50,7 @@ struct ShotDev {
   float* imgc;  // 3 * n2 compensation terms
   float inv_dx, inv_dt, img_w;
   // Born modelling
-  float* bsrc;       // 5 * n2 scattering sources of the current level
+  float* bsrc;       // 5 * n2 scattering sources of the current level (marching forms)
   const float* dm;   // 3 * n2 model perturbation
 };
 

@@ -486,8 +486,9 @@ int Engine::fill_desc(int g, bool true_model, bool born_mode) {
     d.inv_dt = 1.0f / cfg_.dt;
     d.img_w = (float)cfg_.snap_every;
     if (born_mode) {
-      d.bsrc = born_buf_.as<float>() + k * 8 * n2max_;
-      d.dm = born_buf_.as<float>() + k * 8 * n2max_ + 5 * n2max_;
+      float* const b = born_buf_.as<float>() + k * born_fields() * n2max_;
+      d.dm = b;
+      if (cfg_.tblock >= 2) d.bsrc = b + 3 * n2max_;
     }
     h_desc_[variant * ns + s] = d;
   }
@@ -824,12 +825,12 @@ int Engine::born(const std::vector<const float*>& dm) {
   if (groups_.size() != 1) { set_error("Born modelling runs single-group engines only"); return E_ARG; }
   if (dm.size() != specs_.size()) { set_error("dm list size mismatch"); return E_ARG; }
   if (cfg_.snap_fmt != SNAP_HIST) { set_error("Born modelling needs the fp32 history format"); return E_ARG; }
-  STCHK(born_buf_.alloc((size_t)G_ * 8 * n2max_ * sizeof(float), "Born sources"));
-  STCHK(launch_fill(born_buf_.as<float>(), (size_t)G_ * 8 * n2max_, 0.f, st_));
+  STCHK(born_buf_.alloc((size_t)G_ * born_fields() * n2max_ * sizeof(float), "Born sources"));
+  STCHK(launch_fill(born_buf_.as<float>(), (size_t)G_ * born_fields() * n2max_, 0.f, st_));
   HIPCHK(hipStreamSynchronize(st_));
   for (size_t k = 0; k < specs_.size(); ++k) {
     const ShotSpec& p = specs_[k];
-    float* d = born_buf_.as<float>() + k * 8 * n2max_ + 5 * n2max_;
+    float* d = born_buf_.as<float>() + k * born_fields() * n2max_;
     const size_t nn = (size_t)p.nz * p.nx;
     const float* c[3] = {dm[k], dm[k] + nn, dm[k] + 2 * nn};
     // component stride = the shot's own n2 (as the kernels index it)

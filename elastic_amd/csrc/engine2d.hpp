@@ -175,6 +175,9 @@ class Engine {
   };
   int build_lcells();
   int tile_code() const { return erm::tile_code(cfg_.txr, cfg_.tblock, cfg_.snap_fmt); }
+  // fields of a shot's Born buffer: the perturbation, and for the marching forms
+  // the scattering sources of a level, which the others form in the step
+  size_t born_fields() const { return cfg_.tblock >= 2 ? 8 : 3; }
   int single_nbz(const Group& gr) const;
   int alloc_working();
   int build_groups();

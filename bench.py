@@ -240,7 +240,7 @@ def cpu_baseline(lib, synth, seed, dx, dt, fp, abc, nt_sample, nthreads):
 
 def load_traffic(variant, kernel):
     """Measured HBM bytes per cell-update of a kernel (profiles/traffic_<variant>.json:
-    one entry per kernel form, from rocprofv3 FETCH_SIZE / WRITE_SIZE passes)."""
+    one entry per kernel form, from rocprofv3 passes of the L2's requests to the fabric)."""
     path = os.path.join(ROOT, "profiles", f"traffic_{variant}.json")
     if not os.path.exists(path):
         return None
@@ -623,7 +623,7 @@ def main():
     cells_per_launch = (info["adj_cells"] / info["adj_launches"]) if dom == "adj" else \
         (info["fwd_cells"] / info["fwd_launches"])
     # HBM bytes per launch of the dominant kernel: measured bytes per
-    # cell-update (rocprofv3 FETCH_SIZE / WRITE_SIZE passes, calibrated on a
+    # cell-update (rocprofv3 counters of the L2's requests to the fabric, calibrated on a
     # copy kernel) times this run's cell-updates per launch; marching figures
     # are kept per strip width, and a width without figures of its own
     # reports null

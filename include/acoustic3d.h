@@ -45,7 +45,7 @@ int ac3d_model_data(ac3d *a, const float *c_true);
 int ac3d_migrate(ac3d *a);
 int ac3d_set_data(ac3d *a, const float *rec);
 int ac3d_get_data(ac3d *a, float *rec);
-int ac3d_get_image(ac3d *a, float *img);
+int ac3d_get_image(ac3d *a, float *img); /* changes nothing in the handle */
 int ac3d_get_snapshot_scales(ac3d *a, float *out, int n);
 /* [0] source-pass ms [1] its launches [2] receiver-pass ms [3] its launches
  * [4] last model_data ms */

@@ -50,7 +50,9 @@ void rtm_op3_c_(int nt, int nz, int nx, int zrec, float *Vx0, float *Vz0, float 
 
 /* Same contract as rtm_op3_c_, returning RTM_OK or RTM_E_*. No counterpart
  * in the reference, which returns void (W/rtmlib-modC.c:29); this is the
- * status-returning form callers should bind when they can check errors. */
+ * status-returning form callers should bind when they can check errors. Nothing
+ * is written to the histories before every step has run: a call that fails on
+ * the way leaves them as they were. */
 int rtm_op3_hip(int nt, int nz, int nx, int zrec, float *Vx0, float *Vz0, float *sigmaxx0,
                 float *sigmazz0, float *sigmaxz0, const float *m1_x, const float *m1_z,
                 const float *aux_m2_c, const float *aux_m3_c, const float *aux_m2m3_c);
@@ -228,7 +230,7 @@ int rtm_batch_get_stack(rtm_batch *b, float *img3);            /* 3*(stack_nz,st
  * [5] fwd cell-updates [6] adj cell-updates [7] shots per group */
 int rtm_batch_info(rtm_batch *b, double *out8);
 int rtm_batch_destroy(rtm_batch *b);
-/* Tile width and kernel form the batch runs with (form 0: one level per
+/* Tile width and kernel form the batch runs (form 0: one level per
  * launch on tiles, 1: two levels per launch, 2: one level per launch,
  * strips marching along x, 3: the marching forward with the tile adjoint). */
 int rtm_batch_txr(rtm_batch *b);
@@ -241,7 +243,7 @@ int rtm_batch_tblock(rtm_batch *b);
  * groups, RTM_MARCH_FIT=0 turns the fitting off. */
 int rtm_batch_march_w(rtm_batch *b);
 /* Tile autotuner: runs a short copy of the workload (the shots of the full
- * run's first group, at most 24 or RTM_TUNE_MAXSHOTS; max(48, 8*snap_every)
+ * run's first group, at most 24 or RTM_TUNE_MAXSHOTS; max(96, 16*snap_every)
  * levels; same options) with tile widths 1, 2, 4, 8 at one level per
  * launch, 1, 2, 4 at two levels per launch (temporal blocking) and the
  * marching forms (strips of 16, 24, 28 and 32 columns), and returns the fastest in
